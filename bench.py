@@ -744,19 +744,22 @@ def main() -> None:
     # fp32) is its own kernel
     adj_w4 = _native.get_tm2d_adjoint_waves() == 4 and 64 * _native.get_tm2d_tuning()[3] <= 256
     for name, d in summ.items():
-        spl = int(d["steps_per_launch"])
         k_ms, k_launches, _ = loop_ms.get(name, (d["ms"], d["launches"], 0))
+        # the launches made (the setting 0 leaves their number to the library)
+        spl = max(1, round(d["steps"] / max(k_launches, 1)))
         achieved = b_alg[name] * d["cell_updates"] / (k_ms * 1e-3) / 1e9
         stem = "adj" if name == "adjoint" else "fwd"
         kname = f"{stem}_step" if spl == 1 else (f"{stem}2_step" if spl == 2 else f"{stem}k_step")
         if stem == "adj" and spl >= 3 and adj_w4:
             kname = "adjk_step_w4"
+        if spl > 4:
+            kname = f"tile_{stem}"
         kernels[name] = {
             "kernel": kname,
             "steps_per_launch": spl,
             "launches": k_launches,
             "avg_launch_us": round(k_ms / max(k_launches, 1) * 1e3, 2),
-            "call_avg_launch_us": round(d["ms"] / d["launches"] * 1e3, 2),
+            "call_avg_launch_us": round(d["ms"] / max(k_launches, 1) * 1e3, 2),
             "bytes_per_cell_update": b_alg[name],
             "achieved_GBs": round(achieved, 1),
             "gcell_per_s": round(d["cell_updates"] / (k_ms * 1e-3) / 1e9, 2),

@@ -1,0 +1,110 @@
+"""Workgroup tiles of the 2-D TM time loops (one launch advances a tile by
+several steps) against the CPU oracle, at the edges of their shapes: grids
+narrower than a tile, one column or row beside a tile's owned cells, every
+remainder of the time loop, per-shot coefficients, several points in one
+cell and points in several rows.
+
+Tolerances: fields, receivers, snapshots, adjoint fields and source
+gradients bit-identical (the single-step expressions in their order, and an
+exactly rounded CPML division); FP64 coefficient gradients within 1e-12, the
+bound of a reordered sum of nt * shots terms.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import tide
+from gpu_abi import gpu_backward, gpu_forward
+from helpers import FIELD_NAMES, relative_l2
+from oracle import oracle as O
+from tide.maxwell.tm2d import prepare_tm2d
+
+gpu = pytest.mark.gpu
+
+
+def _case(ny, nx, nt, *, stencil=2, dtype=torch.float32, shots=2, pml=(3, 4, 5, 2), batched=False,
+          seed=5):
+    """A padded ny x nx problem with doubled points and two source rows."""
+    half = stencil // 2
+    my, mx = ny - pml[0] - pml[1] - 2 * half + 1, nx - pml[2] - pml[3] - 2 * half + 1
+    g = torch.Generator().manual_seed(seed)
+    shape = (shots, my, mx) if batched else (my, mx)
+    eps = (1.0 + 8.0 * torch.rand(*shape, generator=g, dtype=torch.float64)).to(dtype)
+    sig = (0.01 * torch.rand(*shape, generator=g, dtype=torch.float64)).to(dtype)
+    dx = 0.01
+    dt = 0.7 * dx / (2**0.5 * tide.C0)
+    amp = tide.ricker(9e8, nt + 8, dt, peak_time=4 * dt, dtype=dtype)[:nt].reshape(1, 1, -1)
+    amp = amp.repeat(shots, 3, 1) * torch.tensor([1.0, 0.5, -0.7], dtype=dtype)[None, :, None]
+    src = torch.stack([torch.tensor([[1, (2 + 3 * s) % mx], [1, (2 + 3 * s) % mx], [my - 1, s % mx]])
+                       for s in range(shots)])
+    cols = list(range(0, mx, 2)) + [1 % mx, 1 % mx]
+    rec = torch.stack([torch.tensor([[1, x] for x in cols] + [[my // 2, 0]])] * shots)
+    st = prepare_tm2d(eps, sig, torch.ones_like(eps), dx, dt, amp, src, rec, stencil=stencil,
+                      pml_width=list(pml))
+    assert (st.ny, st.nx) == (ny, nx)
+    return O.case_from_setup(st)
+
+
+def _check(case, store="full"):
+    f_o, r_o, es, cs = O.tm2d_forward(case, store=store)
+    f_g, r_g, es_g, cs_g = gpu_forward(case, store=store)
+    assert np.array_equal(r_g, r_o)
+    assert np.array_equal(es_g, es) and np.array_equal(cs_g, cs)
+    for name, a, b in zip(FIELD_NAMES, f_g, f_o):
+        assert np.array_equal(a, b), name
+    f_n, r_n, _, _ = gpu_forward(case)
+    assert np.array_equal(r_n, r_o) and all(np.array_equal(a, b) for a, b in zip(f_n, f_o))
+    w = np.random.default_rng(3).standard_normal(r_o.shape).astype(case.dtype)
+    ga_o, gb_o, gf_o, lam_o = O.tm2d_backward(case, w, es, cs, store=store)
+    ga, gb, gf, lam = gpu_backward(case, w, es_g, cs_g, store=store)
+    for a, b in zip(lam, lam_o):
+        assert np.array_equal(a.reshape(b.shape), b)
+    assert np.array_equal(gf, gf_o)
+    for a, b in ((ga, ga_o), (gb, gb_o)):  # a single step from rest has no gradient
+        assert relative_l2(a, b) < 1e-12 if b.any() else not a.any()
+
+
+@gpu
+@pytest.mark.parametrize("ny,nx", [(14, 14), (48, 64), (49, 65), (47, 63), (17, 130), (97, 33),
+                                   (128, 49)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_grids_beside_the_tile_edges(ny, nx, dtype):
+    print(f"grid {ny}x{nx} {dtype}", flush=True)
+    _check(_case(ny, nx, 21, dtype=dtype))
+
+
+@gpu
+@pytest.mark.parametrize("nt", [1, 2, 7, 8, 9, 15, 16, 17, 33])
+def test_every_remainder_of_the_time_loop(nt):
+    print(f"nt {nt}", flush=True)
+    _check(_case(40, 70, nt))
+
+
+@gpu
+def test_many_tiles_and_shots_take_the_larger_tiles():
+    _check(_case(230, 310, 13, shots=7, pml=(12, 9, 11, 10)))
+
+
+@gpu
+def test_bf16_snapshots_and_per_shot_coefficients():
+    _check(_case(60, 75, 19, shots=3), store="bf16")
+    _check(_case(60, 75, 19, shots=3, batched=True))
+
+
+def test_cpml_division_by_held_reciprocal_is_exact():
+    """d / k rounded to 32 bits equals the 64-bit product d * (1 / k)
+    rounded to 32 bits: a quotient of two 24-bit numbers lies at least 2^-49
+    (relative) from the midpoint of two floats, the product within 2^-52 of
+    the quotient.  Random bit patterns (subnormals, infinities and NaN
+    included) over the range of the CPML stretch."""
+    rng = np.random.default_rng(1)
+    d = rng.integers(0, 1 << 32, 4_000_000, dtype=np.uint64).astype(np.uint32).view(np.float32)
+    k = rng.integers(0x3F800000, 0x40A00001, d.size, dtype=np.uint64).astype(np.uint32).view(np.float32)
+    with np.errstate(all="ignore"):
+        want = d / k
+        got = (d.astype(np.float64) * (1.0 / k.astype(np.float64))).astype(np.float32)
+    assert np.array_equal(got, want, equal_nan=True)
+    assert np.array_equal(np.signbit(got[want == 0]), np.signbit(want[want == 0]))

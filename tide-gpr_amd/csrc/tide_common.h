@@ -83,6 +83,15 @@ bool build_point_table_halo(const int64_t *src, int64_t n_src, const int64_t *re
                             int64_t n_rec, int64_t n_shots, int64_t ny, int64_t nx,
                             int tile_w, int lane_offset, PointTable &out);
 
+// As build_point_table_halo, with the entries of a segment sorted by lane
+// (then kind, then point order): ent.x = lane | kind<<8 plus kPointCopy for
+// a halo copy, and kPointFirst / kPointLast on the first and last entry of
+// each lane's run.
+constexpr int kPointCopy = 1 << 9, kPointFirst = 1 << 10, kPointLast = 1 << 11;
+bool build_point_table_lanes(const int64_t *src, int64_t n_src, const int64_t *rec,
+                             int64_t n_rec, int64_t n_shots, int64_t ny, int64_t nx,
+                             int tile_w, int lane_offset, PointTable &out);
+
 // Device copy of a PointTable: either three device allocations of its own
 // (upload) or three caller-provided arrays of the sizes below (place).
 struct DevicePointTable {

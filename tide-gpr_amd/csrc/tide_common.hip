@@ -17,7 +17,7 @@ const char *last_error() { return g_last_error.c_str(); }
 namespace {
 bool build_table(const int64_t *src, int64_t n_src, const int64_t *rec, int64_t n_rec,
                  int64_t n_shots, int64_t ny, int64_t nx, int tile_w, int lane_offset,
-                 bool halo, PointTable &out) {
+                 bool halo, bool by_lane, PointTable &out) {
   const int64_t numel = ny * nx;
   const int64_t n_xt = (nx + tile_w - 1) / tile_w;
   // (y, shot, xt, kind, k, xloc, q); kind bit 1 marks a halo copy
@@ -57,10 +57,18 @@ bool build_table(const int64_t *src, int64_t n_src, const int64_t *rec, int64_t 
     return true;
   };
   if (!add(src, n_src, 0) || !add(rec, n_rec, 1)) return false;
-  std::sort(entries.begin(), entries.end(), [](const Entry &a, const Entry &b) {
-    return std::tie(a.y, a.shot, a.xt, a.kind, a.k) <
-           std::tie(b.y, b.shot, b.xt, b.kind, b.k);
-  });
+  if (by_lane) {
+    std::sort(entries.begin(), entries.end(), [](const Entry &a, const Entry &b) {
+      const int64_t ka = a.kind & 1, kb = b.kind & 1;
+      return std::tie(a.y, a.shot, a.xt, a.xloc, ka, a.k) <
+             std::tie(b.y, b.shot, b.xt, b.xloc, kb, b.k);
+    });
+  } else {
+    std::sort(entries.begin(), entries.end(), [](const Entry &a, const Entry &b) {
+      return std::tie(a.y, a.shot, a.xt, a.kind, a.k) <
+             std::tie(b.y, b.shot, b.xt, b.kind, b.k);
+    });
+  }
   out.n_xt = (int32_t)n_xt;
   out.row_slot.assign((size_t)ny, -1);
   std::vector<int64_t> rows;
@@ -77,11 +85,21 @@ bool build_table(const int64_t *src, int64_t n_src, const int64_t *rec, int64_t 
   }
   for (int64_t i = 0; i < n_seg; ++i) out.seg[(size_t)i + 1] = out.seg[(size_t)i] + counts[(size_t)i];
   out.ent.resize(entries.size());
-  // entries are already in (row, shot, tile, kind, k) order == segment order.
+  // entries are already sorted by (row, shot, tile) == segment order.
   for (size_t i = 0; i < entries.size(); ++i)
     out.ent[i] = make_int2(entries[i].xloc | ((int32_t)(entries[i].kind & 1) << 8) |
                                ((int32_t)(entries[i].kind >> 1) << 9),
                            entries[i].q);
+  if (by_lane) {
+    auto same = [&](size_t i, size_t j) {
+      const Entry &a = entries[i], &b = entries[j];
+      return std::tie(a.y, a.shot, a.xt, a.xloc) == std::tie(b.y, b.shot, b.xt, b.xloc);
+    };
+    for (size_t i = 0; i < entries.size(); ++i) {
+      if (i == 0 || !same(i - 1, i)) out.ent[i].x |= kPointFirst;
+      if (i + 1 == entries.size() || !same(i, i + 1)) out.ent[i].x |= kPointLast;
+    }
+  }
   return true;
 }
 }  // namespace
@@ -89,13 +107,19 @@ bool build_table(const int64_t *src, int64_t n_src, const int64_t *rec, int64_t 
 bool build_point_table(const int64_t *src, int64_t n_src, const int64_t *rec,
                        int64_t n_rec, int64_t n_shots, int64_t ny, int64_t nx,
                        int tile_w, int lane_offset, PointTable &out) {
-  return build_table(src, n_src, rec, n_rec, n_shots, ny, nx, tile_w, lane_offset, false, out);
+  return build_table(src, n_src, rec, n_rec, n_shots, ny, nx, tile_w, lane_offset, false, false, out);
 }
 
 bool build_point_table_halo(const int64_t *src, int64_t n_src, const int64_t *rec,
                             int64_t n_rec, int64_t n_shots, int64_t ny, int64_t nx,
                             int tile_w, int lane_offset, PointTable &out) {
-  return build_table(src, n_src, rec, n_rec, n_shots, ny, nx, tile_w, lane_offset, true, out);
+  return build_table(src, n_src, rec, n_rec, n_shots, ny, nx, tile_w, lane_offset, true, false, out);
+}
+
+bool build_point_table_lanes(const int64_t *src, int64_t n_src, const int64_t *rec,
+                             int64_t n_rec, int64_t n_shots, int64_t ny, int64_t nx,
+                             int tile_w, int lane_offset, PointTable &out) {
+  return build_table(src, n_src, rec, n_rec, n_shots, ny, nx, tile_w, lane_offset, true, true, out);
 }
 
 int DevicePointTable::upload(const PointTable &t, hipStream_t stream) {

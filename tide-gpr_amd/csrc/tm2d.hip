@@ -30,6 +30,7 @@
 #include "tm2d_fused.h"
 #include "tm2d_launch.h"
 #include "tm2d_launch_k.h"
+#include "tm2d_tile_launch.h"
 #include "tide_hip.h"
 #include "tide_storage.h"
 #include "tm2d_highorder.h"
@@ -231,6 +232,188 @@ int upload_points(const Problem<T> &p, const int64_t *src, const int64_t *rec,
   return put_table(table2, *dpt2, arena_scr, stream);
 }
 
+// ------------------------------------------------- workgroup-tile time loops
+
+template <typename T>
+int upload_points_lanes(const Problem<T> &p, const TilePlan &plan, const int64_t *src,
+                        const int64_t *rec, DevicePointTable &dpt, hipStream_t stream,
+                        Scratch *arena_scr = nullptr) {
+  std::vector<int64_t> hsrc, hrec;
+  TIDE_CHECK(fetch_indices(src, (int64_t)p.n_shots * p.n_src, hsrc, stream));
+  TIDE_CHECK(fetch_indices(rec, (int64_t)p.n_shots * p.n_rec, hrec, stream));
+  PointTable table;
+  if (!build_point_table_lanes(hsrc.data(), p.n_src, hrec.data(), p.n_rec, p.n_shots, p.g.ny,
+                               p.g.nx, plan.own_cols, plan.halo, table))
+    return kInvalidArgument;
+  return put_table(table, dpt, arena_scr, stream);
+}
+
+// Steps of each launch of a time loop of nt steps, at most `most` each: the
+// fewest launches, an even number of them where nt allows it (the state ping-
+// pongs between the caller's arrays and a scratch copy, and an even count ends
+// in the caller's arrays), as equal as possible.
+struct LaunchSteps {
+  int64_t nt, launches;
+  LaunchSteps(int64_t nt_, int most) : nt(nt_), launches((nt_ + most - 1) / most) {
+    if ((launches & 1) && nt > launches) ++launches;
+  }
+  int at(int64_t k) const { return (int)(nt * (k + 1) / launches - nt * k / launches); }
+  bool ends_in_scratch() const { return (launches & 1) != 0; }
+};
+
+template <typename T>
+int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_hx_z,
+                  T *m_hz_x, const T *f, T *r, const int64_t *src, const int64_t *rec, int64_t nt,
+                  int64_t start_t, int64_t step_ratio, void *ey_store, void *curl_store, int fmt,
+                  size_t store_step_bytes, hipStream_t stream, char *arena, size_t arena_cap) {
+  const int64_t n_shots = p.n_shots, total = n_shots * p.g.numel;
+  const TilePlan plan = plan_tiles<T>(half, p.g.ny, p.g.nx, p.n_shots, false,
+                                       ey_store || curl_store);
+  const LaunchSteps loop(nt, plan.steps);
+  Scratch scr(stream, arena, arena_cap);
+  DevicePointTable dpt;
+  TIDE_CHECK(upload_points_lanes(p, plan, src, rec, dpt, stream, &scr));
+  TIDE_CHECK(pack_profiles(p, scr, stream));
+  T *const own[7] = {ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x};
+  T *cur[7], *nxt[7];
+  const size_t bytes = (size_t)total * sizeof(T);
+  for (int k = 0; k < 7; ++k) {
+    cur[k] = own[k];
+    TIDE_CHECK(scr.alloc(&nxt[k], (size_t)total));
+    // the memories are only written inside their strips: where the scratch
+    // copy ends up as the result, its other cells must hold the caller's
+    if (k >= 3 && loop.ends_in_scratch())
+      TIDE_HIP_TRY(hipMemcpyAsync(nxt[k], cur[k], bytes, hipMemcpyDeviceToDevice, stream));
+  }
+  TileFwdArgs<T> a;
+  std::memset(&a, 0, sizeof(a));
+  a.g = p.g;
+  a.pts = Points{dpt.row_slot, dpt.seg, dpt.ent, dpt.n_xt};
+  a.ca = p.ca;
+  a.cb = p.cb;
+  a.cq = p.cq;
+  a.n_shots = p.n_shots;
+  a.halo = plan.halo;
+  a.own_rows = plan.own_rows;
+  a.f_stride = n_shots * p.n_src;
+  a.r_stride = n_shots * p.n_rec;
+  LoopTimer timer(0, stream);
+  int64_t t = start_t;
+  for (int64_t k = 0; k < loop.launches; ++k) {
+    a.steps = loop.at(k);
+    for (int q = 0; q < 7; ++q) {
+      a.in[q] = cur[q];
+      a.out[q] = nxt[q];
+    }
+    a.f = p.n_src > 0 ? f + t * a.f_stride : nullptr;
+    a.r = p.n_rec > 0 ? r + t * a.r_stride : nullptr;
+    bool st = false;
+    for (int j = 0; j < a.steps; ++j) {
+      const bool on = ((t + j) % step_ratio) == 0;
+      const size_t at = (size_t)((t + j) / step_ratio) * store_step_bytes;
+      a.ey_store[j] = on && ey_store ? (char *)ey_store + at : nullptr;
+      a.curl_store[j] = on && curl_store ? (char *)curl_store + at : nullptr;
+      st = st || a.ey_store[j] || a.curl_store[j];
+    }
+    launch_tile_fwd<T>(half, plan, st ? fmt : 0, stream, a);
+    t += a.steps;
+    for (int q = 0; q < 7; ++q) std::swap(cur[q], nxt[q]);
+  }
+  timer.finish(loop.launches);
+  TIDE_HIP_TRY(hipGetLastError());
+  for (int q = 0; q < 7; ++q)
+    if (cur[q] != own[q])
+      TIDE_HIP_TRY(hipMemcpyAsync(own[q], cur[q], bytes, hipMemcpyDeviceToDevice, stream));
+  dpt.release(stream);
+  return kOk;
+}
+
+template <typename T>
+int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *ml_ey_x,
+                   T *ml_ey_z, T *ml_hx_z, T *ml_hz_x, const void *ey_store,
+                   const void *curl_store, int fmt, size_t store_step_bytes, T *grad_f,
+                   double *gca, double *gcb, const int64_t *src, const int64_t *rec, int64_t nt,
+                   int64_t start_t, int64_t step_ratio, hipStream_t stream) {
+  const int64_t n_shots = p.n_shots, numel = p.g.numel, total = n_shots * numel;
+  const TilePlan plan = plan_tiles<T>(half, p.g.ny, p.g.nx, p.n_shots, true, true);
+  const LaunchSteps loop(nt, plan.steps);
+  Scratch scr(stream);
+  DevicePointTable dpt;
+  TIDE_CHECK(upload_points_lanes(p, plan, src, rec, dpt, stream));
+  TIDE_CHECK(pack_profiles(p, scr, stream));
+  T *const own[7] = {l_ey, l_hx, l_hz, ml_hz_x, ml_hx_z, ml_ey_x, ml_ey_z};
+  T *cur[7], *nxt[7];
+  const size_t bytes = (size_t)total * sizeof(T);
+  for (int k = 0; k < 7; ++k) {
+    cur[k] = own[k];
+    TIDE_CHECK(scr.alloc(&nxt[k], (size_t)total));
+    if (k >= 3 && loop.ends_in_scratch())
+      TIDE_HIP_TRY(hipMemcpyAsync(nxt[k], cur[k], bytes, hipMemcpyDeviceToDevice, stream));
+  }
+  TileAdjArgs<T> a;
+  std::memset(&a, 0, sizeof(a));
+  a.g = p.g;
+  a.pts = Points{dpt.row_slot, dpt.seg, dpt.ent, dpt.n_xt};
+  a.ca = p.ca;
+  a.cb = p.cb;
+  a.cq = p.cq;
+  a.per_shot_grad = ((gca && p.g.ca_b) || (gcb && p.g.cb_b)) ? 1 : 0;
+  a.step_scale = (double)step_ratio;
+  a.n_shots = p.n_shots;
+  a.halo = plan.halo;
+  a.own_rows = plan.own_rows;
+  a.group = plan.group;
+  a.r_stride = n_shots * p.n_rec;
+  a.f_stride = n_shots * p.n_src;
+  // Several shot groups: each accumulates into its own FP64 slice, folded
+  // into gca / gcb in group order at the end (no atomics, repeatable).
+  const int64_t n_groups = (n_shots + plan.group - 1) / plan.group;
+  double *acc[2] = {nullptr, nullptr}, *const grad[2] = {gca, gcb};
+  if (n_groups > 1 && !a.per_shot_grad) {
+    a.group_stride = numel;
+    for (int k = 0; k < 2; ++k) {
+      if (grad[k] == nullptr) continue;
+      TIDE_CHECK(scr.alloc(&acc[k], (size_t)(n_groups * numel)));
+      TIDE_HIP_TRY(hipMemsetAsync(acc[k], 0, (size_t)(n_groups * numel) * sizeof(double), stream));
+    }
+  }
+  LoopTimer timer(1, stream);
+  int64_t t = start_t - 1;
+  for (int64_t k = 0; k < loop.launches; ++k) {
+    a.steps = loop.at(k);
+    for (int q = 0; q < 7; ++q) {
+      a.in[q] = cur[q];
+      a.out[q] = nxt[q];
+    }
+    a.grad_r = p.n_rec > 0 ? grad_r + t * a.r_stride : nullptr;
+    a.grad_f = (p.n_src > 0 && grad_f) ? grad_f + t * a.f_stride : nullptr;
+    bool g_any = false;
+    for (int j = 0; j < a.steps; ++j) {
+      const bool on = ((t - j) % step_ratio) == 0;
+      const size_t at = (size_t)((t - j) / step_ratio) * store_step_bytes;
+      a.ey_store[j] = on && gca ? (const char *)ey_store + at : nullptr;
+      a.curl_store[j] = on && gcb ? (const char *)curl_store + at : nullptr;
+      g_any = g_any || a.ey_store[j] || a.curl_store[j];
+    }
+    a.gca = g_any ? (acc[0] ? acc[0] : gca) : nullptr;
+    a.gcb = g_any ? (acc[1] ? acc[1] : gcb) : nullptr;
+    launch_tile_adj<T>(half, plan, g_any ? fmt : 0, stream, a);
+    t -= a.steps;
+    for (int q = 0; q < 7; ++q) std::swap(cur[q], nxt[q]);
+  }
+  timer.finish(loop.launches);
+  TIDE_HIP_TRY(hipGetLastError());
+  const unsigned fold_blocks = (unsigned)((numel + 255) / 256);
+  for (int k = 0; k < 2; ++k)
+    if (acc[k]) fold_groups<<<fold_blocks, 256, 0, stream>>>(grad[k], acc[k], numel, (int)n_groups);
+  TIDE_HIP_TRY(hipGetLastError());
+  for (int q = 0; q < 7; ++q)
+    if (cur[q] != own[q])
+      TIDE_HIP_TRY(hipMemcpyAsync(own[q], cur[q], bytes, hipMemcpyDeviceToDevice, stream));
+  dpt.release(stream);
+  return kOk;
+}
+
 template <typename T>
 int forward_impl(Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_hx_z,
                  T *m_hz_x, const T *f, T *r, const int64_t *src, const int64_t *rec,
@@ -252,9 +435,14 @@ int forward_impl(Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_h
   const bool staged = (ey_stage && ey_stage->active()) || (curl_stage && curl_stage->active());
   // K-step launches (K = 3, 4) need K ring slots at once, more than a
   // host-staged ring holds: staged calls use two-step launches.
-  const int kblk = (g_tuning.fwd_steps >= 3 && nt >= g_tuning.fwd_steps && !staged)
-                       ? g_tuning.fwd_steps : 0;
-  const bool fused = g_tuning.fwd_steps >= 2 && nt >= 2;
+  if (g_tuning.fwd_steps == 0 && !staged &&
+      prefer_tiles<T>(p.g.ny, p.g.nx, p.n_shots, false, ey_store || curl_store))
+    return forward_tiles(1, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r, src, rec, nt,
+                         start_t, step_ratio, ey_store, curl_store, fmt, store_step_bytes, stream,
+                         arena, arena_cap);
+  const int per_launch = g_tuning.fwd_steps == 0 ? 2 : g_tuning.fwd_steps;
+  const int kblk = (per_launch >= 3 && nt >= per_launch && !staged) ? per_launch : 0;
+  const bool fused = per_launch >= 2 && nt >= 2;
   Scratch scr(stream, arena, arena_cap);
   DevicePointTable dpt, dpt2, dptk;
   TIDE_CHECK(upload_points(p, src, rec, dpt, stream, fused ? &dpt2 : nullptr, &scr));
@@ -487,9 +675,13 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
   const int64_t n_shots = p.n_shots, total = n_shots * p.g.numel;
   const bool staged = (ey_stage && ey_stage->active()) || (curl_stage && curl_stage->active());
   // K-step launches need K ring slots at once (see forward_impl)
-  const int kblk = (g_tuning.adj_steps >= 3 && nt >= g_tuning.adj_steps && !staged)
-                       ? g_tuning.adj_steps : 0;
-  const bool fused = g_tuning.adj_steps >= 2 && nt >= 2;
+  if (g_tuning.adj_steps == 0 && !staged && prefer_tiles<T>(p.g.ny, p.g.nx, p.n_shots, true, true))
+    return backward_tiles(1, p, grad_r, l_ey, l_hx, l_hz, ml_ey_x, ml_ey_z, ml_hx_z, ml_hz_x,
+                          ey_store, curl_store, fmt, store_step_bytes, grad_f, gca, gcb, src, rec,
+                          nt, start_t, step_ratio, stream);
+  const int per_launch = g_tuning.adj_steps == 0 ? 3 : g_tuning.adj_steps;
+  const int kblk = (per_launch >= 3 && nt >= per_launch && !staged) ? per_launch : 0;
+  const bool fused = per_launch >= 2 && nt >= 2;
   DevicePointTable dpt, dpt2, dptk;
   TIDE_CHECK(upload_points(p, src, rec, dpt, stream, fused ? &dpt2 : nullptr));
   if (kblk) TIDE_CHECK(upload_points_k(p, src, rec, kblk, dptk, stream));
@@ -951,9 +1143,10 @@ int backward_entry(T const *ca, T const *cb, T const *cq, T const *grad_r, T *la
                                                  pml_y1, pml_x1);
     T *const lam[7] = {lambda_ey, lambda_hx, lambda_hz, m_lambda_ey_x, m_lambda_ey_z,
                        m_lambda_hx_z, m_lambda_hz_x};
-    rc = tm2d_ho::backward<T>(stencil, hp, lam, grad_r, ey_store_1, curl_store_1, fmt, step_bytes,
-                              grad_f, ca_rg ? ga : nullptr, cb_rg ? gb : nullptr, sources_i,
-                              receivers_i, nt, start_t, step_ratio, stream, &ey_st, &curl_st);
+    rc = tm2d_ho::backward<T>(stencil, hp, lam, grad_r, ey_store_1, curl_store_1, fmt,
+                                step_bytes, grad_f, ca_rg ? ga : nullptr, cb_rg ? gb : nullptr,
+                                sources_i, receivers_i, nt, start_t, step_ratio, stream, &ey_st,
+                                &curl_st);
   }
   TIDE_CHECK(close_stages(rc, ey_st, curl_st));
   if (own) {
@@ -1457,9 +1650,9 @@ extern "C" int tide_tm2d_get_adjoint_waves(int *out) {
 }
 
 extern "C" int tide_tm2d_set_time_block(int fwd_steps, int adj_steps) {
-  if (fwd_steps < 1 || fwd_steps > kMaxBlockSteps || adj_steps < 1 ||
+  if (fwd_steps < 0 || fwd_steps > kMaxBlockSteps || adj_steps < 0 ||
       adj_steps > kMaxBlockSteps) {
-    set_error("time steps per launch must be 1, 2, 3 or 4");
+    set_error("time steps per launch must be 1, 2, 3 or 4 (0: workgroup tiles)");
     return kInvalidArgument;
   }
   g_tuning.fwd_steps = fwd_steps;

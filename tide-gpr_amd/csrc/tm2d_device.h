@@ -711,7 +711,9 @@ constexpr int kMaxGroup = 8;  // shots (wavefronts) per workgroup
 struct Tuning {
   int fwd_rows = 4, fwd_group = 1, adj_rows = 4, adj_group = 4;
   int fwd_loop = 0, adj_loop = 0;
-  int fwd_steps = 2, adj_steps = 3;
+  // time steps per launch of the wavefront tiles (1 to 4); 0: workgroup
+  // tiles (tm2d_tile.h), whose steps per launch follow from the problem
+  int fwd_steps = 0, adj_steps = 0;
   int fwd_split = 0, adj_split = 0;
   // Border tile height of the two-step kernels: 1, 2 or 0 (the interior
   // height).  The forward is fastest with interior-height border tiles, the

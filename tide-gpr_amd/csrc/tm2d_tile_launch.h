@@ -1,0 +1,168 @@
+// Launch plan and launchers of the workgroup-tile kernels (tm2d_tile.h).
+// The definitions compile in one translation unit per pass and field type
+// (tm2d_tile_{fwd,adj}_{f32,f64}.hip).
+#pragma once
+
+#include "tm2d_tile.h"
+
+#include <algorithm>
+#include <cmath>
+
+namespace tide_hip {
+namespace tm2d {
+
+struct TilePlan {
+  int waves, rows, steps;  // wavefronts per workgroup, rows per wavefront, steps per launch
+  int halo, own_rows, own_cols, n_xt, n_yt, group;
+};
+
+inline TilePlan make_tile_plan(int half, int ny, int nx, int waves, int rows, int steps, int group) {
+  TilePlan p;
+  p.waves = waves;
+  p.rows = rows;
+  p.steps = steps;
+  p.halo = steps * (2 * half - 1);
+  p.own_rows = waves * rows - 2 * p.halo;
+  p.own_cols = 64 - 2 * p.halo;
+  p.n_xt = (nx + p.own_cols - 1) / p.own_cols;
+  p.n_yt = (ny + p.own_rows - 1) / p.own_rows;
+  p.group = group;
+  return p;
+}
+
+// Duration of one launch of `steps` steps when every workgroup runs at once
+// (one per CU), in microseconds: start, loads and stores plus the steps.
+// Measured on 60^2 to 150 x 200 grids; half is the stencil half-width.
+template <typename T>
+double tile_launch_us(int half, int rows, int steps, bool adjoint, bool storing) {
+  if (sizeof(T) == 8)
+    return adjoint ? (rows == 2 ? 11.2 + 1.8 * steps : 22.0 + 6.0 * steps)
+                   : (rows == 2 ? 9.8 + 1.5 * steps : 12.0 + 3.0 * steps);
+  if (adjoint) {
+    if (rows == 2) return 9.2 + 1.7 * steps;
+    return (half == 1 ? 13.0 : 17.0) + (half <= 2 ? 3.0 : 5.0) * steps;
+  }
+  if (rows == 2) return 6.4 + (storing ? 1.2 : 0.9) * steps;
+  return storing ? 6.8 + 2.0 * steps : 9.1 + 1.3 * steps;
+}
+
+// Tile shape and steps per launch of a problem: the shape with the least time
+// per step, a launch taking as many rounds of workgroups as its tiles fill the
+// CUs.  Small problems want small tiles (many CUs at work, few rows per
+// wavefront) and many steps (a launch's start is paid once); once the tiles
+// outnumber the CUs, larger tiles with less halo.  Measured against the model
+// (fp32, order 2, us per step, forward / adjoint): 171 000 cells 2.1 / 3.5
+// with 32-row tiles of 8 steps (64-row: 2.8 / 5.1), 577 000 cells 3.3 / 5.7
+// with 64-row tiles of 6 (32-row: 4.5 / 7.6).
+// `us_per_step` gets the modelled time per step.
+template <typename T>
+TilePlan plan_tiles(int half, int ny, int nx, int n_shots, bool adjoint, bool storing,
+                    double *us_per_step = nullptr) {
+  constexpr int kCus = 256;
+  TilePlan best{};
+  double best_us = 1e30;
+  for (int rows = 2; rows <= 4; rows += 2) {
+    // a wavefront holds at least `half` rows (it exchanges that many), and
+    // 64-row tiles of doubles overflow the registers of 16 wavefronts
+    if (rows < half || (sizeof(T) == 8 && rows == 4 && half <= 2)) continue;
+    const int waves = rows == 4 && (sizeof(T) == 8 || (adjoint && half == 4)) ? 8 : kTileWaves;
+    for (int steps = 1; steps <= kTileSteps; ++steps) {
+      const int halo = steps * (2 * half - 1);
+      // at least a quarter of the tile's rows and half its columns owned
+      if (halo > 16 || waves * rows - 2 * halo < waves * rows / 4) break;
+      const TilePlan p = make_tile_plan(half, ny, nx, waves, rows, steps, 1);
+      const double n = (double)p.n_xt * p.n_yt * n_shots;
+      const double rounds = n <= kCus ? 1.0 : std::min(std::ceil(n / kCus), n / kCus + 0.3);
+      const double us = rounds * tile_launch_us<T>(half, rows, steps, adjoint, storing) / steps;
+      if (us < best_us) {
+        best_us = us;
+        best = p;
+      }
+    }
+  }
+  if (us_per_step) *us_per_step = best_us;
+  return best;
+}
+
+// Whether the order-2 time loop of a problem runs faster on workgroup tiles
+// than on wavefront tiles (tm2d_fused.h, tm2d_blockk.h): fp64 always (fp32
+// wavefront tiles hold 4 rows, fp64 ones 2), fp32 until the wavefront tiles
+// fill the chip.  Their time per step, measured on 1.5 to 5 million cells:
+// forward 6 us + 2.1 us per million cells (2.8 with snapshots), adjoint 11.5 us
+// + 3.7 us.
+template <typename T>
+bool prefer_tiles(int ny, int nx, int n_shots, bool adjoint, bool storing) {
+  if (sizeof(T) == 8) return true;
+  double us;
+  plan_tiles<T>(1, ny, nx, n_shots, adjoint, storing, &us);
+  const double cells = (double)ny * nx * n_shots * 1e-6;
+  const double wave = adjoint ? 11.5 + 3.7 * cells : 6.0 + (storing ? 2.8 : 2.1) * cells;
+  return us < wave;
+}
+
+template <typename T>
+void launch_tile_fwd(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileFwdArgs<T> &a);
+template <typename T>
+void launch_tile_adj(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileAdjArgs<T> &a);
+
+#ifdef TIDE_TM2D_TILE_DEFINITIONS
+
+template <typename T, int P, int R, int W>
+void tile_fwd_fmt(const TilePlan &p, int fmt, hipStream_t stream, const TileFwdArgs<T> &a) {
+  const dim3 block(64, (unsigned)p.waves);
+  const unsigned grid = (unsigned)((int64_t)p.n_xt * p.n_yt * a.n_shots);
+  const size_t lds = TileRows<T, P>::bytes(p.waves, a.steps);
+  if (fmt == 0) return tile_fwd<T, P, R, W, 0><<<grid, block, lds, stream>>>(a);
+  if constexpr (sizeof(T) == 4)
+    if (fmt == 2) return tile_fwd<T, P, R, W, 2><<<grid, block, lds, stream>>>(a);
+  tile_fwd<T, P, R, W, 1><<<grid, block, lds, stream>>>(a);
+}
+
+template <typename T, int P, int R, int W>
+void tile_adj_fmt(const TilePlan &p, int fmt, hipStream_t stream, const TileAdjArgs<T> &a) {
+  const dim3 block(64, (unsigned)p.waves);
+  const int n_groups = (a.n_shots + a.group - 1) / a.group;
+  const unsigned grid = (unsigned)((int64_t)p.n_xt * p.n_yt * n_groups);
+  const size_t lds = TileRows<T, P>::bytes(p.waves, a.steps);
+  if (fmt == 0) return tile_adj<T, P, R, W, 0><<<grid, block, lds, stream>>>(a);
+  if constexpr (sizeof(T) == 4)
+    if (fmt == 2) return tile_adj<T, P, R, W, 2><<<grid, block, lds, stream>>>(a);
+  tile_adj<T, P, R, W, 1><<<grid, block, lds, stream>>>(a);
+}
+
+// The shapes plan_tiles() picks from.
+#define TIDE_TILE_PICK(fn)                                             \
+  if constexpr (P <= 2) {                                              \
+    if (p.rows == 2) return fn<T, P, 2, kTileWaves>(p, fmt, stream, a); \
+  }                                                                    \
+  if constexpr (sizeof(T) == 4) {                                      \
+    if (p.waves > 8) return fn<T, P, 4, kTileWaves>(p, fmt, stream, a); \
+  }                                                                    \
+  if constexpr (P > 2) return fn<T, P, 4, 8>(p, fmt, stream, a);
+
+template <typename T, int P>
+void tile_fwd_shape(const TilePlan &p, int fmt, hipStream_t stream, const TileFwdArgs<T> &a) {
+  TIDE_TILE_PICK(tile_fwd_fmt)
+}
+template <typename T, int P>
+void tile_adj_shape(const TilePlan &p, int fmt, hipStream_t stream, const TileAdjArgs<T> &a) {
+  TIDE_TILE_PICK(tile_adj_fmt)
+}
+
+template <typename T>
+void launch_tile_fwd(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileFwdArgs<T> &a) {
+  switch (half) {
+    default: tile_fwd_shape<T, 1>(p, fmt, stream, a); break;
+  }
+}
+template <typename T>
+void launch_tile_adj(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileAdjArgs<T> &a) {
+  switch (half) {
+    default: tile_adj_shape<T, 1>(p, fmt, stream, a); break;
+  }
+}
+
+#endif  // TIDE_TM2D_TILE_DEFINITIONS
+
+}  // namespace tm2d
+}  // namespace tide_hip

@@ -468,7 +468,8 @@ def get_tm2d_shot_loop() -> tuple[bool, bool]:
 
 
 def set_tm2d_time_block(fwd_steps: int, adj_steps: int) -> None:
-    """Time steps per launch (1 to 4) of the TM2D kernels per pass (see include/tide_hip.h)."""
+    """Time steps per launch (1 to 4; 0: picked from the problem) of the TM2D kernels per
+    pass (see include/tide_hip.h)."""
     check(load().tide_tm2d_set_time_block(int(fwd_steps), int(adj_steps)))
 
 

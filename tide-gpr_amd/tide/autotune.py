@@ -34,14 +34,17 @@ from .maxwell.tm2d import prepare_tm2d
 from .utils import C0
 
 # (rows, group, shot loop, steps per launch, interior/border split,
-#  border tile rows)
+#  border tile rows); 0 steps per launch: the library picks workgroup or
+#  wavefront tiles and their steps from the problem (the default)
 FWD_CANDIDATES: tuple[tuple[int, int, int, int, int, int], ...] = (
+    (4, 1, 0, 0, 0, 0),
     (2, 4, 0, 1, 0, 0), (4, 2, 0, 1, 0, 0), (4, 4, 0, 1, 0, 0), (8, 4, 0, 1, 0, 0),
     (16, 4, 0, 1, 0, 0), (2, 4, 1, 1, 0, 0), (4, 2, 1, 1, 0, 0),
     (2, 2, 0, 2, 0, 0), (4, 1, 0, 2, 0, 0), (4, 2, 0, 2, 0, 0), (4, 4, 0, 2, 0, 0),
     (8, 2, 0, 2, 0, 0), (4, 1, 0, 2, 0, 2), (4, 2, 0, 2, 0, 2),
     (4, 1, 0, 2, 1, 0), (4, 2, 0, 2, 1, 0), (4, 2, 0, 3, 0, 0), (8, 2, 0, 3, 0, 0))
 ADJ_CANDIDATES: tuple[tuple[int, int, int, int, int, int], ...] = (
+    (4, 4, 0, 0, 0, 2),
     (2, 2, 0, 1, 0, 0), (2, 4, 0, 1, 0, 0), (2, 8, 0, 1, 0, 0), (4, 4, 0, 1, 0, 0),
     (8, 2, 0, 1, 0, 0), (2, 4, 1, 1, 0, 0), (4, 2, 1, 1, 0, 0),
     (4, 4, 0, 2, 1, 0), (4, 8, 0, 2, 1, 0), (4, 4, 0, 2, 1, 2), (4, 8, 0, 2, 1, 2),

@@ -80,7 +80,7 @@ class KernelTimer:
              steps_per_launch: int = 1) -> None:
         ev = torch.cuda.Event(enable_timing=True)
         ev.record()
-        self.records.append((name, steps, cells, steps_per_launch, start, ev))
+        self.records.append((name, steps, cells, max(1, steps_per_launch), start, ev))
 
     def summary(self) -> dict[str, dict[str, float]]:
         """Per pass: total ms, launches (time steps / steps per launch), time
