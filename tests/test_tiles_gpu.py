@@ -89,6 +89,16 @@ def test_many_tiles_and_shots_take_the_larger_tiles():
 
 
 @gpu
+@pytest.mark.parametrize("stencil,ny,nx", [(4, 18, 18), (4, 46, 92), (4, 93, 47), (6, 35, 69),
+                                           (8, 33, 51)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("nt", [1, 10])
+def test_higher_orders_beside_the_tile_edges(stencil, ny, nx, dtype, nt):
+    print(f"order {stencil} grid {ny}x{nx} {dtype} nt {nt}", flush=True)
+    _check(_case(ny, nx, nt, stencil=stencil, dtype=dtype))
+
+
+@gpu
 def test_bf16_snapshots_and_per_shot_coefficients():
     _check(_case(60, 75, 19, shots=3), store="bf16")
     _check(_case(60, 75, 19, shots=3, batched=True))

@@ -1014,6 +1014,18 @@ tm2d_ho::Problem<T> ho_problem(const T *ca, const T *cb, const T *cq, const T *c
   return hp;
 }
 
+// Whether a call of stencil order 4, 6 or 8 runs on workgroup tiles: every
+// valid one whose snapshots stay on the device.  (A host-staged call needs the
+// ring slots step by step; an invalid one gets its message from tm2d_ho.)
+template <typename T>
+bool tiled_order(int stencil, const Problem<T> &p, int64_t nt, int fmt, const SnapshotStage &ey,
+                 const SnapshotStage &curl) {
+  const int ny = p.g.ny, nx = p.g.nx;
+  return !ey.active() && !curl.active() && nt > 0 && p.n_shots > 0 && p.n_shots <= 65535 &&
+         ny > stencil && nx > stencil && (int64_t)ny * nx < ((int64_t)1 << 29) &&
+         !(fmt == 2 && sizeof(T) != 4);
+}
+
 template <typename T>
 int forward_entry(T const *ca, T const *cb, T const *cq, T const *f, T *ey, T *hx, T *hz,
                   T *m_ey_x, T *m_ey_z, T *m_hx_z, T *m_hz_x, T *r, T const *ay,
@@ -1054,6 +1066,10 @@ int forward_entry(T const *ca, T const *cb, T const *cq, T const *f, T *ey, T *h
                                                  pml_y1, pml_x1);
     T *const fld[7] = {ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x};
     rc = step_ratio <= 0 ? (set_error("step_ratio must be positive"), (int)kInvalidArgument)
+         : tiled_order(stencil, p, nt, fmt, ey_st, curl_st)
+             ? forward_tiles<T>(stencil / 2, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r,
+                                sources_i, receivers_i, nt, start_t, step_ratio, ey_store,
+                                curl_store, fmt, store_step_bytes, stream, nullptr, 0)
                          : tm2d_ho::forward<T>(stencil, hp, fld, f, r, sources_i, receivers_i, nt,
                                                start_t, step_ratio, ey_store, curl_store, fmt,
                                                store_step_bytes, stream, &ey_st, &curl_st);
@@ -1143,7 +1159,15 @@ int backward_entry(T const *ca, T const *cb, T const *cq, T const *grad_r, T *la
                                                  pml_y1, pml_x1);
     T *const lam[7] = {lambda_ey, lambda_hx, lambda_hz, m_lambda_ey_x, m_lambda_ey_z,
                        m_lambda_hx_z, m_lambda_hz_x};
-    rc = tm2d_ho::backward<T>(stencil, hp, lam, grad_r, ey_store_1, curl_store_1, fmt,
+    if (tiled_order(stencil, p, nt, fmt, ey_st, curl_st) && (!ca_rg || ey_store_1) &&
+        (!cb_rg || curl_store_1))
+      rc = backward_tiles<T>(stencil / 2, p, grad_r, lambda_ey, lambda_hx, lambda_hz,
+                             m_lambda_ey_x, m_lambda_ey_z, m_lambda_hx_z, m_lambda_hz_x,
+                             ey_store_1, curl_store_1, fmt, step_bytes, grad_f,
+                             ca_rg ? ga : nullptr, cb_rg ? gb : nullptr, sources_i, receivers_i, nt,
+                             start_t, step_ratio, stream);
+    else
+      rc = tm2d_ho::backward<T>(stencil, hp, lam, grad_r, ey_store_1, curl_store_1, fmt,
                                 step_bytes, grad_f, ca_rg ? ga : nullptr, cb_rg ? gb : nullptr,
                                 sources_i, receivers_i, nt, start_t, step_ratio, stream, &ey_st,
                                 &curl_st);

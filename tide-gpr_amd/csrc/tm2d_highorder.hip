@@ -5,11 +5,12 @@
 // maxwell_tm_core.cuh:448-599; exact adjoint and reverse loop
 // maxwell_tm_cuda_inst.cu:922-1254, 2540-2731).
 //
-// These orders are the uncommon ones (the reference default and every
-// benchmark workload is order 2, which has the fused, temporally blocked
-// kernels of tm2d_fused.h), so they run one cell per lane: a workgroup is a
-// 64 x 4 tile of one shot (64 consecutive cells of a row per wavefront,
-// coalesced), and every time step is a short sequence of launches:
+// Calls whose snapshots stay on the device run on the workgroup tiles of
+// tm2d_tile.h (one launch for up to four steps).  These kernels serve what
+// those do not: host-staged snapshots, Debye dispersion and the Born products.
+// They run one cell per lane: a workgroup is a 64 x 4 tile of one shot (64
+// consecutive cells of a row per wavefront, coalesced), and every time step is
+// a short sequence of launches:
 //   forward  H half-step, E step (+ snapshots), source injection, receivers;
 //   adjoint  transpose of the E step, transpose of the H half-step,
 //            receiver injection + source-gradient read, FP64 gradient.

@@ -152,13 +152,19 @@ void tile_adj_shape(const TilePlan &p, int fmt, hipStream_t stream, const TileAd
 template <typename T>
 void launch_tile_fwd(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileFwdArgs<T> &a) {
   switch (half) {
-    default: tile_fwd_shape<T, 1>(p, fmt, stream, a); break;
+    case 1: tile_fwd_shape<T, 1>(p, fmt, stream, a); break;
+    case 2: tile_fwd_shape<T, 2>(p, fmt, stream, a); break;
+    case 3: tile_fwd_shape<T, 3>(p, fmt, stream, a); break;
+    default: tile_fwd_shape<T, 4>(p, fmt, stream, a); break;
   }
 }
 template <typename T>
 void launch_tile_adj(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileAdjArgs<T> &a) {
   switch (half) {
-    default: tile_adj_shape<T, 1>(p, fmt, stream, a); break;
+    case 1: tile_adj_shape<T, 1>(p, fmt, stream, a); break;
+    case 2: tile_adj_shape<T, 2>(p, fmt, stream, a); break;
+    case 3: tile_adj_shape<T, 3>(p, fmt, stream, a); break;
+    default: tile_adj_shape<T, 4>(p, fmt, stream, a); break;
   }
 }
 
