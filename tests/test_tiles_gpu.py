@@ -118,3 +118,49 @@ def test_cpml_division_by_held_reciprocal_is_exact():
         got = (d.astype(np.float64) * (1.0 / k.astype(np.float64))).astype(np.float32)
     assert np.array_equal(got, want, equal_nan=True)
     assert np.array_equal(np.signbit(got[want == 0]), np.signbit(want[want == 0]))
+
+
+def _born(case, dca, dcb, df):
+    """born_forward on an oracle case (dca = dcb = None: no scattering)."""
+    ptr = lambda t: 0 if t is None else tide._native.ptr(t)  # noqa: E731
+    dtype = torch.from_numpy(case.ca).dtype
+    d = lambda a: None if a is None else torch.from_numpy(np.ascontiguousarray(a)).to("cuda", dtype)  # noqa: E731
+    bg, sc = [d(x) for x in case.fields], [d(np.zeros_like(x)) for x in case.fields]
+    r = torch.zeros(case.nt, case.n_shots, case.rec.shape[1], device="cuda", dtype=dtype)
+    bg_r = torch.zeros_like(r)
+    fn = getattr(tide._native.load(),
+                 f"maxwell_tm_{case.stencil}_{tide._native.dtype_name(dtype)}_born_forward_cuda")
+    keep = [d(x) for x in (case.ca, case.cb, case.cq, dca, dcb, case.f, df)]
+    prof = [d(x) for x in case.profiles]
+    src, rec = (torch.from_numpy(np.ascontiguousarray(x)) for x in (case.src, case.rec))
+    tide._native.check(fn(
+        *[ptr(t) for t in (*keep, *bg, *sc, r, bg_r, *prof, src, rec)], case.rdy, case.rdx,
+        case.dt, case.nt, case.n_shots, case.ny, case.nx, case.src.shape[1], case.rec.shape[1], 1,
+        False, False, False, 0, *case.pml, 0, 0, tide._native.stream_handle(torch.device("cuda"))))
+    torch.cuda.synchronize()
+    return r.cpu().numpy(), bg_r.cpu().numpy(), [t.cpu().numpy() for t in bg]
+
+
+@gpu
+@pytest.mark.parametrize("stencil", [2, 4, 6, 8])
+@pytest.mark.parametrize("ny,nx,nt", [(17, 130, 1), (49, 65, 7), (33, 49, 8), (40, 97, 17)])
+def test_born_beside_the_tile_edges(stencil, ny, nx, nt):
+    print(f"Born order {stencil} {ny}x{nx} nt {nt}", flush=True)
+    for dtype in (torch.float64, torch.float32):
+        case = _case(ny, nx, nt, stencil=stencil, dtype=dtype)
+        rng = np.random.default_rng(1)
+        dca = (1e-3 * rng.standard_normal((ny, nx))).astype(case.dtype)
+        dcb = (1e-3 * np.abs(case.cb).mean() * rng.standard_normal((ny, nx))).astype(case.dtype)
+        df = (1e-2 * np.abs(case.f).max() * rng.standard_normal(case.f.shape)).astype(case.dtype)
+        f_o, r_f, _, _ = O.tm2d_forward(case)
+        r_o, dr_o = O.tm2d_tangent(case.astype(np.float64), *(a.astype(np.float64)
+                                                              for a in (dca, dcb, df)))
+        dr, r, fields = _born(case, dca, dcb, df)
+        assert np.array_equal(r, r_f)
+        assert all(np.array_equal(a.reshape(b.shape), b) for a, b in zip(fields, f_o))
+        if dtype == torch.float64:
+            assert np.array_equal(r, r_o) and np.array_equal(dr, dr_o)
+        else:  # rounding of at most 17 steps of about 20 fp32 operations each
+            assert relative_l2(dr, dr_o) < 17 * 20 * 2.0**-24
+        none, zero = _born(case, None, None, df), _born(case, 0 * dca, 0 * dcb, df)
+        assert np.array_equal(none[0], zero[0]) and np.array_equal(none[1], r)

@@ -24,7 +24,7 @@ SOURCES = ["tide_common.hip", "tide_storage.hip", "tm2d.hip", "tm2d_highorder.hi
            "tm2d_launch_fwd_f32.hip", "tm2d_launch_fwd_f64.hip", "tm2d_launch_k_fwd_f32.hip",
            "tm2d_launch_k_fwd_f64.hip", "tm2d_launch_k_adj_f32.hip", "tm2d_launch_k_adj_f64.hip",
            "tm2d_tile_fwd_f32.hip", "tm2d_tile_fwd_f64.hip", "tm2d_tile_adj_f32.hip",
-           "tm2d_tile_adj_f64.hip"]
+           "tm2d_tile_adj_f64.hip", "tm2d_tile_born_f32.hip", "tm2d_tile_born_f64.hip"]
 OPTIONAL_SOURCES = ["em3d.hip", "tm2d_batch.hip", "tm2d_serve.hip"]
 ARCH = os.environ.get("TIDE_HIP_ARCH", "gfx950")
 

@@ -118,7 +118,7 @@ template <typename T, int P> struct TileRows {
   T *amp;        // [waves][steps][64]: see TilePoints
   int *entries;  // [waves][3][64] point-table scratch
 
-  static size_t bytes(int waves, int steps) {
+  __host__ __device__ static size_t bytes(int waves, int steps) {
     return (size_t)waves * 64 * ((kRows + steps) * sizeof(T) + 3 * sizeof(int));
   }
   __device__ __forceinline__ TileRows(void *mem, int waves, int steps, int lane) {
@@ -129,6 +129,10 @@ template <typename T, int P> struct TileRows {
     b_first = p + waves * (3 * P - 1) * 64;
     amp = p + waves * kRows * 64;
     entries = (int *)((T *)mem + waves * (kRows + steps) * 64);
+  }
+  // This lane's amplitude of step j.
+  __device__ __forceinline__ const T *amp_at(const TilePlace &c, int steps, int j) const {
+    return amp + (c.w * steps + j) * 64;
   }
 };
 
@@ -291,7 +295,6 @@ template <typename T, int R> struct TilePoints {
   int fast;        // row whose first entries are held (-1: no points at all)
   int first;       // this lane's first entry in that row (-1: none)
   int2 en;
-  T *amp;          // this lane's amplitudes, step stride 64
 
   __device__ __forceinline__ void segment(const Points &pts, int y, int n_shots, int s, int xt,
                                           int &b, int &e) const {
@@ -299,16 +302,12 @@ template <typename T, int R> struct TilePoints {
     b = as_global(pts.seg)[si];
     e = as_global(pts.seg)[si + 1];
   }
-  // kind: of the entries that carry amplitudes (0 sources, 1 receivers);
-  // v: their amplitudes at the first step, `stride` apart from step to step.
   __device__ __forceinline__ void load(const Points &pts, const TilePlace &c, int ny, int n_shots,
-                                       int s, int *entries, T *amps, int steps, int kind,
-                                       const T *v, int64_t stride) {
+                                       int s, int *entries) {
     mask = 0;
     fast = -1;
     first = -1;
     en = make_int2(0, 0);
-    amp = amps + c.w * steps * 64;
 #pragma unroll
     for (int r = R - 1; r >= 0; --r) {
       const int y = c.y + r;
@@ -337,8 +336,15 @@ template <typename T, int R> struct TilePoints {
     first = mine[c.lane];
     if (first < 0) return;
     en = make_int2(mine[64 + c.lane], mine[128 + c.lane]);
-    if (((en.x >> 8) & 1) == kind && v != nullptr)
-      for (int j = 0; j < steps; ++j) amp[j * 64] = as_global(v)[j * stride + en.y];
+  }
+  // Keeps the amplitudes of this lane's first entry, when it is of kind
+  // `kind` (0 source, 1 receiver), in LDS: v holds those of the first step, the
+  // next step's are `stride` on.
+  __device__ __forceinline__ void amplitudes(T *amp, const TilePlace &c, int steps, int kind,
+                                             const T *v, int64_t stride) const {
+    if (first < 0 || v == nullptr || ((en.x >> 8) & 1) != kind) return;
+    amp += c.w * steps * 64;
+    for (int j = 0; j < steps; ++j) amp[j * 64] = as_global(v)[j * stride + en.y];
   }
   // Calls row(r, v) for each row with points, v this lane's value of the row
   // (one copy of the code for all rows).
@@ -353,16 +359,16 @@ template <typename T, int R> struct TilePoints {
       for (int k = 0; k < R; ++k) v[k] = r == k ? x : v[k];
     }
   }
-  // Forward, step j: sources (halo copies too), then receivers (owned cells
-  // only: lanes `own`, rows of the bits `own_rows`).
+  // Forward: sources (halo copies too; `amp` the held amplitude), then
+  // receivers (owned cells only: lanes `own`, rows of the bits `own_rows`).
   __device__ __forceinline__ void forward(const Points &pts, const TilePlace &c, int n_shots, int s,
-                                          int j, const T *f, T *rec, bool own, int own_rows,
-                                          T (&ey)[R]) const {
+                                          const T *amp, const T *f, T *rec, bool own,
+                                          int own_rows, T (&ey)[R]) const {
     each(ey, [&](int r, T &v) {
       const bool mine = own && (own_rows >> r & 1);
       auto one = [&](int2 q, bool held) {
         if (((q.x >> 8) & 1) == 0) {
-          if (f != nullptr) v += held ? amp[j * 64] : as_global(f)[q.y];
+          if (f != nullptr) v += held ? *amp : as_global(f)[q.y];
         } else if (mine && (q.x & kPointCopy) == 0 && rec != nullptr) {
           as_global(rec)[q.y] = v;
         }
@@ -386,15 +392,15 @@ template <typename T, int R> struct TilePoints {
       }
     });
   }
-  // Adjoint, step j: receivers inject (halo copies too), then sources (owned
+  // Adjoint: receivers inject (halo copies too), then sources (owned
   // cells only) read.
   __device__ __forceinline__ void adjoint(const Points &pts, const TilePlace &c, int n_shots, int s,
-                                          int j, const T *gr, T *gf, bool own, int own_rows,
-                                          T (&ley)[R]) const {
+                                          const T *amp, const T *gr, T *gf, bool own,
+                                          int own_rows, T (&ley)[R]) const {
     each(ley, [&](int r, T &v) {
       const bool mine = own && (own_rows >> r & 1) && gf != nullptr;
       auto add = [&](int2 q, bool held) {
-        if (((q.x >> 8) & 1) == 1 && gr != nullptr) v += held ? amp[j * 64] : as_global(gr)[q.y];
+        if (((q.x >> 8) & 1) == 1 && gr != nullptr) v += held ? *amp : as_global(gr)[q.y];
       };
       auto read = [&](int2 q) {
         if (mine && ((q.x >> 8) & 1) == 0 && (q.x & kPointCopy) == 0) as_global(gf)[q.y] = v;
@@ -446,186 +452,240 @@ __device__ __forceinline__ void tile_offsets(const Geom<T> &g, const TilePlace &
 }
 
 // ----------------------------------------------------------------- forward
+// What a forward tile holds beside its fields: lane masks, profiles and the
+// coefficients of its cells.
+template <typename T, int P, int R, bool EDGE> struct TileCells {
+  bool own;                       // this lane's column is owned and inside the grid
+  bool e_col, hz_col;             // in the update domain of Ey and Hx, of Hz
+  bool pml_xe, pml_xh, any_x;     // in an x strip; some lane of the wavefront is
+  RowBits rows;
+  uint32_t at[R];
+  Prof<T> px, pxh;
+  RowProfs<T> yp;
+  T rdy, rdx;
+  T ca[R], cb[R], cq[R];
+
+  __device__ __forceinline__ void set(const Geom<T> &g, const TilePlace &c, int halo) {
+    const int nx = g.nx, x = c.x, x0 = c.x - c.lane;
+    own = c.lane >= halo && c.lane < 64 - halo && x < nx;
+    e_col = !EDGE || (x >= P && x < nx - P + 1);
+    hz_col = !EDGE || (x >= P && x < nx - P);
+    pml_xe = EDGE && (x < g.pml_x0 || x >= g.pml_x1);
+    pml_xh = EDGE && (x < g.pml_x0 || x >= g.pml_x1h);
+    any_x = EDGE && (x0 < g.pml_x0 || x0 + 63 >= g.pml_x1h);
+    rows.set<T, P, R>(g, c, halo);
+    tile_offsets<T, R>(g, c, at);
+    rdy = g.rdy;
+    rdx = g.rdx;
+  }
+  __device__ __forceinline__ void profiles(const Geom<T> &g, const TilePlace &c) {
+    px = pxh = {(T)0, (T)0, 1.0};
+    if constexpr (EDGE) {
+      if (any_x) {
+        const int xc = min(max(c.x, 0), g.nx - 1);
+        px = prof_at<T>(g.px, g.nx, xc, kA);
+        pxh = prof_at<T>(g.px, g.nx, xc, kAh);
+      }
+      yp.load(g, c.y, c.lane);
+    }
+  }
+};
+
+// The fields of a forward tile and the phases of one step, each followed by a
+// barrier: hz() publishes Ey and updates Hz, hx() updates Hx, publishes it and
+// differences Hz, curl() leaves curl H in `d`.
+template <typename T, int P, int R, bool EDGE> struct TileFields {
+  T ey[R], hx[R], hz[R];
+  T mex[R], mez[R], mhxz[R], mhzx[R];
+  T d[R];
+  using Cells = TileCells<T, P, R, EDGE>;
+
+  __device__ __forceinline__ void load(const Cells &k, const T *const *in, int64_t base) {
+    load_rows<T, R>(ey, as_global(in[0]) + base, k.at);
+    load_rows<T, R>(hx, as_global(in[1]) + base, k.at);
+    load_rows<T, R>(hz, as_global(in[2]) + base, k.at);
+  }
+  __device__ __forceinline__ void load_memories(const Cells &k, const T *const *in, int64_t base) {
+    if constexpr (EDGE) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) mex[r] = mez[r] = mhxz[r] = mhzx[r] = (T)0;
+      if (k.any_x) {
+        load_rows<T, R>(mex, as_global(in[3]) + base, k.at);
+        load_rows<T, R>(mhzx, as_global(in[6]) + base, k.at);
+      }
+      if ((k.rows.pe | k.rows.ph) != 0) {
+        load_rows<T, R>(mez, as_global(in[4]) + base, k.at);
+        load_rows<T, R>(mhxz, as_global(in[5]) + base, k.at);
+      }
+    }
+  }
+  __device__ __forceinline__ void update_hz(const Cells &k, const RowBits &b) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      T e[2 * P + 1];
+      lane_window<T, P>(ey[r], e);
+      T v = d_half<T, P>([&](int o) { return e[P + o]; }, k.rdx);
+      if (k.hz_col && (!EDGE || (b.e >> r & 1))) {
+        if (k.pml_xh) {
+          const T m = k.pxh.b * mex[r] + k.pxh.a * v;
+          mex[r] = m;
+          v = k.pxh.over(v) + m;
+        }
+        hz[r] = hz[r] + k.cq[r] * v;
+      }
+    }
+  }
+  __device__ __forceinline__ void update_hx(const Cells &k, const RowBits &b,
+                                            const TileRows<T, P> &lds, const TilePlace &c) {
+    T e[R + 2 * P - 1];
+    get_a<T, P, R>(lds, c, ey, e);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const bool pyh = EDGE && (b.ph >> r & 1);
+      Prof<T> py = {(T)0, (T)0, 1.0};  // read with every lane active
+      if constexpr (EDGE) py = RowProfs<T>::at(k.yp.h, r, pyh);
+      T v = d_half<T, P>([&](int o) { return e[P - 1 + r + o]; }, k.rdy);
+      if (k.e_col && (!EDGE || (b.h >> r & 1))) {
+        if (pyh) {
+          const T m = py.b * mez[r] + py.a * v;
+          mez[r] = m;
+          v = py.over(v) + m;
+        }
+        hx[r] = hx[r] - k.cq[r] * v;
+      }
+    }
+  }
+  __device__ __forceinline__ void difference_hz(const Cells &k) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      T h[2 * P + 1];
+      lane_window<T, P>(hz[r], h);
+      d[r] = d_int<T, P>([&](int o) { return h[P + o]; }, k.rdx);
+    }
+  }
+  __device__ __forceinline__ void curl(const Cells &k, const RowBits &b, const TileRows<T, P> &lds,
+                                       const TilePlace &c) {
+    T h[R + 2 * P - 1];
+    get_b<T, P, R>(lds, c, hx, h);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const bool pye = EDGE && (b.pe >> r & 1);
+      Prof<T> py = {(T)0, (T)0, 1.0};  // read with every lane active
+      if constexpr (EDGE) py = RowProfs<T>::at(k.yp.e, r, pye);
+      T v = d_int<T, P>([&](int o) { return h[P + r + o]; }, k.rdy);
+      if (k.e_col && (!EDGE || (b.e >> r & 1))) {
+        if (k.pml_xe) {
+          const T m = k.px.b * mhzx[r] + k.px.a * d[r];
+          mhzx[r] = m;
+          d[r] = k.px.over(d[r]) + m;
+        }
+        if (pye) {
+          const T m = py.b * mhxz[r] + py.a * v;
+          mhxz[r] = m;
+          v = py.over(v) + m;
+        }
+      }
+      d[r] = d[r] - v;
+    }
+  }
+  // Snapshots of the owned cells of the update domain: Ey before the update
+  // and curl H (either buffer may be absent).
+  template <int FMT>
+  __device__ __forceinline__ void snapshot(const Cells &k, const RowBits &b, void *ey_buf,
+                                           void *curl_buf, int64_t base) const {
+    const int put_rows = EDGE ? b.own & b.e : b.own;
+    auto put = [&](char *buf, const T (&v)[R]) {
+      if (buf == nullptr) return;  // uniform
+      void *const plane = buf + base * (FMT == 2 ? 2 : (int64_t)sizeof(T));
+      if (!(k.own && k.e_col)) return;
+      if (put_rows == (1 << R) - 1) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) put_store32<T, FMT>(plane, k.at[r], v[r]);
+      } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (put_rows >> r & 1) put_store32<T, FMT>(plane, k.at[r], v[r]);
+      }
+    };
+    put(as_global((char *)ey_buf), ey);
+    put(as_global((char *)curl_buf), d);
+  }
+  __device__ __forceinline__ void update_ey(const Cells &k, const RowBits &b) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (k.e_col && (!EDGE || (b.e >> r & 1))) ey[r] = k.ca[r] * ey[r] + k.cb[r] * d[r];
+  }
+  __device__ __forceinline__ void store(const Cells &k, T *const *out, int64_t base) const {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (!(k.rows.own >> r & 1) || !k.own) continue;
+      const uint32_t o = k.at[r];
+      *elem32(as_global(out[0]) + base, o) = ey[r];
+      *elem32(as_global(out[1]) + base, o) = hx[r];
+      *elem32(as_global(out[2]) + base, o) = hz[r];
+      if constexpr (EDGE) {
+        if (k.pml_xh) *elem32(as_global(out[3]) + base, o) = mex[r];
+        if (k.rows.ph >> r & 1) *elem32(as_global(out[4]) + base, o) = mez[r];
+        if (k.rows.pe >> r & 1) *elem32(as_global(out[5]) + base, o) = mhxz[r];
+        if (k.pml_xe) *elem32(as_global(out[6]) + base, o) = mhzx[r];
+      }
+    }
+  }
+};
+
 template <typename T, int P, int R, int FMT, bool EDGE>
 __device__ __forceinline__ void tile_forward(const TilePlace &c, int s, const TileRows<T, P> &lds) {
   using Args = TileFwdArgs<T>;
   constexpr int HS = 2 * P - 1;  // rim cells that go stale per step
   const Args &a = kernel_args<Args>();
   const Geom<T> &g = a.g;
-  const T rdy = g.rdy, rdx = g.rdx;
-  const int steps = a.steps;
-  const int ny = g.ny, nx = g.nx, x = c.x;
-  const int halo = a.halo;
-  const bool own = c.lane >= halo && c.lane < 64 - halo && x < nx;
-  const bool e_col = !EDGE || (x >= P && x < nx - P + 1);
-  const bool hz_col = !EDGE || (x >= P && x < nx - P);
-  const bool pml_xe = EDGE && (x < g.pml_x0 || x >= g.pml_x1);
-  const bool pml_xh = EDGE && (x < g.pml_x0 || x >= g.pml_x1h);
-  // uniform: some lane in an x strip, some row in a y strip
-  const int x0 = x - c.lane;
-  const bool any_x = EDGE && (x0 < g.pml_x0 || x0 + 63 >= g.pml_x1h);
+  const int steps = a.steps, halo = a.halo;
   const int64_t base = (int64_t)s * g.numel;
-  RowBits rows;
-  rows.set<T, P, R>(g, c, halo);
-
-  uint32_t at[R];
-  tile_offsets<T, R>(g, c, at);
-  T ey[R], hx[R], hz[R], ca[R], cb[R], cq[R];
-  load_rows<T, R>(ey, as_global(a.in[0]) + base, at);
-  load_rows<T, R>(hx, as_global(a.in[1]) + base, at);
-  load_rows<T, R>(hz, as_global(a.in[2]) + base, at);
-  load_rows<T, R>(cq, as_global(a.cq) + (g.cq_b ? base : 0), at);
-  load_rows<T, R>(ca, as_global(a.ca) + (g.ca_b ? base : 0), at);
-  load_rows<T, R>(cb, as_global(a.cb) + (g.cb_b ? base : 0), at);
-  T mex[R], mez[R], mhxz[R], mhzx[R];
-  Prof<T> px = {(T)0, (T)0, 1.0}, pxh = px;
-  RowProfs<T> yp;
-  if constexpr (EDGE) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) mex[r] = mez[r] = mhxz[r] = mhzx[r] = (T)0;
-    if (any_x) {
-      const int xc = min(max(x, 0), nx - 1);
-      px = prof_at<T>(g.px, g.nx, xc, kA);
-      pxh = prof_at<T>(g.px, g.nx, xc, kAh);
-      load_rows<T, R>(mex, as_global(a.in[3]) + base, at);
-      load_rows<T, R>(mhzx, as_global(a.in[6]) + base, at);
-    }
-    if ((rows.pe | rows.ph) != 0) {
-      load_rows<T, R>(mez, as_global(a.in[4]) + base, at);
-      load_rows<T, R>(mhxz, as_global(a.in[5]) + base, at);
-    }
-    yp.load(g, c.y, c.lane);
-  }
+  TileCells<T, P, R, EDGE> k;
+  TileFields<T, P, R, EDGE> u;
+  k.set(g, c, halo);
+  u.load(k, a.in, base);
+  load_rows<T, R>(k.cq, as_global(a.cq) + (g.cq_b ? base : 0), k.at);
+  load_rows<T, R>(k.ca, as_global(a.ca) + (g.ca_b ? base : 0), k.at);
+  load_rows<T, R>(k.cb, as_global(a.cb) + (g.cb_b ? base : 0), k.at);
+  k.profiles(g, c);
+  u.load_memories(k, a.in, base);
   TilePoints<T, R> points;
-  points.load(a.pts, c, ny, a.n_shots, s, lds.entries, lds.amp, a.steps, 0, a.f, a.f_stride);
+  points.load(a.pts, c, g.ny, a.n_shots, s, lds.entries);
+  points.amplitudes(lds.amp, c, steps, 0, a.f, a.f_stride);
   wait_loads();
 
   for (int j = 0; j < steps; ++j) {
     // rows whose new values are still needed; the rest of the tile is stale
     const int lo = halo - (steps - 1 - j) * HS, hi = c.rows - lo;
     const bool active = c.row0 < hi + P - 1 && c.row0 + R > lo - P;  // uniform
-    const RowBits b = rows.again();
-    put_a<T, P, R>(lds, c, ey);
-    if (active) {  // Hz: x neighbours only
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        T e[2 * P + 1];
-        lane_window<T, P>(ey[r], e);
-        T d = d_half<T, P>([&](int o) { return e[P + o]; }, rdx);
-        if (hz_col && (!EDGE || (b.e >> r & 1))) {
-          if (pml_xh) {
-            const T m = pxh.b * mex[r] + pxh.a * d;
-            mex[r] = m;
-            d = pxh.over(d) + m;
-          }
-          hz[r] = hz[r] + cq[r] * d;
-        }
-      }
-    }
+    const RowBits b = k.rows.again();
+    put_a<T, P, R>(lds, c, u.ey);
+    if (active) u.update_hz(k, b);
+    __syncthreads();
+    if (active) u.update_hx(k, b, lds, c);
+    put_b<T, P, R>(lds, c, u.hx);
+    if (active) u.difference_hz(k);
     __syncthreads();
     if (active) {
-      T e[R + 2 * P - 1];
-      get_a<T, P, R>(lds, c, ey, e);
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const bool pyh = EDGE && (b.ph >> r & 1);
-        Prof<T> py = {(T)0, (T)0, 1.0};  // read with every lane active
-        if constexpr (EDGE) py = RowProfs<T>::at(yp.h, r, pyh);
-        T d = d_half<T, P>([&](int o) { return e[P - 1 + r + o]; }, rdy);
-        if (e_col && (!EDGE || (b.h >> r & 1))) {
-          if (pyh) {
-            const T m = py.b * mez[r] + py.a * d;
-            mez[r] = m;
-            d = py.over(d) + m;
-          }
-          hx[r] = hx[r] - cq[r] * d;
-        }
-      }
-    }
-    put_b<T, P, R>(lds, c, hx);
-    T dhz[R];
-    if (active) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        T h[2 * P + 1];
-        lane_window<T, P>(hz[r], h);
-        dhz[r] = d_int<T, P>([&](int o) { return h[P + o]; }, rdx);
-      }
-    }
-    __syncthreads();
-    if (active) {
-      T h[R + 2 * P - 1];
-      get_b<T, P, R>(lds, c, hx, h);
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const bool row = !EDGE || (b.e >> r & 1);
-        const bool pye = EDGE && (b.pe >> r & 1);
-        Prof<T> py = {(T)0, (T)0, 1.0};  // read with every lane active
-        if constexpr (EDGE) py = RowProfs<T>::at(yp.e, r, pye);
-        T dhx = d_int<T, P>([&](int o) { return h[P + r + o]; }, rdy);
-        if (e_col && row) {
-          if (pml_xe) {
-            const T m = px.b * mhzx[r] + px.a * dhz[r];
-            mhzx[r] = m;
-            dhz[r] = px.over(dhz[r]) + m;
-          }
-          if (pye) {
-            const T m = py.b * mhxz[r] + py.a * dhx;
-            mhxz[r] = m;
-            dhx = py.over(dhx) + m;
-          }
-        }
-        dhz[r] = dhz[r] - dhx;  // curl H
-      }
+      u.curl(k, b, lds, c);
       if constexpr (FMT != 0) {
-        const int put_rows = EDGE ? b.own & b.e : b.own;
-        auto put = [&](char *buf, const T (&v)[R]) {
-          if (buf == nullptr) return;  // uniform
-          void *const plane = buf + base * (FMT == 2 ? 2 : (int64_t)sizeof(T));
-          if (!(own && e_col)) return;
-          if (put_rows == (1 << R) - 1) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) put_store32<T, FMT>(plane, at[r], v[r]);
-          } else {
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-              if (put_rows >> r & 1) put_store32<T, FMT>(plane, at[r], v[r]);
-          }
-        };
-        if (put_rows != 0) {  // uniform
+        if (b.own != 0) {  // uniform
           const Args &q = kernel_args<Args>();
-          put(as_global((char *)q.ey_store[j]), ey);
-          put(as_global((char *)q.curl_store[j]), dhz);
+          u.template snapshot<FMT>(k, b, q.ey_store[j], q.curl_store[j], base);
         }
       }
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (e_col && (!EDGE || (b.e >> r & 1))) ey[r] = ca[r] * ey[r] + cb[r] * dhz[r];
-      }
+      u.update_ey(k, b);
       if (points.fast >= 0) {  // uniform
         const Args &q = kernel_args<Args>();
         const T *const f = q.f != nullptr ? q.f + j * q.f_stride : nullptr;
         T *const rec = q.r != nullptr ? q.r + j * q.r_stride : nullptr;
-        points.forward(q.pts, c, q.n_shots, s, j, f, rec, own, b.own, ey);
+        points.forward(q.pts, c, q.n_shots, s, lds.amp_at(c, steps, j), f, rec, k.own, b.own, u.ey);
       }
     }
   }
-
   const Args &z = kernel_args<Args>();
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (!(rows.own >> r & 1) || !own) continue;
-    const uint32_t o = at[r];
-    *elem32(as_global(z.out[0]) + base, o) = ey[r];
-    *elem32(as_global(z.out[1]) + base, o) = hx[r];
-    *elem32(as_global(z.out[2]) + base, o) = hz[r];
-    if constexpr (EDGE) {
-      if (pml_xh) *elem32(as_global(z.out[3]) + base, o) = mex[r];
-      if (rows.ph >> r & 1) *elem32(as_global(z.out[4]) + base, o) = mez[r];
-      if (rows.pe >> r & 1) *elem32(as_global(z.out[5]) + base, o) = mhxz[r];
-      if (pml_xe) *elem32(as_global(z.out[6]) + base, o) = mhzx[r];
-    }
-  }
+  u.store(k, z.out, base);
 }
 
 template <typename T, int P, int R, int W, int FMT>
@@ -640,6 +700,131 @@ __global__ __launch_bounds__(64 * W) void tile_fwd(TileFwdArgs<T>) {
     tile_forward<T, P, R, FMT, true>(c, s, lds);
   else
     tile_forward<T, P, R, FMT, false>(c, s, lds);
+}
+
+// ------------------------------------------------------------ Born forward
+// The background and the Born-scattered field of a tile together: the
+// scattered Ey update adds dca Ey^n + dcb curl H^n of the background (its values
+// before this step's update, still in registers).
+template <typename T> struct TileBornArgs {
+  Geom<T> g;
+  Points pts;
+  const T *ca, *cb, *cq, *dca, *dcb;  // dca, dcb null: no scattering term
+  const T *in[14];                    // the background's seven arrays, then the scattered field's
+  T *out[14];
+  const T *f0, *df;                   // source terms of the first step
+  T *bg_r, *r;                        // receiver rows of the first step
+  int64_t f_stride, r_stride;
+  void *hist[4];  // Ey^n, curl^n of the background, of the scattered field; first
+  int64_t hist_stride;  // step's planes, the next step's hist_stride bytes on
+  int32_t n_shots, steps, halo, own_rows;
+};
+
+template <typename T, int P, int R, bool STORE, bool EDGE>
+__device__ __forceinline__ void tile_born_step(const TilePlace &c, int s, const TileRows<T, P> &lds,
+                                               const TileRows<T, P> &lds2) {
+  using Args = TileBornArgs<T>;
+  constexpr int HS = 2 * P - 1;
+  const Args &a = kernel_args<Args>();
+  const Geom<T> &g = a.g;
+  const int steps = a.steps, halo = a.halo;
+  const int64_t base = (int64_t)s * g.numel;
+  TileCells<T, P, R, EDGE> k;
+  TileFields<T, P, R, EDGE> u, v;  // background, scattered
+  T da[R], db[R];
+  k.set(g, c, halo);
+  u.load(k, a.in, base);
+  v.load(k, a.in + 7, base);
+  load_rows<T, R>(k.cq, as_global(a.cq) + (g.cq_b ? base : 0), k.at);
+  load_rows<T, R>(k.ca, as_global(a.ca) + (g.ca_b ? base : 0), k.at);
+  load_rows<T, R>(k.cb, as_global(a.cb) + (g.cb_b ? base : 0), k.at);
+  const bool scatter = a.dca != nullptr;
+  if (scatter) {
+    load_rows<T, R>(da, as_global(a.dca) + (g.ca_b ? base : 0), k.at);
+    load_rows<T, R>(db, as_global(a.dcb) + (g.cb_b ? base : 0), k.at);
+  }
+  k.profiles(g, c);
+  u.load_memories(k, a.in, base);
+  v.load_memories(k, a.in + 7, base);
+  TilePoints<T, R> points;
+  points.load(a.pts, c, g.ny, a.n_shots, s, lds.entries);
+  points.amplitudes(lds.amp, c, steps, 0, a.f0, a.f_stride);
+  points.amplitudes(lds2.amp, c, steps, 0, a.df, a.f_stride);
+  wait_loads();
+
+  for (int j = 0; j < steps; ++j) {
+    const int lo = halo - (steps - 1 - j) * HS, hi = c.rows - lo;
+    const bool active = c.row0 < hi + P - 1 && c.row0 + R > lo - P;  // uniform
+    const RowBits b = k.rows.again();
+    put_a<T, P, R>(lds, c, u.ey);
+    put_a<T, P, R>(lds2, c, v.ey);
+    if (active) {
+      u.update_hz(k, b);
+      v.update_hz(k, b);
+    }
+    __syncthreads();
+    if (active) {
+      u.update_hx(k, b, lds, c);
+      v.update_hx(k, b, lds2, c);
+    }
+    put_b<T, P, R>(lds, c, u.hx);
+    put_b<T, P, R>(lds2, c, v.hx);
+    if (active) {
+      u.difference_hz(k);
+      v.difference_hz(k);
+    }
+    __syncthreads();
+    if (active) {
+      u.curl(k, b, lds, c);
+      v.curl(k, b, lds2, c);
+      if constexpr (STORE) {
+        if (b.own != 0) {  // uniform
+          const Args &q = kernel_args<Args>();
+          const int64_t at = j * q.hist_stride;
+          u.template snapshot<1>(k, b, (char *)q.hist[0] + at, (char *)q.hist[1] + at, base);
+          v.template snapshot<1>(k, b, (char *)q.hist[2] + at, (char *)q.hist[3] + at, base);
+        }
+      }
+      v.update_ey(k, b);
+      if (scatter) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (k.e_col && (!EDGE || (b.e >> r & 1)))
+            v.ey[r] = v.ey[r] + (da[r] * u.ey[r] + db[r] * u.d[r]);
+      }
+      u.update_ey(k, b);
+      if (points.fast >= 0) {  // uniform
+        const Args &q = kernel_args<Args>();
+        const int64_t fo = j * q.f_stride, ro = j * q.r_stride;
+        points.forward(q.pts, c, q.n_shots, s, lds.amp_at(c, steps, j),
+                       q.f0 != nullptr ? q.f0 + fo : nullptr,
+                       q.bg_r != nullptr ? q.bg_r + ro : nullptr, k.own, b.own, u.ey);
+        points.forward(q.pts, c, q.n_shots, s, lds2.amp_at(c, steps, j),
+                       q.df != nullptr ? q.df + fo : nullptr,
+                       q.r != nullptr ? q.r + ro : nullptr, k.own, b.own, v.ey);
+      }
+    }
+  }
+  const Args &z = kernel_args<Args>();
+  u.store(k, z.out, base);
+  v.store(k, z.out + 7, base);
+}
+
+template <typename T, int P, int R, int W, bool STORE>
+__global__ __launch_bounds__(64 * W) void tile_born(TileBornArgs<T>) {
+  const TileBornArgs<T> &a = kernel_args<TileBornArgs<T>>();
+  extern __shared__ double tile_lds[];
+  const int waves = (int)blockDim.y;
+  const TileRows<T, P> lds(tile_lds, waves, a.steps, (int)threadIdx.x);
+  const TileRows<T, P> lds2((char *)tile_lds + TileRows<T, P>::bytes(waves, a.steps), waves, a.steps,
+                            (int)threadIdx.x);
+  const int flat = (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x);
+  const int tile = flat / a.n_shots, s = flat - tile * a.n_shots;
+  const TilePlace c = tile_place<T, P, R>(a.g, a.pts.n_xt, tile, a.halo, a.own_rows);
+  if (c.edge)  // uniform over the workgroup
+    tile_born_step<T, P, R, STORE, true>(c, s, lds, lds2);
+  else
+    tile_born_step<T, P, R, STORE, false>(c, s, lds, lds2);
 }
 
 // ----------------------------------------------------------------- adjoint
@@ -710,8 +895,8 @@ __device__ __forceinline__ void tile_adjoint(const TilePlace &c, int s0, int s1,
       }
     }
     TilePoints<T, R> points;
-    points.load(a.pts, c, ny, a.n_shots, s, lds.entries, lds.amp, a.steps, 1, a.grad_r,
-                -a.r_stride);
+    points.load(a.pts, c, g.ny, a.n_shots, s, lds.entries);
+    points.amplitudes(lds.amp, c, steps, 1, a.grad_r, -a.r_stride);
     wait_loads();
 
     for (int j = 0; j < steps; ++j) {
@@ -840,7 +1025,7 @@ __device__ __forceinline__ void tile_adjoint(const TilePlace &c, int s0, int s1,
           const Args &q = kernel_args<Args>();
           const T *const gr = q.grad_r != nullptr ? q.grad_r - j * q.r_stride : nullptr;
           T *const gf = q.grad_f != nullptr ? q.grad_f - j * q.f_stride : nullptr;
-          points.adjoint(q.pts, c, q.n_shots, s, j, gr, gf, own, b.own, ley);
+          points.adjoint(q.pts, c, q.n_shots, s, lds.amp_at(c, steps, j), gr, gf, own, b.own, ley);
         }
         if constexpr (FMT != 0) {
           if (have) {  // uniform; rim cells hold snapshots of 0 or are never added

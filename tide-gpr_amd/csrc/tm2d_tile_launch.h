@@ -1,6 +1,6 @@
 // Launch plan and launchers of the workgroup-tile kernels (tm2d_tile.h).
 // The definitions compile in one translation unit per pass and field type
-// (tm2d_tile_{fwd,adj}_{f32,f64}.hip).
+// (tm2d_tile_{fwd,adj,born}_{f32,f64}.hip).
 #pragma once
 
 #include "tm2d_tile.h"
@@ -100,10 +100,40 @@ bool prefer_tiles(int ny, int nx, int n_shots, bool adjoint, bool storing) {
   return us < wave;
 }
 
+// The Born kernel's tiles: 32 rows (two field sets fill the registers that one
+// takes in a 64-row tile), by 16 wavefronts of 2 rows in fp32 up to order 4, else
+// by 8 of 4 (wide stencils exchange up to 4 rows; two sets of doubles need the
+// 256 registers of 8 wavefronts, and their LDS rows fit 160 KB).
+constexpr int kBornRows = 32;
+template <typename T> constexpr int born_rows(int half) {
+  return sizeof(T) == 4 && half <= 2 ? 2 : 4;
+}
+
+template <typename T> TilePlan plan_born(int half, int ny, int nx, int n_shots) {
+  const int rows = born_rows<T>(half), waves = kBornRows / rows;
+  TilePlan best{};
+  double best_us = 1e30;
+  for (int steps = 1; steps <= kTileSteps; ++steps) {
+    const int halo = steps * (2 * half - 1);
+    if (kBornRows - 2 * halo < kBornRows / 4) break;
+    const TilePlan p = make_tile_plan(half, ny, nx, waves, rows, steps, 1);
+    const double rounds = std::max(1.0, (double)p.n_xt * p.n_yt * n_shots / 256.0);
+    const double us = std::min(std::ceil(rounds), rounds + 0.3) *
+                      (10.0 + (rows == 2 ? 1.8 : 3.0) * steps) / steps;
+    if (us < best_us) {
+      best_us = us;
+      best = p;
+    }
+  }
+  return best;
+}
+
 template <typename T>
 void launch_tile_fwd(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileFwdArgs<T> &a);
 template <typename T>
 void launch_tile_adj(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileAdjArgs<T> &a);
+template <typename T>
+void launch_tile_born(int half, const TilePlan &p, bool store, hipStream_t stream, const TileBornArgs<T> &a);
 
 #ifdef TIDE_TM2D_TILE_DEFINITIONS
 
@@ -165,6 +195,28 @@ void launch_tile_adj(int half, const TilePlan &p, int fmt, hipStream_t stream, c
     case 2: tile_adj_shape<T, 2>(p, fmt, stream, a); break;
     case 3: tile_adj_shape<T, 3>(p, fmt, stream, a); break;
     default: tile_adj_shape<T, 4>(p, fmt, stream, a); break;
+  }
+}
+
+template <typename T, int P>
+void tile_born_shape(const TilePlan &p, bool store, hipStream_t stream, const TileBornArgs<T> &a) {
+  constexpr int R = born_rows<T>(P), W = kBornRows / R;
+  const dim3 block(64, (unsigned)p.waves);
+  const unsigned grid = (unsigned)((int64_t)p.n_xt * p.n_yt * a.n_shots);
+  const size_t lds = 2 * TileRows<T, P>::bytes(p.waves, a.steps);
+  if (store)
+    tile_born<T, P, R, W, true><<<grid, block, lds, stream>>>(a);
+  else
+    tile_born<T, P, R, W, false><<<grid, block, lds, stream>>>(a);
+}
+
+template <typename T>
+void launch_tile_born(int half, const TilePlan &p, bool store, hipStream_t stream, const TileBornArgs<T> &a) {
+  switch (half) {
+    case 1: tile_born_shape<T, 1>(p, store, stream, a); break;
+    case 2: tile_born_shape<T, 2>(p, store, stream, a); break;
+    case 3: tile_born_shape<T, 3>(p, store, stream, a); break;
+    default: tile_born_shape<T, 4>(p, store, stream, a); break;
   }
 }
 
