@@ -1730,10 +1730,10 @@ int maxwell_3d_2_double_backward_cuda(
     int64_t execution_backend, void *compute_stream, void *storage_stream);
 
 /*
- * Launch shape of the 3-D step kernels: z planes marched per wavefront
- * (forward 4/8/16, adjoint 4/8) and shots per workgroup (1..8, both
- * passes).  Defaults: 8 / 4 planes, 1 shot per forward workgroup, 8 per
- * adjoint workgroup.  No reference counterpart.
+ * Launch shape of the 3-D step kernels: shots per workgroup (1..8, both
+ * passes; defaults 1 forward, 8 adjoint).  fwd_z (4/8/16) and adj_z (4/8)
+ * are checked and have no effect: a wavefront takes consecutive cells of a
+ * volume whatever its planes.  No reference counterpart.
  */
 int tide_em3d_set_tuning(int fwd_z, int adj_z, int group);
 
@@ -1765,8 +1765,8 @@ int tide_em3d_set_fused(int rows, int planes);
 int tide_em3d_get_fused(int *out2);
 
 /*
- * Workgroup order of the 3-D kernels: 0 runs all tiles of one shot group
- * before the next group, 1 runs the shot groups of one tile next to each
+ * Workgroup order of the 3-D kernels: 0 runs all cells of one shot group
+ * before the next group, 1 runs the shot groups of the same cells next to each
  * other (same XCD, shared L2 for the coefficient lines).  Results do not
  * depend on it.  No reference counterpart.
  */

@@ -38,7 +38,7 @@ template <typename T> struct Fused3 {
   const T *src_amp;
   T *rec_out;
   int32_t n_shots, n_yt, n_zb, src_comp, rec_comp;
-  int32_t shot_fast;  // workgroup order, as decode3
+  int32_t shot_fast;  // workgroup order: the shot groups of a tile adjacent
 };
 
 // CPML correction reading the memory from `mi` and writing the new one to

@@ -92,6 +92,12 @@ bool build_point_table_lanes(const int64_t *src, int64_t n_src, const int64_t *r
                              int64_t n_rec, int64_t n_shots, int64_t ny, int64_t nx,
                              int tile_w, int lane_offset, PointTable &out);
 
+// The rows are runs of `chunk` consecutive cells of the ny x nx plane (any
+// length up to 256), xloc the position in the run.
+bool build_point_table_chunks(const int64_t *src, int64_t n_src, const int64_t *rec,
+                              int64_t n_rec, int64_t n_shots, int64_t ny, int64_t nx, int chunk,
+                              PointTable &out);
+
 // Device copy of a PointTable: either three device allocations of its own
 // (upload) or three caller-provided arrays of the sizes below (place).
 struct DevicePointTable {

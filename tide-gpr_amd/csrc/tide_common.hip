@@ -17,9 +17,11 @@ const char *last_error() { return g_last_error.c_str(); }
 namespace {
 bool build_table(const int64_t *src, int64_t n_src, const int64_t *rec, int64_t n_rec,
                  int64_t n_shots, int64_t ny, int64_t nx, int tile_w, int lane_offset,
-                 bool halo, bool by_lane, PointTable &out) {
+                 bool halo, bool by_lane, PointTable &out, int chunk = 0) {
   const int64_t numel = ny * nx;
-  const int64_t n_xt = (nx + tile_w - 1) / tile_w;
+  const int64_t n_rows = chunk > 0 ? (numel + chunk - 1) / chunk : ny;
+  const int64_t row_len = chunk > 0 ? chunk : nx;
+  const int64_t n_xt = (row_len + tile_w - 1) / tile_w;
   // (y, shot, xt, kind, k, xloc, q); kind bit 1 marks a halo copy
   struct Entry {
     int64_t y, shot, xt, kind, k;
@@ -42,7 +44,7 @@ bool build_table(const int64_t *src, int64_t n_src, const int64_t *rec, int64_t 
           set_error(buf);
           return false;
         }
-        const int64_t y = v / nx, x = v % nx;
+        const int64_t y = v / row_len, x = v % row_len;
         const int64_t xt = x / tile_w;
         const int32_t lane = (int32_t)(x % tile_w + lane_offset);
         entries.push_back({y, s, xt, kind, k, lane, (int32_t)(s * n + k)});
@@ -70,7 +72,7 @@ bool build_table(const int64_t *src, int64_t n_src, const int64_t *rec, int64_t 
     });
   }
   out.n_xt = (int32_t)n_xt;
-  out.row_slot.assign((size_t)ny, -1);
+  out.row_slot.assign((size_t)n_rows, -1);
   std::vector<int64_t> rows;
   for (const Entry &e : entries)
     if (rows.empty() || rows.back() != e.y) rows.push_back(e.y);
@@ -120,6 +122,12 @@ bool build_point_table_lanes(const int64_t *src, int64_t n_src, const int64_t *r
                              int64_t n_rec, int64_t n_shots, int64_t ny, int64_t nx,
                              int tile_w, int lane_offset, PointTable &out) {
   return build_table(src, n_src, rec, n_rec, n_shots, ny, nx, tile_w, lane_offset, true, true, out);
+}
+
+bool build_point_table_chunks(const int64_t *src, int64_t n_src, const int64_t *rec,
+                              int64_t n_rec, int64_t n_shots, int64_t ny, int64_t nx, int chunk,
+                              PointTable &out) {
+  return build_table(src, n_src, rec, n_rec, n_shots, ny, nx, chunk, 0, false, false, out, chunk);
 }
 
 int DevicePointTable::upload(const PointTable &t, hipStream_t stream) {

@@ -400,8 +400,8 @@ def set_tm2d_tuning(fwd_rows: int, fwd_group: int, adj_rows: int, adj_group: int
 
 
 def set_em3d_tuning(fwd_z: int, adj_z: int, group: int) -> None:
-    """z planes marched per wavefront (forward, adjoint) and shots per
-    workgroup of the 3-D kernels (see include/tide_hip.h)."""
+    """Shots per workgroup of the 3-D kernels; fwd_z and adj_z are checked and
+    have no effect (see include/tide_hip.h)."""
     check(load().tide_em3d_set_tuning(fwd_z, adj_z, group))
 
 
