@@ -758,6 +758,11 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
   const size_t bytes = (size_t)total * sizeof(T);
 
   AdjArgs<T> a;
+  a.g = p.g;
+  a.pts = Points{dpt.row_slot, dpt.seg, dpt.ent, dpt.n_xt};
+  a.ca = p.ca;
+  a.cb = p.cb;
+  a.cq = p.cq;
   a.per_shot_grad = ((gca && p.g.ca_b) || (gcb && p.g.cb_b)) ? 1 : 0;
   a.step_scale = (double)step_ratio;
   a.n_shots = p.n_shots;
