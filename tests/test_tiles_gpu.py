@@ -164,3 +164,53 @@ def test_born_beside_the_tile_edges(stencil, ny, nx, nt):
             assert relative_l2(dr, dr_o) < 17 * 20 * 2.0**-24
         none, zero = _born(case, None, None, df), _born(case, 0 * dca, 0 * dcb, df)
         assert np.array_equal(none[0], zero[0]) and np.array_equal(none[1], r)
+
+
+@gpu
+@pytest.mark.parametrize("compression,interval,graph", [(False, 1, True), (False, 3, False),
+                                                        (True, 2, True)])
+def test_batched_plans_on_tiles(compression, interval, graph):
+    """Problems of one and of several tiles and shots, whose loops take one
+    launch, an even and an odd last launch: receivers, states and source
+    gradients as the oracle's, replayed twice."""
+    from tide.batch import TM2DBatch
+
+    dev = torch.device("cuda:0")
+    sizes = [(30, 44, 23, 2), (9, 8, 1, 1), (70, 121, 16, 3), (25, 90, 7, 11), (12, 33, 9, 1)]
+    problems = []
+    for ny, nx, nt, shots in sizes:
+        g = torch.Generator().manual_seed(ny)
+        dx = 0.01
+        dt = 0.7 * dx / (2**0.5 * tide.C0)
+        amp = tide.ricker(9e8, nt + 8, dt, peak_time=4 * dt)[:nt].reshape(1, 1, -1).repeat(shots, 2, 1)
+        src = torch.stack([torch.tensor([[1 + s % (ny - 2), 2], [1 + s % (ny - 2), 2]])
+                           for s in range(shots)])
+        rec = torch.stack([torch.tensor([[2, x] for x in range(0, nx, 2)])] * shots)
+        problems.append(dict(
+            epsilon=(1 + 8 * torch.rand(ny, nx, generator=g)).to(dev),
+            sigma=(0.01 * torch.rand(ny, nx, generator=g)).to(dev),
+            mu=torch.ones(ny, nx, device=dev), grid_spacing=dx, dt=dt,
+            source_amplitude=amp.to(dev), source_location=src.to(dev),
+            receiver_location=rec.to(dev), pml_width=[3, 4, 5, 2]))
+    batch = TM2DBatch(problems, storage_compression=compression, use_graph=graph,
+                      model_gradient_sampling_interval=interval)
+    store = "bf16" if compression else "full"
+    cases = [O.case_from_setup(prepare_tm2d(**kw)) for kw in problems]
+    rng = np.random.default_rng(4)
+    for replay in range(2):
+        batch.reset_state()
+        rs = [r.cpu().numpy() for r in batch.forward()]
+        ws = [rng.standard_normal(r.shape).astype(np.float32) for r in rs]
+        states = [[t.cpu().numpy() for t in st.fields] for st in batch.setups]
+        out = [[t.cpu().numpy() for t in ts]
+               for ts in batch.backward([torch.from_numpy(w).to(dev) for w in ws])]
+        for size, case, r, w, state, (ga, gb, gf) in zip(sizes, cases, rs, ws, states, out):
+            print(f"replay {replay} problem {size}", flush=True)
+            f_o, r_o, es, cs = O.tm2d_forward(case, store=store, interval=interval)
+            assert np.array_equal(r, r_o)
+            assert all(np.array_equal(a.reshape(b.shape), b) for a, b in zip(state, f_o))
+            ga_o, gb_o, gf_o, _ = O.tm2d_backward(case, w, es, cs, store=store, interval=interval)
+            assert np.array_equal(gf.reshape(gf_o.shape), gf_o)
+            for a, b in ((ga, ga_o), (gb, gb_o)):
+                assert relative_l2(a.reshape(b.shape), b) < 1e-12 if b.any() else not a.any()
+    batch.close()

@@ -131,6 +131,7 @@ struct Scratch {
   hipStream_t stream;
   char *arena = nullptr;
   size_t cap = 0, used = 0;
+  bool full = false;  // an allocation did not fit
   explicit Scratch(hipStream_t s, char *arena_ = nullptr, size_t cap_ = 0)
       : stream(s), arena(arena_), cap(cap_) {}
   ~Scratch() {
@@ -141,6 +142,7 @@ struct Scratch {
     if (arena != nullptr) {
       const size_t at = (used + 255) & ~(size_t)255;
       if (at + bytes > cap) {
+        full = true;
         set_error("the call needs more scratch memory than the fixed scratch array holds (" +
                   std::to_string(cap >> 20) + " MiB)");
         return kInvalidArgument;
@@ -247,19 +249,6 @@ int upload_points_lanes(const Problem<T> &p, const TilePlan &plan, const int64_t
     return kInvalidArgument;
   return put_table(table, dpt, arena_scr, stream);
 }
-
-// Steps of each launch of a time loop of nt steps, at most `most` each: the
-// fewest launches, an even number of them where nt allows it (the state ping-
-// pongs between the caller's arrays and a scratch copy, and an even count ends
-// in the caller's arrays), as equal as possible.
-struct LaunchSteps {
-  int64_t nt, launches;
-  LaunchSteps(int64_t nt_, int most) : nt(nt_), launches((nt_ + most - 1) / most) {
-    if ((launches & 1) && nt > launches) ++launches;
-  }
-  int at(int64_t k) const { return (int)(nt * (k + 1) / launches - nt * k / launches); }
-  bool ends_in_scratch() const { return (launches & 1) != 0; }
-};
 
 // The N state arrays of a time loop and the scratch copy they ping-pong with.
 // open() comes before any other use of the device: a problem whose copy does

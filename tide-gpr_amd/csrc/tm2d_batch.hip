@@ -1,8 +1,11 @@
 // Batched 2-D TM plans: many independent problems (different grid sizes,
-// shot counts and nt) advanced together, one launch per time step, or (the
-// default, as in the single-problem path) one launch per two time steps
-// with the two-step kernels of tm2d_fused.h; a problem whose nt is odd takes
-// its last step in a one-step launch over its own tiles.
+// shot counts and nt) advanced together.  By default the time loops run on
+// workgroup tiles (tm2d_tile.h): one launch advances every problem by up to 8
+// steps, each from its own argument record; all problems share one tile shape
+// and step count per pass, chosen for the whole batch.  As settings, and for
+// the adjoint of large batches: one launch per time step, or one per two
+// time steps with the two-step kernels of tm2d_fused.h; a problem whose nt is
+// odd takes its last step in a one-step launch over its own tiles.
 //
 // Every problem keeps its own arrays; a plan holds a device table with one
 // descriptor per problem and a tile -> problem map.  Problems are sorted by
@@ -22,6 +25,7 @@
 
 #include "tide_hip.h"
 #include "tm2d_items.h"
+#include "tm2d_tile_launch.h"
 
 #include <algorithm>
 #include <cstring>
@@ -107,7 +111,30 @@ __global__ void fill_zero(T *__restrict__ p, int64_t n) {
     p[i] = (T)0;
 }
 
+// Zeroes ranges[blockIdx.y] of 32-bit words.
+struct FillRange {
+  uint32_t *p;
+  int64_t words;
+};
+__global__ void fill_ranges(const FillRange *__restrict__ ranges) {
+  const FillRange r = ranges[blockIdx.y];
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < r.words;
+       i += (int64_t)gridDim.x * blockDim.x)
+    r.p[i] = 0;
+}
+
 // ------------------------------------------------------------------ plan
+
+// A pass of a plan on workgroup tiles.
+template <typename A> struct TilePass {
+  TilePlan plan{};
+  int64_t launches = 0;
+  A *table = nullptr;          // [launches][problems]
+  int32_t *tile_item = nullptr;
+  std::vector<int64_t> grid;   // workgroups of launch k
+  FillRange *fills = nullptr;  // arrays that a run starts from zero
+  int64_t n_fills = 0;
+};
 
 struct Plan {
   int device = 0;
@@ -116,6 +143,9 @@ struct Plan {
   int rows_f = 8, rows_a = 4, group = 8;
   int steps_f = 1, steps_a = 1;  // time steps per launch of each pass
   int max_nt = 0;
+  bool tiles_f = false, tiles_a = false;  // the passes on workgroup tiles
+  TilePass<TileFwdArgs<float>> tile_f;
+  TilePass<TileAdjArgs<float>> tile_a;
   std::vector<tide_tm2d_problem> probs;  // sorted by nt, descending
   std::vector<void *> allocs;            // plan-owned device memory
   BatchItem<float> *d_fwd = nullptr, *d_adj = nullptr;
@@ -232,8 +262,67 @@ void launch_pair_a(const Plan &p, int fmt, int64_t grid, hipStream_t s, int k, i
   else adj2_batch<float, TY, 1><<<(unsigned)grid, block, lds, s>>>(p.d_adj, p.d_tiles2a, k, par);
 }
 
+template <typename A> void fill_all(const TilePass<A> &t, hipStream_t s) {
+  for (int64_t i = 0; i < t.n_fills; i += 65535)  // the grid's y limit
+    fill_ranges<<<dim3(64, (unsigned)std::min<int64_t>(t.n_fills - i, 65535)), 256, 0, s>>>(t.fills + i);
+}
+
+// Copies array c of every problem that ends in the scratch copy, back (or, for
+// the strips' memories before the loop, there: their cells outside the strips
+// are never written).
+int copy_scratch_state(const Plan &p, hipStream_t s, bool forward, bool back) {
+  for (size_t m = 0; m < p.probs.size(); ++m) {
+    const tide_tm2d_problem &q = p.probs[m];
+    if (!LaunchSteps(q.nt, (forward ? p.tile_f.plan : p.tile_a.plan).steps).ends_in_scratch()) continue;
+    const size_t bytes = (size_t)(q.n_shots * q.ny * q.nx) * sizeof(float);
+    const BatchItem<float> &it = (forward ? p.h_fwd : p.h_adj)[m];
+    for (int c = back ? 0 : 3; c < 7; ++c) {
+      float *const own = forward ? (c < 5 ? it.fwd[0][c] : (c == 5 ? it.mhxz : it.mhzx)) : it.lam[0][c];
+      float *const copy = forward ? (c < 5 ? it.fwd[1][c] : (c == 5 ? it.mhxz_b : it.mhzx_b)) : it.lam[1][c];
+      TIDE_HIP_TRY(hipMemcpyAsync(back ? own : copy, back ? copy : own, bytes, hipMemcpyDeviceToDevice, s));
+    }
+  }
+  return kOk;
+}
+
+int enqueue_forward_tiles(Plan &p, hipStream_t s) {
+  fill_all(p.tile_f, s);
+  PLAN_CHECK(copy_scratch_state(p, s, true, false));
+  for (int64_t k = 0; k < p.tile_f.launches; ++k)
+    launch_tile_fwd_items(p.tile_f.plan, p.fmt_fwd, p.tile_f.grid[(size_t)k], s,
+                          p.tile_f.table + k * (int64_t)p.probs.size(), p.tile_f.tile_item);
+  PLAN_CHECK(copy_scratch_state(p, s, true, true));
+  TIDE_HIP_TRY(hipGetLastError());
+  return kOk;
+}
+
+void fold_all(const Plan &p, hipStream_t s) {
+  for (size_t m = 0; m < p.probs.size(); ++m) {
+    const BatchItem<float> &it = p.h_adj[m];
+    if (it.group_stride == 0) continue;
+    const tide_tm2d_problem &q = p.probs[m];
+    const int64_t numel = q.ny * q.nx;
+    const unsigned blocks = (unsigned)((numel + 255) / 256);
+    if (it.gca) fold_groups<<<blocks, 256, 0, s>>>(q.grad_ca, it.gca, numel, it.n_groups);
+    if (it.gcb) fold_groups<<<blocks, 256, 0, s>>>(q.grad_cb, it.gcb, numel, it.n_groups);
+  }
+}
+
+int enqueue_backward_tiles(Plan &p, hipStream_t s) {
+  fill_all(p.tile_a, s);
+  PLAN_CHECK(copy_scratch_state(p, s, false, false));
+  for (int64_t k = 0; k < p.tile_a.launches; ++k)
+    launch_tile_adj_items(p.tile_a.plan, p.fmt_adj, p.tile_a.grid[(size_t)k], s,
+                          p.tile_a.table + k * (int64_t)p.probs.size(), p.tile_a.tile_item);
+  fold_all(p, s);
+  PLAN_CHECK(copy_scratch_state(p, s, false, true));
+  TIDE_HIP_TRY(hipGetLastError());
+  return kOk;
+}
+
 // Enqueues one whole forward run on `s`.
 int enqueue_forward(Plan &p, hipStream_t s) {
+  if (p.tiles_f) return enqueue_forward_tiles(p, s);
   const size_t fb = sizeof(float);
   for (size_t m = 0; m < p.probs.size(); ++m) {
     const tide_tm2d_problem &q = p.probs[m];
@@ -285,6 +374,7 @@ int enqueue_forward(Plan &p, hipStream_t s) {
 
 // Enqueues one whole adjoint run on `s` (adjoint state and gradients start at zero).
 int enqueue_backward(Plan &p, hipStream_t s) {
+  if (p.tiles_a) return enqueue_backward_tiles(p, s);
   const size_t fb = sizeof(float);
   for (size_t m = 0; m < p.probs.size(); ++m) {
     const tide_tm2d_problem &q = p.probs[m];
@@ -316,15 +406,7 @@ int enqueue_backward(Plan &p, hipStream_t s) {
       launch_step_a(p, p.fmt_adj, grid, s, k, 0, k & 1);
     }
   }
-  for (size_t m = 0; m < p.probs.size(); ++m) {
-    const BatchItem<float> &it = p.h_adj[m];
-    if (it.group_stride == 0) continue;
-    const tide_tm2d_problem &q = p.probs[m];
-    const int64_t numel = q.ny * q.nx;
-    const unsigned blocks = (unsigned)((numel + 255) / 256);
-    if (it.gca) fold_groups<<<blocks, 256, 0, s>>>(q.grad_ca, it.gca, numel, it.n_groups);
-    if (it.gcb) fold_groups<<<blocks, 256, 0, s>>>(q.grad_cb, it.gcb, numel, it.n_groups);
-  }
+  fold_all(p, s);
   for (size_t m = 0; m < p.probs.size(); ++m) {
     const tide_tm2d_problem &q = p.probs[m];
     if ((((p.steps_a == 2) ? (q.nt + 1) / 2 : q.nt) & 1) == 0) continue;
@@ -366,6 +448,20 @@ void destroy(Plan *p) {
   for (void *a : p->allocs) (void)hipFree(a);
   if (p->capture) (void)hipStreamDestroy(p->capture);
   delete p;
+}
+
+// Captures the time loops, when the plan replays graphs.
+int start_graphs(Plan &p) {
+  if (p.use_graph) {
+    if (hipStreamCreateWithFlags(&p.capture, hipStreamNonBlocking) != hipSuccess) {
+      set_error("plan: stream creation failed");
+      return kHipError;
+    }
+    PLAN_CHECK(capture(p, true, &p.gr_fwd, &p.g_fwd));
+    const bool any_adj = p.probs[0].lambda[0] != nullptr;
+    if (any_adj) PLAN_CHECK(capture(p, false, &p.gr_adj, &p.g_adj));
+  }
+  return kOk;
 }
 
 // Builds descriptors for one tile shape; returns the tile -> item map.
@@ -475,6 +571,206 @@ int build_items2(Plan &p, std::vector<int32_t> &tile_item, std::vector<int32_t> 
   return kOk;
 }
 
+// Workgroups of each launch for a tile plan of the whole batch (problems sorted
+// by nt, descending, so that launches are too).
+std::vector<int64_t> tile_grids(const Plan &p, const TilePlan &t) {
+  std::vector<int64_t> grid;
+  for (const tide_tm2d_problem &q : p.probs) {
+    const TilePlan one = make_tile_plan(1, (int)q.ny, (int)q.nx, t.waves, t.rows, t.steps, 1);
+    const int64_t n = (int64_t)one.n_xt * one.n_yt * q.n_shots, l = LaunchSteps(q.nt, t.steps).launches;
+    if ((int64_t)grid.size() < l) grid.resize((size_t)l, 0);
+    for (int64_t k = 0; k < l; ++k) grid[(size_t)k] += n;
+  }
+  return grid;
+}
+
+// Tile shape and steps per launch of a batch: the least modelled time of the
+// whole loop (see plan_tiles).
+TilePlan plan_batch_tiles(const Plan &p, bool adjoint, bool storing) {
+  TilePlan best{};
+  double best_us = 1e300;
+  for (int rows = 2; rows <= 4; rows += 2) {
+    for (int steps = 1; steps <= kTileSteps; ++steps) {
+      const TilePlan t = make_tile_plan(1, 1, 1, kTileWaves, rows, steps, 1);
+      double us = 0.0;
+      for (int64_t n : tile_grids(p, t)) {
+        const double r = (double)n / 256.0;
+        us += (r <= 1.0 ? 1.0 : std::min(std::ceil(r), r + 0.3)) *
+              tile_launch_us<float>(1, rows, steps, adjoint, storing);
+      }
+      if (us < best_us) {
+        best_us = us;
+        best = t;
+      }
+    }
+  }
+  return best;
+}
+
+// Argument records, workgroup map and zeroed ranges of one pass.
+template <typename A>
+int upload_pass(Plan &p, TilePass<A> &t, const std::vector<A> &table,
+                const std::vector<int32_t> &tile_item, const std::vector<FillRange> &fills) {
+  PLAN_CHECK(plan_alloc(p, &t.table, table.size()));
+  PLAN_CHECK(plan_alloc(p, &t.tile_item, tile_item.size()));
+  PLAN_CHECK(plan_alloc(p, &t.fills, fills.size()));
+  TIDE_HIP_TRY(hipMemcpy(t.table, table.data(), table.size() * sizeof(A), hipMemcpyHostToDevice));
+  TIDE_HIP_TRY(hipMemcpy(t.tile_item, tile_item.data(), tile_item.size() * sizeof(int32_t),
+                         hipMemcpyHostToDevice));
+  TIDE_HIP_TRY(hipMemcpy(t.fills, fills.data(), fills.size() * sizeof(FillRange), hipMemcpyHostToDevice));
+  t.n_fills = (int64_t)fills.size();
+  return kOk;
+}
+
+// Problem m's share of a pass: its plan, point table and workgroups.
+int tile_problem(Plan &p, size_t m, const TilePlan &t, TilePlan &one, Points &pts,
+                 std::vector<int32_t> &tile_item) {
+  const tide_tm2d_problem &q = p.probs[m];
+  one = make_tile_plan(1, (int)q.ny, (int)q.nx, t.waves, t.rows, t.steps, 1);
+  std::vector<int64_t> hs, hr;
+  PLAN_CHECK(fetch_host(q.sources_i, q.n_shots * q.n_src, hs));
+  PLAN_CHECK(fetch_host(q.receivers_i, q.n_shots * q.n_rec, hr));
+  PointTable table;
+  if (!build_point_table_lanes(hs.data(), q.n_src, hr.data(), q.n_rec, q.n_shots, q.ny, q.nx,
+                               one.own_cols, one.halo, table))
+    return kInvalidArgument;
+  p.dpts.emplace_back();
+  PLAN_CHECK(p.dpts.back().upload(table, nullptr));
+  const DevicePointTable &d = p.dpts.back();
+  pts = Points{d.row_slot, d.seg, d.ent, d.n_xt};
+  const int64_t n = (int64_t)one.n_xt * one.n_yt * q.n_shots;
+  if ((int64_t)tile_item.size() + n >= ((int64_t)1 << 31)) {
+    set_error("batch: too many tiles for one launch");
+    return kInvalidArgument;
+  }
+  tile_item.insert(tile_item.end(), (size_t)n, (int32_t)m);
+  return kOk;
+}
+
+int build_tiles_forward(Plan &p) {
+  TilePass<TileFwdArgs<float>> &t = p.tile_f;
+  t.plan = plan_batch_tiles(p, false, p.fmt_fwd != 0);
+  t.grid = tile_grids(p, t.plan);
+  t.launches = (int64_t)t.grid.size();
+  const size_t n = p.probs.size();
+  std::vector<TileFwdArgs<float>> table((size_t)t.launches * n);
+  std::vector<int32_t> tile_item;
+  std::vector<FillRange> fills;
+  for (size_t m = 0; m < n; ++m) {
+    const tide_tm2d_problem &q = p.probs[m];
+    const BatchItem<float> &it = p.h_fwd[m];
+    TileFwdArgs<float> a;
+    std::memset(&a, 0, sizeof(a));
+    a.tile0 = (int32_t)tile_item.size();
+    TilePlan one;
+    PLAN_CHECK(tile_problem(p, m, t.plan, one, a.pts, tile_item));
+    a.g = it.g;
+    a.ca = q.ca;
+    a.cb = q.cb;
+    a.cq = q.cq;
+    a.n_shots = (int32_t)q.n_shots;
+    a.halo = one.halo;
+    a.own_rows = one.own_rows;
+    a.f_stride = q.n_shots * q.n_src;
+    a.r_stride = q.n_shots * q.n_rec;
+    float *const state[2][7] = {
+        {it.fwd[0][0], it.fwd[0][1], it.fwd[0][2], it.fwd[0][3], it.fwd[0][4], it.mhxz, it.mhzx},
+        {it.fwd[1][0], it.fwd[1][1], it.fwd[1][2], it.fwd[1][3], it.fwd[1][4], it.mhxz_b, it.mhzx_b}};
+    const LaunchSteps loop(q.nt, t.plan.steps);
+    int64_t s = 0;
+    for (int64_t k = 0; k < loop.launches; ++k) {
+      a.steps = loop.at(k);
+      for (int c = 0; c < 7; ++c) {
+        a.in[c] = state[k & 1][c];
+        a.out[c] = state[(k & 1) ^ 1][c];
+      }
+      a.f = q.n_src > 0 ? q.f + s * a.f_stride : nullptr;
+      a.r = q.n_rec > 0 ? q.r + s * a.r_stride : nullptr;
+      for (int j = 0; j < kTileSteps; ++j) {
+        const bool on = j < a.steps && (s + j) % q.interval == 0;
+        const int64_t at = (s + j) / q.interval * it.store_step_bytes;
+        a.ey_store[j] = on && q.ey_store ? (char *)q.ey_store + at : nullptr;
+        a.curl_store[j] = on && q.curl_store ? (char *)q.curl_store + at : nullptr;
+      }
+      table[(size_t)k * n + m] = a;
+      s += a.steps;
+    }
+    if (q.n_rec > 0) fills.push_back({(uint32_t *)q.r, q.nt * q.n_shots * q.n_rec});
+  }
+  return upload_pass(p, t, table, tile_item, fills);
+}
+
+int build_tiles_backward(Plan &p) {
+  TilePass<TileAdjArgs<float>> &t = p.tile_a;
+  t.plan = plan_batch_tiles(p, true, p.fmt_adj != 0);
+  t.grid = tile_grids(p, t.plan);
+  t.launches = (int64_t)t.grid.size();
+  const size_t n = p.probs.size();
+  std::vector<TileAdjArgs<float>> table((size_t)t.launches * n);
+  std::vector<int32_t> tile_item;
+  std::vector<FillRange> fills;
+  for (size_t m = 0; m < n; ++m) {
+    const tide_tm2d_problem &q = p.probs[m];
+    BatchItem<float> &it = p.h_adj[m];
+    const int64_t numel = q.ny * q.nx, total = q.n_shots * numel;
+    TileAdjArgs<float> a;
+    std::memset(&a, 0, sizeof(a));
+    a.tile0 = (int32_t)tile_item.size();
+    TilePlan one;
+    PLAN_CHECK(tile_problem(p, m, t.plan, one, a.pts, tile_item));
+    a.g = it.g;
+    a.ca = q.ca;
+    a.cb = q.cb;
+    a.cq = q.cq;
+    a.step_scale = (double)q.interval;
+    a.n_shots = (int32_t)q.n_shots;
+    a.halo = one.halo;
+    a.own_rows = one.own_rows;
+    a.group = 1;
+    a.r_stride = q.n_shots * q.n_rec;
+    a.f_stride = q.n_shots * q.n_src;
+    // one FP64 slice per shot, folded in shot order after the loop
+    it.n_groups = a.n_shots;
+    if (q.n_shots > 1 && (q.grad_ca || q.grad_cb)) {
+      it.group_stride = a.group_stride = numel;
+      if (q.grad_ca) PLAN_CHECK(plan_alloc(p, &it.gca, (size_t)total));
+      if (q.grad_cb) PLAN_CHECK(plan_alloc(p, &it.gcb, (size_t)total));
+    }
+    const LaunchSteps loop(q.nt, t.plan.steps);
+    int64_t s = q.nt - 1;
+    for (int64_t k = 0; k < loop.launches; ++k) {
+      a.steps = loop.at(k);
+      for (int c = 0; c < 7; ++c) {
+        a.in[c] = it.lam[k & 1][c];
+        a.out[c] = it.lam[(k & 1) ^ 1][c];
+      }
+      a.grad_r = q.n_rec > 0 ? q.grad_r + s * a.r_stride : nullptr;
+      a.grad_f = q.n_src > 0 && q.grad_f ? q.grad_f + s * a.f_stride : nullptr;
+      bool any = false;
+      for (int j = 0; j < kTileSteps; ++j) {
+        const bool on = j < a.steps && (s - j) % q.interval == 0;
+        const int64_t at = on ? (s - j) / q.interval * it.store_step_bytes : 0;
+        a.ey_store[j] = on && q.grad_ca ? (const char *)q.ey_store + at : nullptr;
+        a.curl_store[j] = on && q.grad_cb ? (const char *)q.curl_store + at : nullptr;
+        any = any || a.ey_store[j] || a.curl_store[j];
+      }
+      a.gca = any && q.grad_ca ? it.gca : nullptr;
+      a.gcb = any && q.grad_cb ? it.gcb : nullptr;
+      table[(size_t)k * n + m] = a;
+      s -= a.steps;
+    }
+    for (int c = 0; c < 7; ++c) fills.push_back({(uint32_t *)it.lam[0][c], total});
+    if (q.grad_ca) fills.push_back({(uint32_t *)q.grad_ca, 2 * numel});
+    if (q.grad_cb) fills.push_back({(uint32_t *)q.grad_cb, 2 * numel});
+    if (it.group_stride > 0) {
+      if (q.grad_ca) fills.push_back({(uint32_t *)it.gca, 2 * total});
+      if (q.grad_cb) fills.push_back({(uint32_t *)it.gcb, 2 * total});
+    }
+    if (q.grad_f && q.n_src > 0) fills.push_back({(uint32_t *)q.grad_f, q.nt * q.n_shots * q.n_src});
+  }
+  return upload_pass(p, t, table, tile_item, fills);
+}
+
 }  // namespace
 }  // namespace tm2d
 }  // namespace tide_hip
@@ -510,6 +806,47 @@ extern "C" int tide_tm2d_plan_create(const tide_tm2d_problem *problems, int64_t 
 }
 
 namespace {
+// Descriptors, workgroup maps and launch sizes of the one- and two-step launches.
+int build_step_launches(Plan &p, const std::vector<BatchItem<float>> &proto, bool two) {
+  std::vector<int32_t> tiles_f, tiles_a;
+  PLAN_CHECK(build_items(p, p.rows_f, p.h_fwd, tiles_f, p.active_fwd, proto));
+  PLAN_CHECK(build_items(p, p.rows_a, p.h_adj, tiles_a, p.active_adj, proto));
+  std::vector<int32_t> tiles2, tiles2a;
+  if (two) PLAN_CHECK(build_items2(p, tiles2, tiles2a));
+  // problems with several shot groups accumulate into per-group FP64 slices
+  for (size_t m = 0; m < p.probs.size(); ++m) {
+    BatchItem<float> &it = p.h_adj[m];
+    it.group_stride = 0;
+    if (it.n_groups > 1 && (it.gca || it.gcb)) {
+      const int64_t numel = p.probs[m].ny * p.probs[m].nx;
+      it.group_stride = numel;
+      if (it.gca) PLAN_CHECK(plan_alloc(p, &it.gca, (size_t)(it.n_groups * numel)));
+      if (it.gcb) PLAN_CHECK(plan_alloc(p, &it.gcb, (size_t)(it.n_groups * numel)));
+    }
+  }
+  PLAN_CHECK(plan_alloc(p, &p.d_fwd, p.h_fwd.size()));
+  PLAN_CHECK(plan_alloc(p, &p.d_adj, p.h_adj.size()));
+  PLAN_CHECK(plan_alloc(p, &p.d_tiles_fwd, tiles_f.size()));
+  PLAN_CHECK(plan_alloc(p, &p.d_tiles_adj, tiles_a.size()));
+  if (two) {
+    PLAN_CHECK(plan_alloc(p, &p.d_tiles2, tiles2.size()));
+    TIDE_HIP_TRY(hipMemcpy(p.d_tiles2, tiles2.data(), tiles2.size() * sizeof(int32_t),
+                           hipMemcpyHostToDevice));
+    PLAN_CHECK(plan_alloc(p, &p.d_tiles2a, tiles2a.size()));
+    TIDE_HIP_TRY(hipMemcpy(p.d_tiles2a, tiles2a.data(), tiles2a.size() * sizeof(int32_t),
+                           hipMemcpyHostToDevice));
+  }
+  TIDE_HIP_TRY(hipMemcpy(p.d_fwd, p.h_fwd.data(), p.h_fwd.size() * sizeof(BatchItem<float>),
+                         hipMemcpyHostToDevice));
+  TIDE_HIP_TRY(hipMemcpy(p.d_adj, p.h_adj.data(), p.h_adj.size() * sizeof(BatchItem<float>),
+                         hipMemcpyHostToDevice));
+  TIDE_HIP_TRY(hipMemcpy(p.d_tiles_fwd, tiles_f.data(), tiles_f.size() * sizeof(int32_t),
+                         hipMemcpyHostToDevice));
+  TIDE_HIP_TRY(hipMemcpy(p.d_tiles_adj, tiles_a.data(), tiles_a.size() * sizeof(int32_t),
+                         hipMemcpyHostToDevice));
+  return kOk;
+}
+
 int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t storage_format,
                int64_t use_graph, int64_t device) {
   p->device = (int)device;
@@ -518,10 +855,23 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
   p->rows_f = rows_for<float>(g_tuning.fwd_rows);
   p->rows_a = rows_for<float>(g_tuning.adj_rows);
   p->group = g_tuning.adj_group;  // one group size for both passes
-  // plans run one- or two-step launches (a K-step setting runs at 2)
+  // One- or two-step launches as set (a K-step setting runs at 2).  Where
+  // neither pass has a setting the forward runs on tiles, the adjoint up to
+  // kBatchTileCells padded cells.  fp32, us per step, tiles / two-step launches,
+  // forward with snapshots and adjoint: 24 grids of 81 x 101 cells (x 1 shot)
+  // 3.4 / 9.8 and 6.3 / 21; 12 of 241 x 261 x 3 12 / 19 and 21 / 34; 12 of 341 x
+  // 361 x 4 27 / 40 and 49 / 51; 8 of 541 x 561 x 4 54 / 70 and 87 / 82; 8 of
+  // 741 x 781 x 4 107 / 139 and 144 / 139.
+  constexpr int64_t kBatchTileCells = 7000000;
+  int64_t cells = 0;
+  for (int64_t m = 0; m < n; ++m)
+    cells += std::max<int64_t>(problems[m].n_shots, 0) * std::max<int64_t>(problems[m].ny, 0) *
+             std::max<int64_t>(problems[m].nx, 0);
+  p->tiles_f = g_tuning.fwd_steps == 0 && g_tuning.adj_steps == 0;
+  p->tiles_a = p->tiles_f && cells <= kBatchTileCells;
   p->steps_f = g_tuning.fwd_steps == 1 ? 1 : 2;
   p->steps_a = g_tuning.adj_steps == 1 ? 1 : 2;
-  const bool two = p->steps_f == 2 || p->steps_a == 2;
+  const bool two = !p->tiles_a && (p->steps_f == 2 || p->steps_a == 2);
   p->probs.assign(problems, problems + n);
   std::stable_sort(p->probs.begin(), p->probs.end(),
                    [](const tide_tm2d_problem &a, const tide_tm2d_problem &b) { return a.nt > b.nt; });
@@ -529,7 +879,7 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
   bool any_store = false, any_grad = false;
   auto fail = [](int rc) { return rc; };
   std::vector<BatchItem<float>> proto(p->probs.size());
-  p->dpts.reserve(p->probs.size());
+  p->dpts.reserve(3 * p->probs.size());
   p->dpts2.reserve(p->probs.size());
   for (size_t m = 0; m < p->probs.size(); ++m) {
     const tide_tm2d_problem &q = p->probs[m];
@@ -576,18 +926,19 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
     }
     g.py = pbuf;
     g.px = pbuf + (size_t)6 * q.ny;
-    // point table
     std::vector<int64_t> hs, hr;
     PLAN_CHECK(fetch_host(q.sources_i, q.n_shots * q.n_src, hs));
     PLAN_CHECK(fetch_host(q.receivers_i, q.n_shots * q.n_rec, hr));
-    PointTable table;
-    if (!build_point_table(hs.data(), q.n_src, hr.data(), q.n_rec, q.n_shots, q.ny, q.nx, kOwn,
-                           1, table))
-      return fail(kInvalidArgument);
-    p->dpts.emplace_back();
-    DevicePointTable &dpt = p->dpts.back();
-    PLAN_CHECK(dpt.upload(table, nullptr));
-    it.pts = Points{dpt.row_slot, dpt.seg, dpt.ent, dpt.n_xt};
+    if (!p->tiles_a) {
+      PointTable table;
+      if (!build_point_table(hs.data(), q.n_src, hr.data(), q.n_rec, q.n_shots, q.ny, q.nx, kOwn,
+                             1, table))
+        return fail(kInvalidArgument);
+      p->dpts.emplace_back();
+      DevicePointTable &dpt = p->dpts.back();
+      PLAN_CHECK(dpt.upload(table, nullptr));
+      it.pts = Points{dpt.row_slot, dpt.seg, dpt.ent, dpt.n_xt};
+    }
     if (two) {  // point table of the two-step tiles (halo copies included)
       PointTable table2;
       if (!build_point_table_halo(hs.data(), q.n_src, hr.data(), q.n_rec, q.n_shots, q.ny, q.nx,
@@ -649,53 +1000,15 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
   }
   p->fmt_fwd = any_store ? fmt : 0;
   p->fmt_adj = any_grad ? fmt : 0;
-  std::vector<int32_t> tiles_f, tiles_a;
-  PLAN_CHECK(build_items(*p, p->rows_f, p->h_fwd, tiles_f, p->active_fwd, proto));
-  PLAN_CHECK(build_items(*p, p->rows_a, p->h_adj, tiles_a, p->active_adj, proto));
-  std::vector<int32_t> tiles2, tiles2a;
-  if (two) PLAN_CHECK(build_items2(*p, tiles2, tiles2a));
-  // problems with several shot groups accumulate into per-group FP64 slices
-  for (size_t m = 0; m < p->probs.size(); ++m) {
-    BatchItem<float> &it = p->h_adj[m];
-    it.group_stride = 0;
-    if (it.n_groups > 1 && (it.gca || it.gcb)) {
-      const int64_t numel = p->probs[m].ny * p->probs[m].nx;
-      it.group_stride = numel;
-      if (it.gca) PLAN_CHECK(plan_alloc(*p, &it.gca, (size_t)(it.n_groups * numel)));
-      if (it.gcb) PLAN_CHECK(plan_alloc(*p, &it.gcb, (size_t)(it.n_groups * numel)));
-    }
+  if (p->tiles_a) {
+    p->h_fwd = p->h_adj = proto;
+  } else {
+    PLAN_CHECK(build_step_launches(*p, proto, two));
   }
-  PLAN_CHECK(plan_alloc(*p, &p->d_fwd, p->h_fwd.size()));
-  PLAN_CHECK(plan_alloc(*p, &p->d_adj, p->h_adj.size()));
-  PLAN_CHECK(plan_alloc(*p, &p->d_tiles_fwd, tiles_f.size()));
-  PLAN_CHECK(plan_alloc(*p, &p->d_tiles_adj, tiles_a.size()));
-  if (two) {
-    PLAN_CHECK(plan_alloc(*p, &p->d_tiles2, tiles2.size()));
-    TIDE_HIP_TRY(hipMemcpy(p->d_tiles2, tiles2.data(), tiles2.size() * sizeof(int32_t),
-                           hipMemcpyHostToDevice));
-    PLAN_CHECK(plan_alloc(*p, &p->d_tiles2a, tiles2a.size()));
-    TIDE_HIP_TRY(hipMemcpy(p->d_tiles2a, tiles2a.data(), tiles2a.size() * sizeof(int32_t),
-                           hipMemcpyHostToDevice));
-  }
-  TIDE_HIP_TRY(hipMemcpy(p->d_fwd, p->h_fwd.data(), p->h_fwd.size() * sizeof(BatchItem<float>),
-                         hipMemcpyHostToDevice));
-  TIDE_HIP_TRY(hipMemcpy(p->d_adj, p->h_adj.data(), p->h_adj.size() * sizeof(BatchItem<float>),
-                         hipMemcpyHostToDevice));
-  TIDE_HIP_TRY(hipMemcpy(p->d_tiles_fwd, tiles_f.data(), tiles_f.size() * sizeof(int32_t),
-                         hipMemcpyHostToDevice));
-  TIDE_HIP_TRY(hipMemcpy(p->d_tiles_adj, tiles_a.data(), tiles_a.size() * sizeof(int32_t),
-                         hipMemcpyHostToDevice));
+  if (p->tiles_f) PLAN_CHECK(build_tiles_forward(*p));
+  if (p->tiles_a && p->probs[0].lambda[0] != nullptr) PLAN_CHECK(build_tiles_backward(*p));
   TIDE_HIP_TRY(hipDeviceSynchronize());
-  if (p->use_graph) {
-    if (hipStreamCreateWithFlags(&p->capture, hipStreamNonBlocking) != hipSuccess) {
-      set_error("plan: stream creation failed");
-      return fail(kHipError);
-    }
-    PLAN_CHECK(capture(*p, true, &p->gr_fwd, &p->g_fwd));
-    const bool any_adj = p->probs[0].lambda[0] != nullptr;
-    if (any_adj) PLAN_CHECK(capture(*p, false, &p->gr_adj, &p->g_adj));
-  }
-  return kOk;
+  return start_graphs(*p);
 }
 }  // namespace
 

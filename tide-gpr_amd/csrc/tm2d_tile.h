@@ -44,6 +44,7 @@ template <typename T> struct TileFwdArgs {
   int64_t f_stride, r_stride;  // step's are one stride further
   void *ey_store[kTileSteps], *curl_store[kTileSteps];  // null: no snapshot
   int32_t n_shots, steps, halo, own_rows;
+  int32_t tile0;  // first workgroup of the problem in a launch of several
 };
 
 template <typename T> struct TileAdjArgs {
@@ -59,22 +60,29 @@ template <typename T> struct TileAdjArgs {
   double *gca, *gcb;  // FP64 accumulators; null: not wanted
   int32_t per_shot_grad;
   double step_scale;
-  int32_t n_shots, steps, halo, own_rows, group;
+  int32_t n_shots, steps, halo, own_rows, group, tile0;
   int64_t group_stride;  // shot group k adds into gca / gcb + k * group_stride
 };
 
-// The kernel's one argument, read anew: the compiler loads every kernel
-// argument it can at the kernel's start and keeps it for its last use, which
-// overflows the scalar registers; values read through this reference are
-// loaded where they are used.
-template <typename A> __device__ __forceinline__ const A &kernel_args() {
+// A kernel's arguments, read anew at each call: the compiler loads every
+// kernel argument it can at the kernel's start and keeps it for its last use,
+// which overflows the scalar registers; values read through this reference are
+// loaded where they are used.  The arguments are those of the kernel itself, or
+// an entry of a table that was complete before the launch.
+template <typename A> struct ArgRef {
   using P = const A __attribute__((address_space(4))) *;
-  P p = (P)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(p));
-  return *(const A *)p;
+  P p;
+  __device__ __forceinline__ const A &operator()() const {
+    P q = p;
+    asm volatile("" : "+s"(q));
+    return *(const A *)q;
+  }
+};
+template <typename A> __device__ __forceinline__ ArgRef<A> kernel_args() {
+  return {(typename ArgRef<A>::P)__builtin_amdgcn_kernarg_segment_ptr()};
 }
 
-// A pointer read through kernel_args(), which the compiler does not know to
+// A pointer read through an ArgRef, which the compiler does not know to
 // point to global memory (it would use flat accesses, whose waits include LDS).
 template <typename U> __device__ __forceinline__ U *as_global(U *p) {
   using G = U __attribute__((address_space(1))) *;
@@ -634,10 +642,11 @@ template <typename T, int P, int R, bool EDGE> struct TileFields {
 };
 
 template <typename T, int P, int R, int FMT, bool EDGE>
-__device__ __forceinline__ void tile_forward(const TilePlace &c, int s, const TileRows<T, P> &lds) {
+__device__ __forceinline__ void tile_forward(ArgRef<TileFwdArgs<T>> args, const TilePlace &c, int s,
+                                             const TileRows<T, P> &lds) {
   using Args = TileFwdArgs<T>;
   constexpr int HS = 2 * P - 1;  // rim cells that go stale per step
-  const Args &a = kernel_args<Args>();
+  const Args &a = args();
   const Geom<T> &g = a.g;
   const int steps = a.steps, halo = a.halo;
   const int64_t base = (int64_t)s * g.numel;
@@ -671,35 +680,51 @@ __device__ __forceinline__ void tile_forward(const TilePlace &c, int s, const Ti
       u.curl(k, b, lds, c);
       if constexpr (FMT != 0) {
         if (b.own != 0) {  // uniform
-          const Args &q = kernel_args<Args>();
+          const Args &q = args();
           u.template snapshot<FMT>(k, b, q.ey_store[j], q.curl_store[j], base);
         }
       }
       u.update_ey(k, b);
       if (points.fast >= 0) {  // uniform
-        const Args &q = kernel_args<Args>();
+        const Args &q = args();
         const T *const f = q.f != nullptr ? q.f + j * q.f_stride : nullptr;
         T *const rec = q.r != nullptr ? q.r + j * q.r_stride : nullptr;
         points.forward(q.pts, c, q.n_shots, s, lds.amp_at(c, steps, j), f, rec, k.own, b.own, u.ey);
       }
     }
   }
-  const Args &z = kernel_args<Args>();
+  const Args &z = args();
   u.store(k, z.out, base);
+}
+
+// Workgroup `flat` of a problem.
+template <typename T, int P, int R, int FMT>
+__device__ __forceinline__ void tile_fwd_group(ArgRef<TileFwdArgs<T>> args, int flat) {
+  extern __shared__ double tile_lds[];
+  const TileFwdArgs<T> &a = args();
+  const TileRows<T, P> lds(tile_lds, (int)blockDim.y, a.steps, (int)threadIdx.x);
+  const int tile = flat / a.n_shots, s = flat - tile * a.n_shots;
+  const TilePlace c = tile_place<T, P, R>(a.g, a.pts.n_xt, tile, a.halo, a.own_rows);
+  if (c.edge)  // uniform over the workgroup
+    tile_forward<T, P, R, FMT, true>(args, c, s, lds);
+  else
+    tile_forward<T, P, R, FMT, false>(args, c, s, lds);
 }
 
 template <typename T, int P, int R, int W, int FMT>
 __global__ __launch_bounds__(64 * W) void tile_fwd(TileFwdArgs<T>) {
-  const TileFwdArgs<T> &a = kernel_args<TileFwdArgs<T>>();
-  extern __shared__ double tile_lds[];
-  const TileRows<T, P> lds(tile_lds, (int)blockDim.y, a.steps, (int)threadIdx.x);
+  tile_fwd_group<T, P, R, FMT>(kernel_args<TileFwdArgs<T>>(),
+                               (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x));
+}
+
+// Several problems in one launch: workgroup b of the launch belongs to problem
+// tile_item[b], whose arguments for this launch are table[tile_item[b]].
+template <typename T, int P, int R, int W, int FMT>
+__global__ __launch_bounds__(64 * W) void tile_fwd_items(const TileFwdArgs<T> *__restrict__ table,
+                                                         const int32_t *__restrict__ tile_item) {
   const int flat = (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x);
-  const int tile = flat / a.n_shots, s = flat - tile * a.n_shots;
-  const TilePlace c = tile_place<T, P, R>(a.g, a.pts.n_xt, tile, a.halo, a.own_rows);
-  if (c.edge)  // uniform over the workgroup
-    tile_forward<T, P, R, FMT, true>(c, s, lds);
-  else
-    tile_forward<T, P, R, FMT, false>(c, s, lds);
+  const ArgRef<TileFwdArgs<T>> args{(typename ArgRef<TileFwdArgs<T>>::P)(table + tile_item[flat])};
+  tile_fwd_group<T, P, R, FMT>(args, flat - args().tile0);
 }
 
 // ------------------------------------------------------------ Born forward
@@ -721,11 +746,12 @@ template <typename T> struct TileBornArgs {
 };
 
 template <typename T, int P, int R, bool STORE, bool EDGE>
-__device__ __forceinline__ void tile_born_step(const TilePlace &c, int s, const TileRows<T, P> &lds,
+__device__ __forceinline__ void tile_born_step(ArgRef<TileBornArgs<T>> args, const TilePlace &c, int s,
+                                               const TileRows<T, P> &lds,
                                                const TileRows<T, P> &lds2) {
   using Args = TileBornArgs<T>;
   constexpr int HS = 2 * P - 1;
-  const Args &a = kernel_args<Args>();
+  const Args &a = args();
   const Geom<T> &g = a.g;
   const int steps = a.steps, halo = a.halo;
   const int64_t base = (int64_t)s * g.numel;
@@ -779,7 +805,7 @@ __device__ __forceinline__ void tile_born_step(const TilePlace &c, int s, const 
       v.curl(k, b, lds2, c);
       if constexpr (STORE) {
         if (b.own != 0) {  // uniform
-          const Args &q = kernel_args<Args>();
+          const Args &q = args();
           const int64_t at = j * q.hist_stride;
           u.template snapshot<1>(k, b, (char *)q.hist[0] + at, (char *)q.hist[1] + at, base);
           v.template snapshot<1>(k, b, (char *)q.hist[2] + at, (char *)q.hist[3] + at, base);
@@ -794,7 +820,7 @@ __device__ __forceinline__ void tile_born_step(const TilePlace &c, int s, const 
       }
       u.update_ey(k, b);
       if (points.fast >= 0) {  // uniform
-        const Args &q = kernel_args<Args>();
+        const Args &q = args();
         const int64_t fo = j * q.f_stride, ro = j * q.r_stride;
         points.forward(q.pts, c, q.n_shots, s, lds.amp_at(c, steps, j),
                        q.f0 != nullptr ? q.f0 + fo : nullptr,
@@ -805,14 +831,15 @@ __device__ __forceinline__ void tile_born_step(const TilePlace &c, int s, const 
       }
     }
   }
-  const Args &z = kernel_args<Args>();
+  const Args &z = args();
   u.store(k, z.out, base);
   v.store(k, z.out + 7, base);
 }
 
 template <typename T, int P, int R, int W, bool STORE>
 __global__ __launch_bounds__(64 * W) void tile_born(TileBornArgs<T>) {
-  const TileBornArgs<T> &a = kernel_args<TileBornArgs<T>>();
+  const ArgRef<TileBornArgs<T>> args = kernel_args<TileBornArgs<T>>();
+  const TileBornArgs<T> &a = args();
   extern __shared__ double tile_lds[];
   const int waves = (int)blockDim.y;
   const TileRows<T, P> lds(tile_lds, waves, a.steps, (int)threadIdx.x);
@@ -822,9 +849,9 @@ __global__ __launch_bounds__(64 * W) void tile_born(TileBornArgs<T>) {
   const int tile = flat / a.n_shots, s = flat - tile * a.n_shots;
   const TilePlace c = tile_place<T, P, R>(a.g, a.pts.n_xt, tile, a.halo, a.own_rows);
   if (c.edge)  // uniform over the workgroup
-    tile_born_step<T, P, R, STORE, true>(c, s, lds, lds2);
+    tile_born_step<T, P, R, STORE, true>(args, c, s, lds, lds2);
   else
-    tile_born_step<T, P, R, STORE, false>(c, s, lds, lds2);
+    tile_born_step<T, P, R, STORE, false>(args, c, s, lds, lds2);
 }
 
 // ----------------------------------------------------------------- adjoint
@@ -832,11 +859,11 @@ __global__ __launch_bounds__(64 * W) void tile_born(TileBornArgs<T>) {
 // memories; dHx/dz carries the negated term, so that its differences swap
 // their operands instead of negating (bit-identical).
 template <typename T, int P, int R, int FMT, bool EDGE>
-__device__ __forceinline__ void tile_adjoint(const TilePlace &c, int s0, int s1, int group,
+__device__ __forceinline__ void tile_adjoint(ArgRef<TileAdjArgs<T>> args, const TilePlace &c, int s0, int s1, int group,
                                              const TileRows<T, P> &lds) {
   using Args = TileAdjArgs<T>;
   constexpr int HS = 2 * P - 1;
-  const Args &a = kernel_args<Args>();
+  const Args &a = args();
   const Geom<T> &g = a.g;
   const T rdy = g.rdy, rdx = g.rdx;
   const int steps = a.steps;
@@ -872,7 +899,7 @@ __device__ __forceinline__ void tile_adjoint(const TilePlace &c, int s0, int s1,
 
   for (int s = s0; s < s1; ++s) {
     const int64_t base = (int64_t)s * numel;
-    const Args &a = kernel_args<Args>();
+    const Args &a = args();
     const Geom<T> &g = a.g;
     T ley[R], lhx[R], lhz[R], ca[R], cb[R], cq[R];
     load_rows<T, R>(ley, as_global(a.in[0]) + base, at);
@@ -904,7 +931,7 @@ __device__ __forceinline__ void tile_adjoint(const TilePlace &c, int s0, int s1,
       const bool active = c.row0 < hi + P - 1 && c.row0 + R > lo - P;  // uniform
       const RowBits b = rows.again();
       // this step's snapshots, read well before the gradient needs them
-      const Args &a = kernel_args<Args>();
+      const Args &a = args();
       const bool have = want && (a.ey_store[j] != nullptr || a.curl_store[j] != nullptr);
       T se[R], sc[R];
       if constexpr (FMT != 0) {
@@ -1022,7 +1049,7 @@ __device__ __forceinline__ void tile_adjoint(const TilePlace &c, int s0, int s1,
           if (in) ley[r] = ca[r] * ley[r] + (dz + dx[r]);
         }
         if (points.fast >= 0) {  // uniform
-          const Args &q = kernel_args<Args>();
+          const Args &q = args();
           const T *const gr = q.grad_r != nullptr ? q.grad_r - j * q.r_stride : nullptr;
           T *const gf = q.grad_f != nullptr ? q.grad_f - j * q.f_stride : nullptr;
           points.adjoint(q.pts, c, q.n_shots, s, lds.amp_at(c, steps, j), gr, gf, own, b.own, ley);
@@ -1040,7 +1067,7 @@ __device__ __forceinline__ void tile_adjoint(const TilePlace &c, int s0, int s1,
       }
     }
 
-    const Args &z = kernel_args<Args>();
+    const Args &z = args();
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (!(rows.own >> r & 1) || !own) continue;
@@ -1073,20 +1100,34 @@ __device__ __forceinline__ void tile_adjoint(const TilePlace &c, int s0, int s1,
   }
 }
 
-template <typename T, int P, int R, int W, int FMT>
-__global__ __launch_bounds__(64 * W) void tile_adj(TileAdjArgs<T>) {
-  const TileAdjArgs<T> &a = kernel_args<TileAdjArgs<T>>();
+template <typename T, int P, int R, int FMT>
+__device__ __forceinline__ void tile_adj_group(ArgRef<TileAdjArgs<T>> args, int flat) {
   extern __shared__ double tile_lds[];
+  const TileAdjArgs<T> &a = args();
   const TileRows<T, P> lds(tile_lds, (int)blockDim.y, a.steps, (int)threadIdx.x);
   const int n_groups = (a.n_shots + a.group - 1) / a.group;
-  const int flat = (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x);
   const int tile = flat / n_groups, k = flat - tile * n_groups;
   const int s0 = k * a.group, s1 = min(s0 + a.group, a.n_shots);
   const TilePlace c = tile_place<T, P, R>(a.g, a.pts.n_xt, tile, a.halo, a.own_rows);
   if (c.edge)  // uniform over the workgroup
-    tile_adjoint<T, P, R, FMT, true>(c, s0, s1, k, lds);
+    tile_adjoint<T, P, R, FMT, true>(args, c, s0, s1, k, lds);
   else
-    tile_adjoint<T, P, R, FMT, false>(c, s0, s1, k, lds);
+    tile_adjoint<T, P, R, FMT, false>(args, c, s0, s1, k, lds);
+}
+
+template <typename T, int P, int R, int W, int FMT>
+__global__ __launch_bounds__(64 * W) void tile_adj(TileAdjArgs<T>) {
+  tile_adj_group<T, P, R, FMT>(kernel_args<TileAdjArgs<T>>(),
+                               (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x));
+}
+
+// Several problems in one launch, as tile_fwd_items.
+template <typename T, int P, int R, int W, int FMT>
+__global__ __launch_bounds__(64 * W) void tile_adj_items(const TileAdjArgs<T> *__restrict__ table,
+                                                         const int32_t *__restrict__ tile_item) {
+  const int flat = (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x);
+  const ArgRef<TileAdjArgs<T>> args{(typename ArgRef<TileAdjArgs<T>>::P)(table + tile_item[flat])};
+  tile_adj_group<T, P, R, FMT>(args, flat - args().tile0);
 }
 
 }  // namespace tm2d

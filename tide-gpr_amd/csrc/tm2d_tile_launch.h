@@ -128,12 +128,31 @@ template <typename T> TilePlan plan_born(int half, int ny, int nx, int n_shots) 
   return best;
 }
 
+// Steps of each launch of a time loop of nt steps, at most `most` each: the
+// fewest launches, an even number of them where nt allows it (the state ping-
+// pongs between the caller's arrays and a scratch copy, and an even count ends
+// in the caller's arrays), as equal as possible.
+struct LaunchSteps {
+  int64_t nt, launches;
+  LaunchSteps(int64_t nt_, int most) : nt(nt_), launches((nt_ + most - 1) / most) {
+    if ((launches & 1) && nt > launches) ++launches;
+  }
+  int at(int64_t k) const { return (int)(nt * (k + 1) / launches - nt * k / launches); }
+  bool ends_in_scratch() const { return (launches & 1) != 0; }
+};
+
 template <typename T>
 void launch_tile_fwd(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileFwdArgs<T> &a);
 template <typename T>
 void launch_tile_adj(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileAdjArgs<T> &a);
 template <typename T>
 void launch_tile_born(int half, const TilePlan &p, bool store, hipStream_t stream, const TileBornArgs<T> &a);
+
+// Several order-2 fp32 problems of tile shape p: `grid` workgroups.
+void launch_tile_fwd_items(const TilePlan &p, int fmt, int64_t grid, hipStream_t stream,
+                           const TileFwdArgs<float> *table, const int32_t *tile_item);
+void launch_tile_adj_items(const TilePlan &p, int fmt, int64_t grid, hipStream_t stream,
+                           const TileAdjArgs<float> *table, const int32_t *tile_item);
 
 #ifdef TIDE_TM2D_TILE_DEFINITIONS
 
