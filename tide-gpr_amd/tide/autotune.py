@@ -34,22 +34,24 @@ from .maxwell.tm2d import prepare_tm2d
 from .utils import C0
 
 # (rows, group, shot loop, steps per launch, interior/border split,
-#  border tile rows); 0 steps per launch: the library picks workgroup or
-#  wavefront tiles and their steps from the problem (the default)
+#  border tile rows)
 FWD_CANDIDATES: tuple[tuple[int, int, int, int, int, int], ...] = (
-    (4, 1, 0, 0, 0, 0),
     (2, 4, 0, 1, 0, 0), (4, 2, 0, 1, 0, 0), (4, 4, 0, 1, 0, 0), (8, 4, 0, 1, 0, 0),
     (16, 4, 0, 1, 0, 0), (2, 4, 1, 1, 0, 0), (4, 2, 1, 1, 0, 0),
     (2, 2, 0, 2, 0, 0), (4, 1, 0, 2, 0, 0), (4, 2, 0, 2, 0, 0), (4, 4, 0, 2, 0, 0),
     (8, 2, 0, 2, 0, 0), (4, 1, 0, 2, 0, 2), (4, 2, 0, 2, 0, 2),
     (4, 1, 0, 2, 1, 0), (4, 2, 0, 2, 1, 0), (4, 2, 0, 3, 0, 0), (8, 2, 0, 3, 0, 0))
 ADJ_CANDIDATES: tuple[tuple[int, int, int, int, int, int], ...] = (
-    (4, 4, 0, 0, 0, 2),
     (2, 2, 0, 1, 0, 0), (2, 4, 0, 1, 0, 0), (2, 8, 0, 1, 0, 0), (4, 4, 0, 1, 0, 0),
     (8, 2, 0, 1, 0, 0), (2, 4, 1, 1, 0, 0), (4, 2, 1, 1, 0, 0),
     (4, 4, 0, 2, 1, 0), (4, 8, 0, 2, 1, 0), (4, 4, 0, 2, 1, 2), (4, 8, 0, 2, 1, 2),
     (2, 4, 0, 2, 0, 0), (4, 2, 0, 2, 0, 0), (4, 4, 0, 2, 0, 0), (4, 8, 0, 2, 0, 0),
     (4, 4, 0, 2, 0, 2), (4, 8, 0, 2, 0, 2), (4, 4, 0, 3, 0, 2), (4, 2, 0, 3, 0, 2))
+
+# 0 steps per launch: the library picks workgroup or wavefront tiles and
+# their steps from the problem (its default); tried beside the above
+FWD_AUTOMATIC = (4, 1, 0, 0, 0, 0)
+ADJ_AUTOMATIC = (4, 4, 0, 0, 0, 2)
 
 _cache: dict[tuple, tuple[tuple[int, ...], tuple[int, ...]]] = {}
 
@@ -136,8 +138,8 @@ def tune_tm2d(
     nt: int = 400,
     max_store_bytes: int = 24 << 30,
     device: torch.device | str = "cuda:0",
-    fwd_candidates: Sequence[tuple[int, ...]] = FWD_CANDIDATES,
-    adj_candidates: Sequence[tuple[int, ...]] = ADJ_CANDIDATES,
+    fwd_candidates: Sequence[tuple[int, ...]] = (FWD_AUTOMATIC, *FWD_CANDIDATES),
+    adj_candidates: Sequence[tuple[int, ...]] = (ADJ_AUTOMATIC, *ADJ_CANDIDATES),
     use_cache: bool = True,
 ) -> dict:
     """Pick and install the fastest (rows, group, shot loop, steps, split,
