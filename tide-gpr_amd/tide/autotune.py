@@ -48,8 +48,9 @@ ADJ_CANDIDATES: tuple[tuple[int, int, int, int, int, int], ...] = (
     (2, 4, 0, 2, 0, 0), (4, 2, 0, 2, 0, 0), (4, 4, 0, 2, 0, 0), (4, 8, 0, 2, 0, 0),
     (4, 4, 0, 2, 0, 2), (4, 8, 0, 2, 0, 2), (4, 4, 0, 3, 0, 2), (4, 2, 0, 3, 0, 2))
 
-# 0 steps per launch: the library picks workgroup or wavefront tiles and
-# their steps from the problem (its default); tried beside the above
+# 0 steps per launch (the library's default): it picks workgroup or wavefront
+# tiles and their steps from the problem.  Add these to the lists to time
+# them against the fixed shapes.
 FWD_AUTOMATIC = (4, 1, 0, 0, 0, 0)
 ADJ_AUTOMATIC = (4, 4, 0, 0, 0, 2)
 
@@ -138,8 +139,8 @@ def tune_tm2d(
     nt: int = 400,
     max_store_bytes: int = 24 << 30,
     device: torch.device | str = "cuda:0",
-    fwd_candidates: Sequence[tuple[int, ...]] = (FWD_AUTOMATIC, *FWD_CANDIDATES),
-    adj_candidates: Sequence[tuple[int, ...]] = (ADJ_AUTOMATIC, *ADJ_CANDIDATES),
+    fwd_candidates: Sequence[tuple[int, ...]] = FWD_CANDIDATES,
+    adj_candidates: Sequence[tuple[int, ...]] = ADJ_CANDIDATES,
     use_cache: bool = True,
 ) -> dict:
     """Pick and install the fastest (rows, group, shot loop, steps, split,
@@ -265,4 +266,5 @@ def tune_tm2d(
     }
 
 
-__all__ = ["tune_tm2d", "current", "FWD_CANDIDATES", "ADJ_CANDIDATES"]
+__all__ = ["tune_tm2d", "current", "FWD_CANDIDATES", "ADJ_CANDIDATES", "FWD_AUTOMATIC",
+           "ADJ_AUTOMATIC"]
