@@ -337,3 +337,14 @@ def test_autotune_rejects_bad_chunk_lists_before_touching_a_device():
     assert _pick(times, (4, 4)) == (2, 2)
     assert _pick({(4, 4): 100.0, (4, 8): 98.0}, (4, 4)) == (4, 4)
     assert _pick({(4, 4): 100.0, (4, 8): 98.0}, (8, 8)) == (4, 8)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("widths", [(4, 6), (0, 5), (0, 0)])
+def test_pml_pair_equals_the_separate_profiles(widths, dtype):
+    args = (list(widths), [float(widths[0]), 30.0 - widths[1]], 0.1, 2e-11, 31, 3e8, dtype,
+            torch.device("cpu"), 1e10)
+    whole, half = utils.setup_pml_pair(*args, grid_spacing=0.02)
+    for got, want in ((whole, utils.setup_pml(*args, grid_spacing=0.02)),
+                      (half, utils.setup_pml_half(*args, grid_spacing=0.02))):
+        assert all(torch.equal(a, b) for a, b in zip(got, want))

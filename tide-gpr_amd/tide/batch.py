@@ -23,8 +23,11 @@ from typing import Any
 import torch
 
 from . import _native
+from .grid_utils import _normalize_grid_spacing_2d
 from .maxwell.tm2d import prepare_tm2d
+from .padding import create_or_pad
 from .storage import STORAGE_FORMAT_BF16, STORAGE_FORMAT_FULL
+from .utils import prepare_parameters
 
 _P = ctypes.c_void_p
 
@@ -205,6 +208,10 @@ class TM2DBatch:
         """Forward from zero state, L2 misfit ``0.5 |d - d_obs|^2`` (FP64) and
         its epsilon / sigma gradients per problem.  Returns
         ``(misfits, eps_grads, sigma_grads)``."""
+        # the models may have been changed in place since the plan was built
+        # (one wait here, before the loops, instead of one per problem behind them)
+        if bool(torch.stack([torch.any(kw["epsilon"] <= 0) for kw in self.problems]).any()):
+            raise ValueError("epsilon must be strictly positive.")
         self.reset_state()
         rs = self.forward()
         resid = [(r.double() - o.double()) for r, o in zip(rs, observed)]
@@ -214,19 +221,31 @@ class TM2DBatch:
         for kw, st, (gca, gcb, gf) in zip(self.problems, self.setups, grads):
             e = kw["epsilon"].detach().clone().requires_grad_(True)
             s = kw["sigma"].detach().clone().requires_grad_(True)
-            st2 = prepare_tm2d(e, s, kw["mu"].detach(), kw["grid_spacing"], kw["dt"],
-                               kw.get("source_amplitude"), kw.get("source_location"),
-                               kw.get("receiver_location"), pml_width=kw.get("pml_width", 20),
-                               nt=kw.get("nt"))
-            outs = [st2.ca, st2.cb]
-            cots = [gca.to(torch.float32).reshape(st2.ca.shape), gcb.to(torch.float32).reshape(st2.cb.shape)]
+            ca, cb, f = self._coefficients(kw, st, e, s)
+            outs = [ca, cb]
+            cots = [gca.to(torch.float32).reshape(ca.shape), gcb.to(torch.float32).reshape(cb.shape)]
             if st.n_src > 0:
-                outs.append(st2.f)
+                outs.append(f)
                 cots.append(gf)
             torch.autograd.backward(outs, cots)
             eps_g.append(e.grad)
             sig_g.append(s.grad)
         return misfit, eps_g, sig_g
+
+    def _coefficients(self, kw, st, epsilon, sigma):
+        """``ca``, ``cb`` and the source term of a problem as functions of its
+        model: the operations of ``prepare_tm2d`` that depend on it."""
+        total = [a + b for a, b in zip(st.fd_pad, st.pml_width)]
+        eps_p, sig_p = (create_or_pad(t, total, t.device, t.dtype, (st.ny, st.nx), mode="replicate")
+                        for t in (epsilon, sigma))
+        ca, cb, _ = prepare_parameters(eps_p, sig_p, torch.ones_like(eps_p[:1, :1]), kw["dt"])
+        f = None
+        if st.n_src > 0:
+            cb_src = cb.reshape(1, -1).expand(st.n_shots, -1).gather(1, st.extra["src"])
+            amp = kw["source_amplitude"].permute(2, 0, 1).contiguous().to(cb.dtype)
+            dy, dx = _normalize_grid_spacing_2d(kw["grid_spacing"])
+            f = amp * cb_src.unsqueeze(0) * (-1.0 / (dx * dy))
+        return ca, cb, f
 
     def update_models(self, epsilon: Sequence[torch.Tensor], sigma: Sequence[torch.Tensor]) -> None:
         """Replace every problem's model in place (the plan's graphs stay valid)."""

@@ -246,8 +246,9 @@ def prepare_tm2d(
             fields.append(
                 create_or_pad(t0.detach(), fd_pad, device, dtype, (n_shots, ny, nx)).contiguous()
             )
-    for wf, dim in zip(fields[3:], (1, 0, 0, 1)):
-        zero_interior(wf, fd_pad, widths, dim)
+    for wf, t0, dim in zip(fields[3:], initial[3:], (1, 0, 0, 1)):
+        if t0 is not None:
+            zero_interior(wf, fd_pad, widths, dim)
 
     if max_vel is None:  # a caller's max_vel also sets the profiles (reference tm2d_cuda.py:124-130)
         max_vel = float((1.0 / torch.sqrt(epsilon.detach() * mu.detach())).max().item()) * C0

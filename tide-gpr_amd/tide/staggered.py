@@ -43,27 +43,14 @@ def set_pml_profiles(
         pml_width[3] * grid_spacing[1],
     )
 
-    def axis(widths, edges, n, spacing, half):
-        setup = utils.setup_pml_half if half else utils.setup_pml
-        return setup(
-            widths,
-            edges,
-            max_pml,
-            dt,
-            n,
-            max_vel,
-            dtype,
-            device,
-            pml_freq,
-            start=0.0,
-            grid_spacing=spacing,
-            eps_scale=eps_scale,
+    def axis(widths, edges, n, spacing):
+        return utils.setup_pml_pair(
+            widths, edges, max_pml, dt, n, max_vel, dtype, device, pml_freq,
+            grid_spacing=spacing, eps_scale=eps_scale,
         )
 
-    ay, by, ky = axis(pml_width[:2], edges_y, ny, grid_spacing[0], False)
-    ax, bx, kx = axis(pml_width[2:], edges_x, nx, grid_spacing[1], False)
-    ayh, byh, kyh = axis(pml_width[:2], edges_y, ny, grid_spacing[0], True)
-    axh, bxh, kxh = axis(pml_width[2:], edges_x, nx, grid_spacing[1], True)
+    (ay, by, ky), (ayh, byh, kyh) = axis(pml_width[:2], edges_y, ny, grid_spacing[0])
+    (ax, bx, kx), (axh, bxh, kxh) = axis(pml_width[2:], edges_x, nx, grid_spacing[1])
 
     def col(v):  # varies along y
         return v[None, :, None]
@@ -109,25 +96,13 @@ def set_pml_profiles_3d(
         n = sizes[name]
         widths = pml_width[2 * d : 2 * d + 2]
         edges = _pml_edges(n, widths[0], widths[1], fd_pad[2 * d], fd_pad[2 * d + 1])
-        for half, setup in ((False, utils.setup_pml), (True, utils.setup_pml_half)):
-            a, b, k = setup(
-                widths,
-                edges,
-                max_pml,
-                dt,
-                n,
-                0.0,
-                dtype,
-                device,
-                0.5 / dt,
-                start=0.0,
-                grid_spacing=grid_spacing[d],
-                eps_scale=eps_scale,
-            )
-            suffix = "h" if half else ""
-            out[f"a{name}{suffix}"] = a
-            out[f"b{name}{suffix}"] = b
-            out[f"k{name}{suffix}"] = k
+        pair = utils.setup_pml_pair(
+            widths, edges, max_pml, dt, n, 0.0, dtype, device, 0.5 / dt,
+            grid_spacing=grid_spacing[d], eps_scale=eps_scale,
+        )
+        for suffix, values in zip(("", "h"), pair):
+            for key, v in zip("abk", values):
+                out[f"{key}{name}{suffix}"] = v
     return out
 
 

@@ -165,12 +165,14 @@ def setup_pml(
     eps: float = 1e-9,
     grid_spacing: float = 1.0,
     eps_scale: float = EP0,
+    coord: torch.Tensor | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """CPML (a, b, kappa) along one axis of length ``n``.
 
     ``pml_width`` = [low, high] cells, ``pml_start`` = inner edge coordinate
     of each strip (in cells), ``start`` = coordinate of element 0 (0 for
-    integer points, 0.5 for half points).  ``max_vel``, ``pml_freq`` and
+    integer points, 0.5 for half points); ``coord`` gives all ``n``
+    coordinates instead.  ``max_vel``, ``pml_freq`` and
     ``r_val`` are accepted for signature compatibility; the electromagnetic
     grading does not use them.
     """
@@ -182,7 +184,8 @@ def setup_pml(
         return a, b, k
 
     sigma0 = (n_power + 1) / (150.0 * math.pi * grid_spacing)
-    coord = torch.arange(start, start + n, device=device, dtype=dtype)
+    if coord is None:
+        coord = torch.arange(start, start + n, device=device, dtype=dtype)
 
     for side in (0, 1):
         width = pml_width[side]
@@ -202,6 +205,26 @@ def setup_pml(
         a_side = torch.where(sig > 1e-6, a_side, torch.zeros_like(a_side))
         a = torch.where(inside, a_side, a)
     return a, b, k
+
+
+def setup_pml_pair(
+    pml_width: Sequence[int],
+    pml_start: Sequence[float],
+    max_pml: float,
+    dt: float,
+    n: int,
+    max_vel: float,
+    dtype: torch.dtype,
+    device: torch.device,
+    pml_freq: float,
+    **kwargs,
+) -> tuple[tuple[torch.Tensor, ...], tuple[torch.Tensor, ...]]:
+    """``setup_pml`` and ``setup_pml_half`` of one axis, computed together
+    (some thirty small device operations instead of sixty)."""
+    coord = torch.cat([torch.arange(s, s + n, device=device, dtype=dtype) for s in (0.0, 0.5)])
+    both = setup_pml(pml_width, pml_start, max_pml, dt, 2 * n, max_vel, dtype, device, pml_freq,
+                     coord=coord, **kwargs)
+    return tuple(t[:n] for t in both), tuple(t[n:] for t in both)
 
 
 def setup_pml_half(
@@ -250,5 +273,6 @@ __all__ = [
     "prepare_parameters",
     "setup_pml",
     "setup_pml_half",
+    "setup_pml_pair",
     "validate_material_inputs",
 ]
