@@ -298,10 +298,14 @@ int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_e
   const LaunchSteps loop(nt, plan.steps);
   Scratch scr(stream, arena, arena_cap);
   StatePair<T, 7> state({ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x}, (size_t)total);
-  TIDE_CHECK(state.open(scr, loop, stream));
   DevicePointTable dpt;
-  TIDE_CHECK(upload_points_lanes(p, plan, src, rec, dpt, stream, &scr));
-  TIDE_CHECK(pack_profiles(p, scr, stream));
+  int rc = state.open(scr, loop, stream);
+  if (rc == kOk) rc = upload_points_lanes(p, plan, src, rec, dpt, stream, &scr);
+  if (rc == kOk) rc = pack_profiles(p, scr, stream);
+  if (rc != kOk) {
+    dpt.release(stream);
+    return scr.full ? (int)kOutOfMemory : rc;
+  }
   TileFwdArgs<T> a;
   std::memset(&a, 0, sizeof(a));
   a.g = p.g;
@@ -312,6 +316,7 @@ int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_e
   a.n_shots = p.n_shots;
   a.halo = plan.halo;
   a.own_rows = plan.own_rows;
+  a.order = tile_order(plan, p.g, half);
   a.f_stride = n_shots * p.n_src;
   a.r_stride = n_shots * p.n_rec;
   LoopTimer timer(0, stream);
@@ -378,6 +383,7 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
   a.n_shots = p.n_shots;
   a.halo = plan.halo;
   a.own_rows = plan.own_rows;
+  a.order = tile_order(plan, p.g, half);
   a.group = plan.group;
   a.r_stride = n_shots * p.n_rec;
   a.f_stride = n_shots * p.n_src;
@@ -441,6 +447,7 @@ int born_tiles(int half, Problem<T> p, T *const bg[7], T *const sc[7], const T *
   a.n_shots = p.n_shots;
   a.halo = plan.halo;
   a.own_rows = plan.own_rows;
+  a.order = tile_order(plan, p.g, half);
   a.f_stride = n_shots * p.n_src;
   a.r_stride = n_shots * p.n_rec;
   a.hist_stride = total * (int64_t)sizeof(T);
@@ -484,11 +491,19 @@ int forward_impl(Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_h
   const bool staged = (ey_stage && ey_stage->active()) || (curl_stage && curl_stage->active());
   // K-step launches (K = 3, 4) need K ring slots at once, more than a
   // host-staged ring holds: staged calls use two-step launches.
-  if (g_tuning.fwd_steps == 0 && !staged &&
-      prefer_tiles<T>(p.g.ny, p.g.nx, p.n_shots, false, ey_store || curl_store))
-    return forward_tiles(1, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r, src, rec, nt,
-                         start_t, step_ratio, ey_store, curl_store, fmt, store_step_bytes, stream,
-                         arena, arena_cap);
+  // Without a setting the loop runs on workgroup tiles, whatever the size.
+  // fp32, us per step, tiles / two-step wavefront tiles, forward and with
+  // snapshots: 300 x 517 cells and 8 shots 6.1 / 8.2 and 7.7 / 9.3; 1024 x 1024
+  // and 4 11.7 / 16.3 and 20.9 / 22.0; 1500 x 1500 and 4 22.7 / 43 and 47 / 60;
+  // 400 x 901 and 12 13.7 / 18.0 and 26.4 / 23.7 (with its adjoint 62 / 66).
+  // Calls whose tables or state copy do not fit their memory go on below.
+  if (g_tuning.fwd_steps == 0 && !staged) {
+    const int rc = forward_tiles(1, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r, src, rec,
+                                 nt, start_t, step_ratio, ey_store, curl_store, fmt,
+                                 store_step_bytes, stream, arena, arena_cap);
+    if (rc != kOutOfMemory) return rc;
+    (void)hipGetLastError();
+  }
   const int per_launch = g_tuning.fwd_steps == 0 ? 2 : g_tuning.fwd_steps;
   const int kblk = (per_launch >= 3 && nt >= per_launch && !staged) ? per_launch : 0;
   const bool fused = per_launch >= 2 && nt >= 2;
@@ -724,10 +739,16 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
   const int64_t n_shots = p.n_shots, total = n_shots * p.g.numel;
   const bool staged = (ey_stage && ey_stage->active()) || (curl_stage && curl_stage->active());
   // K-step launches need K ring slots at once (see forward_impl)
-  if (g_tuning.adj_steps == 0 && !staged && prefer_tiles<T>(p.g.ny, p.g.nx, p.n_shots, true, true))
-    return backward_tiles(1, p, grad_r, l_ey, l_hx, l_hz, ml_ey_x, ml_ey_z, ml_hx_z, ml_hz_x,
-                          ey_store, curl_store, fmt, store_step_bytes, grad_f, gca, gcb, src, rec,
-                          nt, start_t, step_ratio, stream);
+  // As the forward: 300 x 517 cells and 8 shots 12.8 / 14.8 us per step, tiles
+  // / three-step wavefront tiles; 1024 x 1024 and 4 30.7 / 32.5; 400 x 901 and
+  // 12 35.5 / 42; 1500 x 1500 and 4 62.7 / 62.
+  if (g_tuning.adj_steps == 0 && !staged) {
+    const int rc = backward_tiles(1, p, grad_r, l_ey, l_hx, l_hz, ml_ey_x, ml_ey_z, ml_hx_z,
+                                  ml_hz_x, ey_store, curl_store, fmt, store_step_bytes, grad_f, gca,
+                                  gcb, src, rec, nt, start_t, step_ratio, stream);
+    if (rc != kOutOfMemory) return rc;
+    (void)hipGetLastError();
+  }
   const int per_launch = g_tuning.adj_steps == 0 ? 3 : g_tuning.adj_steps;
   const int kblk = (per_launch >= 3 && nt >= per_launch && !staged) ? per_launch : 0;
   const bool fused = per_launch >= 2 && nt >= 2;

@@ -671,6 +671,7 @@ int build_tiles_forward(Plan &p) {
     a.n_shots = (int32_t)q.n_shots;
     a.halo = one.halo;
     a.own_rows = one.own_rows;
+    a.order = tile_order(one, it.g, 1);
     a.f_stride = q.n_shots * q.n_src;
     a.r_stride = q.n_shots * q.n_rec;
     float *const state[2][7] = {
@@ -726,6 +727,7 @@ int build_tiles_backward(Plan &p) {
     a.n_shots = (int32_t)q.n_shots;
     a.halo = one.halo;
     a.own_rows = one.own_rows;
+    a.order = tile_order(one, it.g, 1);
     a.group = 1;
     a.r_stride = q.n_shots * q.n_rec;
     a.f_stride = q.n_shots * q.n_src;
@@ -859,9 +861,9 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
   // neither pass has a setting the forward runs on tiles, the adjoint up to
   // kBatchTileCells padded cells.  fp32, us per step, tiles / two-step launches,
   // forward with snapshots and adjoint: 24 grids of 81 x 101 cells (x 1 shot)
-  // 3.4 / 9.8 and 6.3 / 21; 12 of 241 x 261 x 3 12 / 19 and 21 / 34; 12 of 341 x
-  // 361 x 4 27 / 40 and 49 / 51; 8 of 541 x 561 x 4 54 / 70 and 87 / 82; 8 of
-  // 741 x 781 x 4 107 / 139 and 144 / 139.
+  // 3.5 / 9.8 and 6.5 / 21; 12 of 241 x 261 x 3 11 / 19 and 21 / 34; 12 of 341 x
+  // 361 x 4 26 / 38 and 50 / 50; 8 of 541 x 561 x 4 49 / 64 and 81 / 78; 8 of
+  // 741 x 781 x 4 99 / 104 to 137 and 139 / 129.
   constexpr int64_t kBatchTileCells = 7000000;
   int64_t cells = 0;
   for (int64_t m = 0; m < n; ++m)

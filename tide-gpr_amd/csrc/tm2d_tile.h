@@ -33,6 +33,53 @@ namespace tm2d {
 constexpr int kTileSteps = 8;   // most steps per launch
 constexpr int kTileWaves = 16;  // most wavefronts per workgroup
 
+// Order of a problem's tiles in a launch: the tiles that meet a grid edge or a
+// CPML strip first, then the rectangle [xa, xb) x [ya, yb) of the others.  Edge
+// tiles take longer, so they neither leave a tail nor, dealt by dealt_index,
+// load one XCD more than another.  Rows of tiles in one contiguous run per XCD
+// gave the first and the last XCD the top and bottom rows; fp32, us per step,
+// before and after: 400 x 901 cells and 12 shots forward 18.3 -> 14.0, adjoint
+// 49 -> 42; 1024 x 1024 and 4 shots 15.0 -> 11.9 and 32.7 -> 29.7.
+struct TileOrder {
+  int32_t n_yt, xa, xb, ya, yb;
+  __host__ __device__ __forceinline__ int edges(int n_xt) const {
+    return n_xt * n_yt - (xb - xa) * (yb - ya);
+  }
+  // Column and row of the o-th tile.
+  __device__ __forceinline__ void at(int o, int n_xt, int &xt, int &yt) const {
+    const int wide = xb - xa, top = ya * n_xt, side = (yb - ya) * (n_xt - wide);
+    int first = 0, width = n_xt, skip_from = n_xt, skip = 0;  // columns from skip_from on move by skip
+    if (o >= edges(n_xt)) {
+      o -= edges(n_xt);
+      first = ya;
+      width = wide;
+      skip_from = 0;
+      skip = xa;
+    } else if (o >= top + side) {
+      o -= top + side;
+      first = yb;
+    } else if (o >= top) {
+      o -= top;
+      first = ya;
+      width = n_xt - wide;
+      skip_from = xa;
+      skip = wide;
+    }
+    yt = o / width;
+    xt = o - yt * width;
+    yt += first;
+    if (xt >= skip_from) xt += skip;
+  }
+};
+
+// Index of workgroup b among n: runs of 16 tiles go to the XCDs in turn.  Each
+// XCD gets its share of the edge tiles, and neighbours mostly share an L2.
+__device__ __forceinline__ int dealt_index(int b, int n) {
+  constexpr int kRun = 16, kAll = 8 * kRun;
+  const int first = b & ~(kAll - 1);
+  return first + kAll > n ? b : first + (b & 7) * kRun + ((b >> 3) & (kRun - 1));
+}
+
 template <typename T> struct TileFwdArgs {
   Geom<T> g;
   Points pts;  // built with build_point_table_lanes(64 - 2 halo, halo)
@@ -44,6 +91,7 @@ template <typename T> struct TileFwdArgs {
   int64_t f_stride, r_stride;  // step's are one stride further
   void *ey_store[kTileSteps], *curl_store[kTileSteps];  // null: no snapshot
   int32_t n_shots, steps, halo, own_rows;
+  TileOrder order;
   int32_t tile0;  // first workgroup of the problem in a launch of several
 };
 
@@ -61,6 +109,7 @@ template <typename T> struct TileAdjArgs {
   int32_t per_shot_grad;
   double step_scale;
   int32_t n_shots, steps, halo, own_rows, group, tile0;
+  TileOrder order;
   int64_t group_stride;  // shot group k adds into gca / gcb + k * group_stride
 };
 
@@ -98,15 +147,15 @@ struct TilePlace {
 };
 
 template <typename T, int P, int R>
-__device__ __forceinline__ TilePlace tile_place(const Geom<T> &g, int n_xt, int tile, int halo,
-                                                int own_rows) {
+__device__ __forceinline__ TilePlace tile_place(const Geom<T> &g, const TileOrder &order, int n_xt,
+                                                int tile, int halo, int own_rows) {
   TilePlace c;
   c.lane = threadIdx.x;
   c.w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
   c.waves = (int)blockDim.y;
   c.rows = c.waves * R;
-  const int yt = tile / n_xt;
-  c.xt = tile - yt * n_xt;
+  int yt;
+  order.at(tile, n_xt, c.xt, yt);
   const int x0 = c.xt * (64 - 2 * halo) - halo, y0 = yt * own_rows - halo;
   c.x = x0 + c.lane;
   c.row0 = c.w * R;
@@ -704,7 +753,7 @@ __device__ __forceinline__ void tile_fwd_group(ArgRef<TileFwdArgs<T>> args, int 
   const TileFwdArgs<T> &a = args();
   const TileRows<T, P> lds(tile_lds, (int)blockDim.y, a.steps, (int)threadIdx.x);
   const int tile = flat / a.n_shots, s = flat - tile * a.n_shots;
-  const TilePlace c = tile_place<T, P, R>(a.g, a.pts.n_xt, tile, a.halo, a.own_rows);
+  const TilePlace c = tile_place<T, P, R>(a.g, a.order, a.pts.n_xt, tile, a.halo, a.own_rows);
   if (c.edge)  // uniform over the workgroup
     tile_forward<T, P, R, FMT, true>(args, c, s, lds);
   else
@@ -714,7 +763,7 @@ __device__ __forceinline__ void tile_fwd_group(ArgRef<TileFwdArgs<T>> args, int 
 template <typename T, int P, int R, int W, int FMT>
 __global__ __launch_bounds__(64 * W) void tile_fwd(TileFwdArgs<T>) {
   tile_fwd_group<T, P, R, FMT>(kernel_args<TileFwdArgs<T>>(),
-                               (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x));
+                               dealt_index((int)blockIdx.x, (int)gridDim.x));
 }
 
 // Several problems in one launch: workgroup b of the launch belongs to problem
@@ -722,7 +771,7 @@ __global__ __launch_bounds__(64 * W) void tile_fwd(TileFwdArgs<T>) {
 template <typename T, int P, int R, int W, int FMT>
 __global__ __launch_bounds__(64 * W) void tile_fwd_items(const TileFwdArgs<T> *__restrict__ table,
                                                          const int32_t *__restrict__ tile_item) {
-  const int flat = (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x);
+  const int flat = dealt_index((int)blockIdx.x, (int)gridDim.x);
   const ArgRef<TileFwdArgs<T>> args{(typename ArgRef<TileFwdArgs<T>>::P)(table + tile_item[flat])};
   tile_fwd_group<T, P, R, FMT>(args, flat - args().tile0);
 }
@@ -743,6 +792,7 @@ template <typename T> struct TileBornArgs {
   void *hist[4];  // Ey^n, curl^n of the background, of the scattered field; first
   int64_t hist_stride;  // step's planes, the next step's hist_stride bytes on
   int32_t n_shots, steps, halo, own_rows;
+  TileOrder order;
 };
 
 template <typename T, int P, int R, bool STORE, bool EDGE>
@@ -845,9 +895,9 @@ __global__ __launch_bounds__(64 * W) void tile_born(TileBornArgs<T>) {
   const TileRows<T, P> lds(tile_lds, waves, a.steps, (int)threadIdx.x);
   const TileRows<T, P> lds2((char *)tile_lds + TileRows<T, P>::bytes(waves, a.steps), waves, a.steps,
                             (int)threadIdx.x);
-  const int flat = (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x);
+  const int flat = dealt_index((int)blockIdx.x, (int)gridDim.x);
   const int tile = flat / a.n_shots, s = flat - tile * a.n_shots;
-  const TilePlace c = tile_place<T, P, R>(a.g, a.pts.n_xt, tile, a.halo, a.own_rows);
+  const TilePlace c = tile_place<T, P, R>(a.g, a.order, a.pts.n_xt, tile, a.halo, a.own_rows);
   if (c.edge)  // uniform over the workgroup
     tile_born_step<T, P, R, STORE, true>(args, c, s, lds, lds2);
   else
@@ -1108,7 +1158,7 @@ __device__ __forceinline__ void tile_adj_group(ArgRef<TileAdjArgs<T>> args, int 
   const int n_groups = (a.n_shots + a.group - 1) / a.group;
   const int tile = flat / n_groups, k = flat - tile * n_groups;
   const int s0 = k * a.group, s1 = min(s0 + a.group, a.n_shots);
-  const TilePlace c = tile_place<T, P, R>(a.g, a.pts.n_xt, tile, a.halo, a.own_rows);
+  const TilePlace c = tile_place<T, P, R>(a.g, a.order, a.pts.n_xt, tile, a.halo, a.own_rows);
   if (c.edge)  // uniform over the workgroup
     tile_adjoint<T, P, R, FMT, true>(args, c, s0, s1, k, lds);
   else
@@ -1118,14 +1168,14 @@ __device__ __forceinline__ void tile_adj_group(ArgRef<TileAdjArgs<T>> args, int 
 template <typename T, int P, int R, int W, int FMT>
 __global__ __launch_bounds__(64 * W) void tile_adj(TileAdjArgs<T>) {
   tile_adj_group<T, P, R, FMT>(kernel_args<TileAdjArgs<T>>(),
-                               (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x));
+                               dealt_index((int)blockIdx.x, (int)gridDim.x));
 }
 
 // Several problems in one launch, as tile_fwd_items.
 template <typename T, int P, int R, int W, int FMT>
 __global__ __launch_bounds__(64 * W) void tile_adj_items(const TileAdjArgs<T> *__restrict__ table,
                                                          const int32_t *__restrict__ tile_item) {
-  const int flat = (int)xcd_remap((int64_t)blockIdx.x, (int64_t)gridDim.x);
+  const int flat = dealt_index((int)blockIdx.x, (int)gridDim.x);
   const ArgRef<TileAdjArgs<T>> args{(typename ArgRef<TileAdjArgs<T>>::P)(table + tile_item[flat])};
   tile_adj_group<T, P, R, FMT>(args, flat - args().tile0);
 }

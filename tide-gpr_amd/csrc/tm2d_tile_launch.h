@@ -30,6 +30,26 @@ inline TilePlan make_tile_plan(int half, int ny, int nx, int waves, int rows, in
   return p;
 }
 
+// The tiles of a plan that meet no grid edge and no CPML strip (see
+// tile_place); half is the stencil half-width.
+template <typename T> TileOrder tile_order(const TilePlan &p, const Geom<T> &g, int half) {
+  auto inner = [&](int n_tiles, int own, int len, int n, int pml0, int pml1h, int &a, int &b) {
+    a = b = 0;
+    for (int t = 0; t < n_tiles; ++t) {
+      const int c0 = t * own - p.halo, c1 = c0 + len - 1;
+      if (c0 < half || c1 > n - half - 1 || c0 < pml0 || c1 >= pml1h) continue;
+      if (a == b) a = t;
+      b = t + 1;
+    }
+  };
+  TileOrder o;
+  o.n_yt = p.n_yt;
+  inner(p.n_xt, p.own_cols, 64, g.nx, g.pml_x0, g.pml_x1h, o.xa, o.xb);
+  inner(p.n_yt, p.own_rows, p.waves * p.rows, g.ny, g.pml_y0, g.pml_y1h, o.ya, o.yb);
+  if (o.xa == o.xb || o.ya == o.yb) o.xa = o.xb = o.ya = o.yb = 0;
+  return o;
+}
+
 // Duration of one launch of `steps` steps when every workgroup runs at once
 // (one per CU), in microseconds: start, loads and stores plus the steps.
 // Measured on 60^2 to 150 x 200 grids; half is the stencil half-width.
@@ -82,22 +102,6 @@ TilePlan plan_tiles(int half, int ny, int nx, int n_shots, bool adjoint, bool st
   }
   if (us_per_step) *us_per_step = best_us;
   return best;
-}
-
-// Whether the order-2 time loop of a problem runs faster on workgroup tiles
-// than on wavefront tiles (tm2d_fused.h, tm2d_blockk.h): fp64 always (fp32
-// wavefront tiles hold 4 rows, fp64 ones 2), fp32 until the wavefront tiles
-// fill the chip.  Their time per step, measured on 1.5 to 5 million cells:
-// forward 6 us + 2.1 us per million cells (2.8 with snapshots), adjoint 11.5 us
-// + 3.7 us.
-template <typename T>
-bool prefer_tiles(int ny, int nx, int n_shots, bool adjoint, bool storing) {
-  if (sizeof(T) == 8) return true;
-  double us;
-  plan_tiles<T>(1, ny, nx, n_shots, adjoint, storing, &us);
-  const double cells = (double)ny * nx * n_shots * 1e-6;
-  const double wave = adjoint ? 11.5 + 3.7 * cells : 6.0 + (storing ? 2.8 : 2.1) * cells;
-  return us < wave;
 }
 
 // The Born kernel's tiles: 32 rows (two field sets fill the registers that one
