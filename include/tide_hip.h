@@ -1250,6 +1250,19 @@ int tide_tm2d_set_time_block(int fwd_steps, int adj_steps);
 int tide_tm2d_get_time_block(int *out2);
 
 /*
+ * Scratch of the workgroup-tile loops, as settings of the calling thread.
+ * They need a second copy of the state (and the adjoint one FP64 gradient
+ * slice per shot).  Where that does not fit in device memory, a call goes on
+ * with kernels that need less (fallback 1, the default), or returns status 4
+ * (out of memory) with nothing changed (fallback 0), so that a caller whose own
+ * allocator holds memory unused can release it and call again.  The limit is
+ * the most bytes a tile loop takes (negative, the default: what the device
+ * has); a loop that needs more has no room.  No reference counterpart.
+ */
+int tide_tm2d_set_tile_fallback(int on);
+int tide_tm2d_set_tile_scratch_limit(int64_t bytes);
+
+/*
  * Two-step launches per pass: 1 runs the interior tiles (no CPML strip, no
  * grid edge within the halo) and the border tiles as two kernels, each with
  * its own register budget; 0 runs one kernel over all tiles.  Results are

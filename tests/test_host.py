@@ -348,3 +348,30 @@ def test_pml_pair_equals_the_separate_profiles(widths, dtype):
     for got, want in ((whole, utils.setup_pml(*args, grid_spacing=0.02)),
                       (half, utils.setup_pml_half(*args, grid_spacing=0.02))):
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("fits_after", [1, 2, 3])
+def test_out_of_memory_frees_cached_blocks_before_it_falls_back(monkeypatch, fits_after):
+    """A native call without room is repeated once torch's unused blocks are
+    released; only the attempt after that may take the kernels that need less."""
+    from tide import _native
+
+    attempts, events = [], []
+    fallback = [True]
+    lib = type("Lib", (), {"tide_tm2d_set_tile_fallback":
+                           staticmethod(lambda on: fallback.__setitem__(0, bool(on)))})
+    monkeypatch.setattr(_native, "load", lambda: lib)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda: 2)
+    monkeypatch.setattr(torch.cuda, "memory_allocated", lambda: 1)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
+    monkeypatch.setattr(torch.cuda, "empty_cache", lambda: events.append(len(attempts)))
+
+    def entry(value):
+        attempts.append(fallback[0])
+        return 0 if len(attempts) >= fits_after or fallback[0] else _native.OUT_OF_MEMORY
+
+    _native.call(entry, 7)
+    assert attempts == [False, False, True][:fits_after]
+    assert events == ([] if fits_after == 1 else [1])
+    assert fallback[0]

@@ -214,3 +214,56 @@ def test_batched_plans_on_tiles(compression, interval, graph):
             for a, b in ((ga, ga_o), (gb, gb_o)):
                 assert relative_l2(a.reshape(b.shape), b) < 1e-12 if b.any() else not a.any()
     batch.close()
+
+
+@pytest.fixture
+def no_room():
+    """Every tile loop of the test's thread finds its scratch too large."""
+    lib = tide._native.load()
+    lib.tide_tm2d_set_tile_scratch_limit(0)
+    yield lib
+    lib.tide_tm2d_set_tile_scratch_limit(-1)
+
+
+@gpu
+@pytest.mark.parametrize("stencil", [2, 4, 6, 8])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_calls_without_room_for_tiles_fall_back(no_room, stencil, dtype):
+    print(f"order {stencil} {dtype}", flush=True)
+    _check(_case(49, 65, 13, stencil=stencil, dtype=dtype, shots=5))
+    case = _case(33, 49, 9, stencil=stencil, dtype=dtype)
+    rng = np.random.default_rng(1)
+    dca = (1e-3 * rng.standard_normal((33, 49))).astype(case.dtype)
+    dcb = (1e-3 * np.abs(case.cb).mean() * rng.standard_normal((33, 49))).astype(case.dtype)
+    df = np.zeros_like(case.f)
+    small = _born(case, dca, dcb, df)
+    no_room.tide_tm2d_set_tile_scratch_limit(-1)
+    tiles = _born(case, dca, dcb, df)
+    assert np.array_equal(small[1], tiles[1])
+    assert all(np.array_equal(a, b) for a, b in zip(small[2], tiles[2]))
+    # the two sum the scattering term of a step in another order: rounding of 9
+    # steps of about 20 operations
+    assert relative_l2(small[0], tiles[0]) < 9 * 20 * np.finfo(case.dtype).eps
+
+
+@gpu
+@pytest.mark.parametrize("stencil", [2, 4])
+def test_a_caller_that_can_make_room_is_told(no_room, stencil):
+    """Without the fallback a call returns status 4, and the next is none the worse."""
+    case = _case(40, 50, 9, stencil=stencil)
+    no_room.tide_tm2d_set_tile_fallback(0)
+    try:
+        with pytest.raises(tide._native.TideNativeError, match="status 4"):
+            gpu_forward(case)
+        with pytest.raises(tide._native.TideNativeError, match="status 4"):
+            gpu_forward(case, store="full")
+        stores = np.zeros((case.nt, case.n_shots, case.ny, case.nx), case.dtype)
+        w = np.ones((case.nt, case.n_shots, case.rec.shape[1]), case.dtype)
+        with pytest.raises(tide._native.TideNativeError, match="status 4"):
+            gpu_backward(case, w, stores, stores)
+        with pytest.raises(tide._native.TideNativeError, match="status 4"):
+            _born(case, None, None, np.zeros_like(case.f))
+    finally:
+        no_room.tide_tm2d_set_tile_fallback(1)
+    no_room.tide_tm2d_set_tile_scratch_limit(-1)
+    _check(case)  # an earlier call's failure is not a later one's

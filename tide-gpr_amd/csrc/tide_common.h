@@ -25,10 +25,13 @@ enum Status : int {
 void set_error(const std::string &msg);
 const char *last_error();
 
+// The error is reported through the status, so it does not stay the thread's
+// last error, where the check behind a later call's launches would find it.
 #define TIDE_HIP_TRY(expr)                                                   \
   do {                                                                       \
     hipError_t _e = (expr);                                                  \
     if (_e != hipSuccess) {                                                  \
+      (void)hipGetLastError();                                               \
       ::tide_hip::set_error(std::string(#expr) + ": " + hipGetErrorString(_e)); \
       return _e == hipErrorOutOfMemory ? ::tide_hip::kOutOfMemory            \
                                        : ::tide_hip::kHipError;              \

@@ -131,7 +131,8 @@ struct Scratch {
   hipStream_t stream;
   char *arena = nullptr;
   size_t cap = 0, used = 0;
-  bool full = false;  // an allocation did not fit
+  size_t limit = SIZE_MAX;  // most bytes of stream-ordered allocations
+  bool full = false;        // an allocation did not fit
   explicit Scratch(hipStream_t s, char *arena_ = nullptr, size_t cap_ = 0)
       : stream(s), arena(arena_), cap(cap_) {}
   ~Scratch() {
@@ -151,9 +152,16 @@ struct Scratch {
       used = at + bytes;
       return kOk;
     }
+    if (bytes > limit - used) {
+      full = true;
+      set_error("the call needs more scratch memory than its limit of " + std::to_string(limit) +
+                " bytes");
+      return kOutOfMemory;
+    }
     void *p = nullptr;
     TIDE_HIP_TRY(hipMallocAsync(&p, bytes, stream));
     bufs.push_back(p);
+    used += bytes;
     *out = (U *)p;
     return kOk;
   }
@@ -236,6 +244,36 @@ int upload_points(const Problem<T> &p, const int64_t *src, const int64_t *rec,
 
 // ------------------------------------------------- workgroup-tile time loops
 
+// What a tile loop returns where its scratch does not fit: nothing is launched
+// and nothing of the caller's has changed.  Any later failure has another
+// status, so that no call is run again on arrays that it has advanced.
+constexpr int kNoRoom = -1;
+inline int no_room(int rc, const Scratch &scr) {
+  return rc == kOutOfMemory || scr.full ? kNoRoom : rc;
+}
+
+inline int launched() {
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) return kOk;
+  set_error(std::string("tile loop: ") + hipGetErrorString(e));
+  return kHipError;
+}
+
+// Of the calling thread: whether a call whose tile loop has no room goes on
+// with the kernels that need less scratch (else it returns kOutOfMemory, and a
+// caller that holds device memory unused may release it and call again), and
+// the most scratch of a tile loop in bytes.
+thread_local bool tile_fallback = true;
+thread_local size_t tile_scratch_limit = SIZE_MAX;
+
+// True where the call goes on with the smaller kernels; else rc is its status.
+inline bool falls_back(int &rc, const char *arena = nullptr) {
+  if (rc != kNoRoom) return false;
+  if (tile_fallback || arena != nullptr) return true;
+  rc = kOutOfMemory;
+  return false;
+}
+
 template <typename T>
 int upload_points_lanes(const Problem<T> &p, const TilePlan &plan, const int64_t *src,
                         const int64_t *rec, DevicePointTable &dpt, hipStream_t stream,
@@ -251,8 +289,6 @@ int upload_points_lanes(const Problem<T> &p, const TilePlan &plan, const int64_t
 }
 
 // The N state arrays of a time loop and the scratch copy they ping-pong with.
-// open() comes before any other use of the device: a problem whose copy does
-// not fit in memory returns kOutOfMemory from there with nothing changed.
 // The strips' memories (all but the first three of each seven) are only
 // written inside their strips: where the scratch copy ends up as the result,
 // its other cells must hold the caller's.
@@ -297,6 +333,7 @@ int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_e
                                        ey_store || curl_store);
   const LaunchSteps loop(nt, plan.steps);
   Scratch scr(stream, arena, arena_cap);
+  scr.limit = tile_scratch_limit;
   StatePair<T, 7> state({ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x}, (size_t)total);
   DevicePointTable dpt;
   int rc = state.open(scr, loop, stream);
@@ -304,7 +341,7 @@ int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_e
   if (rc == kOk) rc = pack_profiles(p, scr, stream);
   if (rc != kOk) {
     dpt.release(stream);
-    return scr.full ? (int)kOutOfMemory : rc;
+    return no_room(rc, scr);
   }
   TileFwdArgs<T> a;
   std::memset(&a, 0, sizeof(a));
@@ -338,7 +375,7 @@ int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_e
     t += a.steps;
   }
   timer.finish(loop.launches);
-  TIDE_HIP_TRY(hipGetLastError());
+  TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
   dpt.release(stream);
   return kOk;
@@ -354,8 +391,8 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
   const TilePlan plan = plan_tiles<T>(half, p.g.ny, p.g.nx, p.n_shots, true, true);
   const LaunchSteps loop(nt, plan.steps);
   Scratch scr(stream);
+  scr.limit = tile_scratch_limit;
   StatePair<T, 7> state({l_ey, l_hx, l_hz, ml_hz_x, ml_hx_z, ml_ey_x, ml_ey_z}, (size_t)total);
-  TIDE_CHECK(state.open(scr, loop, stream));
   TileAdjArgs<T> a;
   std::memset(&a, 0, sizeof(a));
   a.per_shot_grad = ((gca && p.g.ca_b) || (gcb && p.g.cb_b)) ? 1 : 0;
@@ -363,17 +400,21 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
   // into gca / gcb in group order at the end (no atomics, repeatable).
   const int64_t n_groups = (n_shots + plan.group - 1) / plan.group;
   double *acc[2] = {nullptr, nullptr}, *const grad[2] = {gca, gcb};
-  if (n_groups > 1 && !a.per_shot_grad) {
-    a.group_stride = numel;
-    for (int k = 0; k < 2; ++k) {
-      if (grad[k] == nullptr) continue;
-      TIDE_CHECK(scr.alloc(&acc[k], (size_t)(n_groups * numel)));
-      TIDE_HIP_TRY(hipMemsetAsync(acc[k], 0, (size_t)(n_groups * numel) * sizeof(double), stream));
-    }
-  }
+  const size_t slices = (size_t)(n_groups * numel);
+  const bool sliced = n_groups > 1 && !a.per_shot_grad;
   DevicePointTable dpt;
-  TIDE_CHECK(upload_points_lanes(p, plan, src, rec, dpt, stream));
-  TIDE_CHECK(pack_profiles(p, scr, stream));
+  int rc = state.open(scr, loop, stream);
+  for (int k = 0; k < 2; ++k)
+    if (rc == kOk && sliced && grad[k] != nullptr) rc = scr.alloc(&acc[k], slices);
+  if (rc == kOk) rc = upload_points_lanes(p, plan, src, rec, dpt, stream);
+  if (rc == kOk) rc = pack_profiles(p, scr, stream);
+  if (rc != kOk) {
+    dpt.release(stream);
+    return no_room(rc, scr);
+  }
+  if (sliced) a.group_stride = numel;
+  for (int k = 0; k < 2; ++k)
+    if (acc[k]) TIDE_HIP_TRY(hipMemsetAsync(acc[k], 0, slices * sizeof(double), stream));
   a.g = p.g;
   a.pts = Points{dpt.row_slot, dpt.seg, dpt.ent, dpt.n_xt};
   a.ca = p.ca;
@@ -408,11 +449,11 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
     t -= a.steps;
   }
   timer.finish(loop.launches);
-  TIDE_HIP_TRY(hipGetLastError());
+  TIDE_CHECK(launched());
   const unsigned fold_blocks = (unsigned)((numel + 255) / 256);
   for (int k = 0; k < 2; ++k)
     if (acc[k]) fold_groups<<<fold_blocks, 256, 0, stream>>>(grad[k], acc[k], numel, (int)n_groups);
-  TIDE_HIP_TRY(hipGetLastError());
+  TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
   dpt.release(stream);
   return kOk;
@@ -428,13 +469,18 @@ int born_tiles(int half, Problem<T> p, T *const bg[7], T *const sc[7], const T *
   const TilePlan plan = plan_born<T>(half, p.g.ny, p.g.nx, p.n_shots);
   const LaunchSteps loop(nt, plan.steps);
   Scratch scr(stream);
+  scr.limit = tile_scratch_limit;
   StatePair<T, 14> state({bg[0], bg[1], bg[2], bg[3], bg[4], bg[5], bg[6], sc[0], sc[1], sc[2],
                           sc[3], sc[4], sc[5], sc[6]},
                          (size_t)total);
-  TIDE_CHECK(state.open(scr, loop, stream));
   DevicePointTable dpt;
-  TIDE_CHECK(upload_points_lanes(p, plan, src, rec, dpt, stream));
-  TIDE_CHECK(pack_profiles(p, scr, stream));
+  int rc = state.open(scr, loop, stream);
+  if (rc == kOk) rc = upload_points_lanes(p, plan, src, rec, dpt, stream);
+  if (rc == kOk) rc = pack_profiles(p, scr, stream);
+  if (rc != kOk) {
+    dpt.release(stream);
+    return no_room(rc, scr);
+  }
   TileBornArgs<T> a;
   std::memset(&a, 0, sizeof(a));
   a.g = p.g;
@@ -464,7 +510,7 @@ int born_tiles(int half, Problem<T> p, T *const bg[7], T *const sc[7], const T *
     launch_tile_born<T>(half, plan, hist != nullptr, stream, a);
     t += a.steps;
   }
-  TIDE_HIP_TRY(hipGetLastError());
+  TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
   dpt.release(stream);
   return kOk;
@@ -496,13 +542,11 @@ int forward_impl(Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_h
   // snapshots: 300 x 517 cells and 8 shots 6.1 / 8.2 and 7.7 / 9.3; 1024 x 1024
   // and 4 11.7 / 16.3 and 20.9 / 22.0; 1500 x 1500 and 4 22.7 / 43 and 47 / 60;
   // 400 x 901 and 12 13.7 / 18.0 and 26.4 / 23.7 (with its adjoint 62 / 66).
-  // Calls whose tables or state copy do not fit their memory go on below.
   if (g_tuning.fwd_steps == 0 && !staged) {
-    const int rc = forward_tiles(1, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r, src, rec,
+    int rc = forward_tiles(1, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r, src, rec,
                                  nt, start_t, step_ratio, ey_store, curl_store, fmt,
                                  store_step_bytes, stream, arena, arena_cap);
-    if (rc != kOutOfMemory) return rc;
-    (void)hipGetLastError();
+    if (!falls_back(rc, arena)) return rc;
   }
   const int per_launch = g_tuning.fwd_steps == 0 ? 2 : g_tuning.fwd_steps;
   const int kblk = (per_launch >= 3 && nt >= per_launch && !staged) ? per_launch : 0;
@@ -743,11 +787,10 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
   // / three-step wavefront tiles; 1024 x 1024 and 4 30.7 / 32.5; 400 x 901 and
   // 12 35.5 / 42; 1500 x 1500 and 4 62.7 / 62.
   if (g_tuning.adj_steps == 0 && !staged) {
-    const int rc = backward_tiles(1, p, grad_r, l_ey, l_hx, l_hz, ml_ey_x, ml_ey_z, ml_hx_z,
+    int rc = backward_tiles(1, p, grad_r, l_ey, l_hx, l_hz, ml_ey_x, ml_ey_z, ml_hx_z,
                                   ml_hz_x, ey_store, curl_store, fmt, store_step_bytes, grad_f, gca,
                                   gcb, src, rec, nt, start_t, step_ratio, stream);
-    if (rc != kOutOfMemory) return rc;
-    (void)hipGetLastError();
+    if (!falls_back(rc)) return rc;
   }
   const int per_launch = g_tuning.adj_steps == 0 ? 3 : g_tuning.adj_steps;
   const int kblk = (per_launch >= 3 && nt >= per_launch && !staged) ? per_launch : 0;
@@ -1087,8 +1130,7 @@ tm2d_ho::Problem<T> ho_problem(const T *ca, const T *cb, const T *cq, const T *c
 // Whether a call of stencil order 4, 6 or 8 runs on workgroup tiles: every
 // valid one whose snapshots stay on the device.  (A host-staged call needs the
 // ring slots step by step; an invalid one gets its message from tm2d_ho.)
-// tm2d_ho, which advances in place, also takes the calls whose second copy of
-// the state does not fit in device memory.
+// tm2d_ho, which advances in place, also takes the calls that fall back.
 template <typename T>
 bool tiled_order(int stencil, const Problem<T> &p, int64_t nt, int fmt, const SnapshotStage &ey,
                  const SnapshotStage &curl) {
@@ -1137,17 +1179,19 @@ int forward_entry(T const *ca, T const *cb, T const *cq, T const *f, T *ey, T *h
                                                  n_src, n_rec, ca_b, cb_b, cq_b, pml_y0, pml_x0,
                                                  pml_y1, pml_x1);
     T *const fld[7] = {ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x};
-    rc = kOutOfMemory;
+    bool in_place = false;
     if (step_ratio <= 0) {
       set_error("step_ratio must be positive");
       rc = kInvalidArgument;
-    } else if (tiled_order(stencil, p, nt, fmt, ey_st, curl_st)) {
+    } else if (!tiled_order(stencil, p, nt, fmt, ey_st, curl_st)) {
+      in_place = true;
+    } else {
       rc = forward_tiles<T>(stencil / 2, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r,
                             sources_i, receivers_i, nt, start_t, step_ratio, ey_store, curl_store,
                             fmt, store_step_bytes, stream, nullptr, 0);
+      in_place = falls_back(rc);
     }
-    if (rc == kOutOfMemory) {
-      (void)hipGetLastError();
+    if (in_place) {
       rc = tm2d_ho::forward<T>(stencil, hp, fld, f, r, sources_i, receivers_i, nt, start_t,
                                step_ratio, ey_store, curl_store, fmt, store_step_bytes, stream,
                                &ey_st, &curl_st);
@@ -1238,16 +1282,17 @@ int backward_entry(T const *ca, T const *cb, T const *cq, T const *grad_r, T *la
                                                  pml_y1, pml_x1);
     T *const lam[7] = {lambda_ey, lambda_hx, lambda_hz, m_lambda_ey_x, m_lambda_ey_z,
                        m_lambda_hx_z, m_lambda_hz_x};
-    rc = kOutOfMemory;
+    bool in_place = true;
     if (tiled_order(stencil, p, nt, fmt, ey_st, curl_st) && (!ca_rg || ey_store_1) &&
-        (!cb_rg || curl_store_1))
+        (!cb_rg || curl_store_1)) {
       rc = backward_tiles<T>(stencil / 2, p, grad_r, lambda_ey, lambda_hx, lambda_hz,
                              m_lambda_ey_x, m_lambda_ey_z, m_lambda_hx_z, m_lambda_hz_x,
                              ey_store_1, curl_store_1, fmt, step_bytes, grad_f,
                              ca_rg ? ga : nullptr, cb_rg ? gb : nullptr, sources_i, receivers_i, nt,
                              start_t, step_ratio, stream);
-    if (rc == kOutOfMemory) {
-      (void)hipGetLastError();
+      in_place = falls_back(rc);
+    }
+    if (in_place) {
       rc = tm2d_ho::backward<T>(stencil, hp, lam, grad_r, ey_store_1, curl_store_1, fmt,
                                 step_bytes, grad_f, ca_rg ? ga : nullptr, cb_rg ? gb : nullptr,
                                 sources_i, receivers_i, nt, start_t, step_ratio, stream, &ey_st,
@@ -1263,7 +1308,7 @@ int backward_entry(T const *ca, T const *cb, T const *cq, T const *grad_r, T *la
 }
 
 // The Born forward of a valid call (of every order) runs on workgroup tiles,
-// unless its state copy does not fit in device memory: those, and the messages
+// unless its state copy does not fit and it falls back: those, and the messages
 // of invalid calls, stay with the step-by-step kernels of tm2d_ho.  A whole
 // Jacobian product, 200 x 301 cells and 16-cell CPML, 4 shots, 600 steps, fp32:
 // 17.9 ms with 8 launches per step, 3.5 ms with one per 4 to 8 steps.
@@ -1276,16 +1321,13 @@ int born_entry(int stencil, const tm2d_ho::Problem<T> &hp, T *const bg[7], T *co
                                        hp.ny, hp.nx, hp.n_src, hp.n_rec, hp.ca_b, hp.cb_b, hp.cq_b,
                                        hp.pml_y0, hp.pml_x0, hp.pml_y1, hp.pml_x1);
   const SnapshotStage none;
-  int rc = kOutOfMemory;
-  if ((dca == nullptr) == (dcb == nullptr) && tiled_order(stencil, p, nt, 1, none, none))
-    rc = born_tiles<T>(stencil / 2, p, bg, sc, dca, dcb, f0, df, r, bg_r, src, rec, nt, start_t,
-                       stream, hist);
-  if (rc == kOutOfMemory) {
-    (void)hipGetLastError();
-    rc = tm2d_ho::born_forward<T>(stencil, hp, bg, sc, dca, dcb, f0, df, r, bg_r, src, rec, nt,
-                                  start_t, stream, hist);
+  if ((dca == nullptr) == (dcb == nullptr) && tiled_order(stencil, p, nt, 1, none, none)) {
+    int rc = born_tiles<T>(stencil / 2, p, bg, sc, dca, dcb, f0, df, r, bg_r, src, rec, nt, start_t,
+                           stream, hist);
+    if (!falls_back(rc)) return rc;
   }
-  return rc;
+  return tm2d_ho::born_forward<T>(stencil, hp, bg, sc, dca, dcb, f0, df, r, bg_r, src, rec, nt,
+                                  start_t, stream, hist);
 }
 
 }  // namespace
@@ -1778,6 +1820,15 @@ extern "C" int tide_tm2d_get_adjoint_waves(int *out) {
     return kInvalidArgument;
   }
   *out = g_tuning.adj_waves;
+  return kOk;
+}
+
+extern "C" int tide_tm2d_set_tile_fallback(int on) {
+  tile_fallback = on != 0;
+  return kOk;
+}
+extern "C" int tide_tm2d_set_tile_scratch_limit(int64_t bytes) {
+  tile_scratch_limit = bytes < 0 ? SIZE_MAX : (size_t)bytes;
   return kOk;
 }
 

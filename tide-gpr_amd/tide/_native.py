@@ -317,6 +317,10 @@ def load() -> ctypes.CDLL:
     lib.tide_tm2d_set_time_block.argtypes = [ctypes.c_int] * 2
     lib.tide_tm2d_get_time_block.restype = ctypes.c_int
     lib.tide_tm2d_get_time_block.argtypes = [ctypes.POINTER(ctypes.c_int)]
+    lib.tide_tm2d_set_tile_fallback.restype = ctypes.c_int
+    lib.tide_tm2d_set_tile_fallback.argtypes = [ctypes.c_int]
+    lib.tide_tm2d_set_tile_scratch_limit.restype = ctypes.c_int
+    lib.tide_tm2d_set_tile_scratch_limit.argtypes = [ctypes.c_int64]
     lib.tide_tm2d_set_tile_split.restype = ctypes.c_int
     lib.tide_tm2d_set_tile_split.argtypes = [ctypes.c_int] * 2
     lib.tide_tm2d_get_tile_split.restype = ctypes.c_int
@@ -354,13 +358,22 @@ def call(fn, *args) -> None:
     The library allocates its scratch from HIP's stream-ordered pool, which
     cannot use blocks that torch's caching allocator holds unused: on an
     out-of-memory status the call runs once more after those blocks are
-    released.  The entry points allocate all scratch before they write any
-    caller array, so the retried call starts from the same state."""
-    status = fn(*args)
-    if (status == OUT_OF_MEMORY and torch.cuda.is_initialized()
-            and torch.cuda.memory_reserved() > torch.cuda.memory_allocated()):
-        torch.cuda.synchronize()
-        torch.cuda.empty_cache()
+    released.  Only where that does not help either may it use the slower
+    kernels that need less scratch.  The entry points allocate all scratch
+    before they write any caller array, so the retried call starts from the
+    same state."""
+    fallback = load().tide_tm2d_set_tile_fallback  # a setting of this thread
+    fallback(0)
+    try:
+        status = fn(*args)
+        if (status == OUT_OF_MEMORY and torch.cuda.is_initialized()
+                and torch.cuda.memory_reserved() > torch.cuda.memory_allocated()):
+            torch.cuda.synchronize()
+            torch.cuda.empty_cache()
+            status = fn(*args)
+    finally:
+        fallback(1)
+    if status == OUT_OF_MEMORY:
         status = fn(*args)
     check(status)
 
