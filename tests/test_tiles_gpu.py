@@ -170,6 +170,10 @@ def test_born_beside_the_tile_edges(stencil, ny, nx, nt):
 @pytest.mark.parametrize("compression,interval,graph", [(False, 1, True), (False, 3, False),
                                                         (True, 2, True)])
 def test_batched_plans_on_tiles(compression, interval, graph):
+    _check_batch(compression, interval, graph)
+
+
+def _check_batch(compression, interval, graph):
     """Problems of one and of several tiles and shots, whose loops take one
     launch, an even and an odd last launch: receivers, states and source
     gradients as the oracle's, replayed twice."""
@@ -267,3 +271,9 @@ def test_a_caller_that_can_make_room_is_told(no_room, stencil):
         no_room.tide_tm2d_set_tile_fallback(1)
     no_room.tide_tm2d_set_tile_scratch_limit(-1)
     _check(case)  # an earlier call's failure is not a later one's
+
+
+@gpu
+@pytest.mark.parametrize("graph", [False, True])
+def test_batched_plans_without_room_for_tiles_fall_back(no_room, graph):
+    _check_batch(False, 1, graph)

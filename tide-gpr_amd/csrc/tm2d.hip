@@ -259,10 +259,6 @@ inline int launched() {
   return kHipError;
 }
 
-// Of the calling thread: whether a call whose tile loop has no room goes on
-// with the kernels that need less scratch (else it returns kOutOfMemory, and a
-// caller that holds device memory unused may release it and call again), and
-// the most scratch of a tile loop in bytes.
 thread_local bool tile_fallback = true;
 thread_local size_t tile_scratch_limit = SIZE_MAX;
 

@@ -144,6 +144,7 @@ struct Plan {
   int steps_f = 1, steps_a = 1;  // time steps per launch of each pass
   int max_nt = 0;
   bool tiles_f = false, tiles_a = false;  // the passes on workgroup tiles
+  size_t tile_bytes = 0;                  // their memory
   TilePass<TileFwdArgs<float>> tile_f;
   TilePass<TileAdjArgs<float>> tile_a;
   std::vector<tide_tm2d_problem> probs;  // sorted by nt, descending
@@ -174,6 +175,19 @@ template <typename U> int plan_alloc(Plan &p, U **out, size_t count) {
   p.allocs.push_back(ptr);
   *out = (U *)ptr;
   return kOk;
+}
+
+// Memory that only the tile passes need.
+template <typename U> int tile_alloc(Plan &p, U **out, size_t count) {
+  const size_t bytes = std::max<size_t>(count, 1) * sizeof(U);
+  if (bytes > tile_scratch_limit - std::min(p.tile_bytes, tile_scratch_limit)) {
+    set_error("plan: the tile passes need more memory than their limit of " +
+              std::to_string(tile_scratch_limit) + " bytes");
+    return kOutOfMemory;
+  }
+  const int rc = plan_alloc(p, out, count);
+  if (rc == kOk) p.tile_bytes += bytes;
+  return rc;
 }
 
 int fetch_host(const int64_t *p, int64_t n, std::vector<int64_t> &out) {
@@ -611,9 +625,9 @@ TilePlan plan_batch_tiles(const Plan &p, bool adjoint, bool storing) {
 template <typename A>
 int upload_pass(Plan &p, TilePass<A> &t, const std::vector<A> &table,
                 const std::vector<int32_t> &tile_item, const std::vector<FillRange> &fills) {
-  PLAN_CHECK(plan_alloc(p, &t.table, table.size()));
-  PLAN_CHECK(plan_alloc(p, &t.tile_item, tile_item.size()));
-  PLAN_CHECK(plan_alloc(p, &t.fills, fills.size()));
+  PLAN_CHECK(tile_alloc(p, &t.table, table.size()));
+  PLAN_CHECK(tile_alloc(p, &t.tile_item, tile_item.size()));
+  PLAN_CHECK(tile_alloc(p, &t.fills, fills.size()));
   TIDE_HIP_TRY(hipMemcpy(t.table, table.data(), table.size() * sizeof(A), hipMemcpyHostToDevice));
   TIDE_HIP_TRY(hipMemcpy(t.tile_item, tile_item.data(), tile_item.size() * sizeof(int32_t),
                          hipMemcpyHostToDevice));
@@ -735,8 +749,8 @@ int build_tiles_backward(Plan &p) {
     it.n_groups = a.n_shots;
     if (q.n_shots > 1 && (q.grad_ca || q.grad_cb)) {
       it.group_stride = a.group_stride = numel;
-      if (q.grad_ca) PLAN_CHECK(plan_alloc(p, &it.gca, (size_t)total));
-      if (q.grad_cb) PLAN_CHECK(plan_alloc(p, &it.gcb, (size_t)total));
+      if (q.grad_ca) PLAN_CHECK(tile_alloc(p, &it.gca, (size_t)total));
+      if (q.grad_cb) PLAN_CHECK(tile_alloc(p, &it.gcb, (size_t)total));
     }
     const LaunchSteps loop(q.nt, t.plan.steps);
     int64_t s = q.nt - 1;
@@ -782,7 +796,7 @@ using namespace tide_hip::tm2d;
 
 namespace {
 int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t storage_format,
-               int64_t use_graph, int64_t device);
+               int64_t use_graph, int64_t device, bool tiles);
 }  // namespace
 
 extern "C" int tide_tm2d_plan_create(const tide_tm2d_problem *problems, int64_t n,
@@ -798,7 +812,14 @@ extern "C" int tide_tm2d_plan_create(const tide_tm2d_problem *problems, int64_t 
     return kHipError;
   }
   Plan *p = new Plan();
-  const int rc = build_plan(p, problems, n, storage_format, use_graph, device);
+  int rc = build_plan(p, problems, n, storage_format, use_graph, device, true);
+  if (rc == kOutOfMemory && tile_fallback && (p->tiles_f || p->tiles_a)) {
+    // the step launches need less: no argument records, a gradient slice per
+    // group of shots instead of one per shot
+    destroy(p);
+    p = new Plan();
+    rc = build_plan(p, problems, n, storage_format, use_graph, device, false);
+  }
   if (rc != kOk) {
     destroy(p);
     return rc;
@@ -850,7 +871,7 @@ int build_step_launches(Plan &p, const std::vector<BatchItem<float>> &proto, boo
 }
 
 int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t storage_format,
-               int64_t use_graph, int64_t device) {
+               int64_t use_graph, int64_t device, bool tiles) {
   p->device = (int)device;
   p->n = n;
   p->use_graph = use_graph != 0;
@@ -869,7 +890,7 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
   for (int64_t m = 0; m < n; ++m)
     cells += std::max<int64_t>(problems[m].n_shots, 0) * std::max<int64_t>(problems[m].ny, 0) *
              std::max<int64_t>(problems[m].nx, 0);
-  p->tiles_f = g_tuning.fwd_steps == 0 && g_tuning.adj_steps == 0;
+  p->tiles_f = tiles && g_tuning.fwd_steps == 0 && g_tuning.adj_steps == 0;
   p->tiles_a = p->tiles_f && cells <= kBatchTileCells;
   p->steps_f = g_tuning.fwd_steps == 1 ? 1 : 2;
   p->steps_a = g_tuning.adj_steps == 1 ? 1 : 2;

@@ -145,6 +145,13 @@ struct LaunchSteps {
   bool ends_in_scratch() const { return (launches & 1) != 0; }
 };
 
+// Of the calling thread: whether a call whose tile loop has no room goes on
+// with the kernels that need less scratch (else it returns kOutOfMemory, and a
+// caller that holds device memory unused may release it and call again), and
+// the most scratch of a tile loop in bytes.
+extern thread_local bool tile_fallback;
+extern thread_local size_t tile_scratch_limit;
+
 template <typename T>
 void launch_tile_fwd(int half, const TilePlan &p, int fmt, hipStream_t stream, const TileFwdArgs<T> &a);
 template <typename T>

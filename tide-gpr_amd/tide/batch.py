@@ -123,10 +123,11 @@ class TM2DBatch:
             self._fill(table[i], st)
         self._table = table
         handle = _P()
-        _native.check(self._lib.tide_tm2d_plan_create(
+        _native.call(
+            self._lib.tide_tm2d_plan_create,
             table, len(self.problems), 1 if bf16 else 0, 1 if use_graph else 0,
             dev.index if dev.index is not None else torch.cuda.current_device(),
-            ctypes.byref(handle)))
+            ctypes.byref(handle))
         self._plan = handle
 
     # ------------------------------------------------------------ buffers
