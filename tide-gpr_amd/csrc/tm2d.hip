@@ -125,14 +125,14 @@ inline int fetch_indices(const int64_t *p, int64_t n, std::vector<int64_t> &out,
 
 // Scratch device memory of one call: stream-ordered allocations freed when
 // the call returns, or, with an arena, consecutive 256-byte aligned pieces
-// of caller-provided device memory (nothing allocated or freed).
+// of caller-provided device memory (nothing allocated or freed) or of one
+// allocation made by reserve().
 struct Scratch {
   std::vector<void *> bufs;
   hipStream_t stream;
   char *arena = nullptr;
   size_t cap = 0, used = 0;
-  size_t limit = SIZE_MAX;  // most bytes of stream-ordered allocations
-  bool full = false;        // an allocation did not fit
+  bool full = false;  // a piece did not fit
   explicit Scratch(hipStream_t s, char *arena_ = nullptr, size_t cap_ = 0)
       : stream(s), arena(arena_), cap(cap_) {}
   ~Scratch() {
@@ -152,8 +152,21 @@ struct Scratch {
       used = at + bytes;
       return kOk;
     }
-    if (bytes > limit - used) {
-      full = true;
+    void *p = nullptr;
+    TIDE_HIP_TRY(hipMallocAsync(&p, bytes, stream));
+    bufs.push_back(p);
+    *out = (U *)p;
+    return kOk;
+  }
+  // Bytes of an arena that `count` values take at most.
+  template <typename U> static size_t space(size_t count) {
+    return (std::max<size_t>(count, 1) * sizeof(U) + 255) & ~(size_t)255;
+  }
+  // One allocation for all pieces of the call, unless it has an arena.  (An
+  // allocation per array took up to 0.2 ms of a call, more than a few steps.)
+  int reserve(size_t bytes, size_t limit) {
+    if (arena != nullptr) return kOk;
+    if (bytes > limit) {
       set_error("the call needs more scratch memory than its limit of " + std::to_string(limit) +
                 " bytes");
       return kOutOfMemory;
@@ -161,8 +174,8 @@ struct Scratch {
     void *p = nullptr;
     TIDE_HIP_TRY(hipMallocAsync(&p, bytes, stream));
     bufs.push_back(p);
-    used += bytes;
-    *out = (U *)p;
+    arena = (char *)p;
+    cap = bytes;
     return kOk;
   }
 };
@@ -270,20 +283,6 @@ inline bool falls_back(int &rc, const char *arena = nullptr) {
   return false;
 }
 
-template <typename T>
-int upload_points_lanes(const Problem<T> &p, const TilePlan &plan, const int64_t *src,
-                        const int64_t *rec, DevicePointTable &dpt, hipStream_t stream,
-                        Scratch *arena_scr = nullptr) {
-  std::vector<int64_t> hsrc, hrec;
-  TIDE_CHECK(fetch_indices(src, (int64_t)p.n_shots * p.n_src, hsrc, stream));
-  TIDE_CHECK(fetch_indices(rec, (int64_t)p.n_shots * p.n_rec, hrec, stream));
-  PointTable table;
-  if (!build_point_table_lanes(hsrc.data(), p.n_src, hrec.data(), p.n_rec, p.n_shots, p.g.ny,
-                               p.g.nx, plan.own_cols, plan.halo, table))
-    return kInvalidArgument;
-  return put_table(table, dpt, arena_scr, stream);
-}
-
 // The N state arrays of a time loop and the scratch copy they ping-pong with.
 // The strips' memories (all but the first three of each seven) are only
 // written inside their strips: where the scratch copy ends up as the result,
@@ -319,6 +318,38 @@ template <typename T, int N> struct StatePair {
   }
 };
 
+// Scratch of a tile loop: the state copy, the profiles and the point table, and
+// up to two FP64 arrays of `slices` values each.
+template <typename T, int N>
+int open_tiles(Problem<T> &p, const TilePlan &plan, const int64_t *src, const int64_t *rec,
+               const LaunchSteps &loop, Scratch &scr, StatePair<T, N> &state,
+               DevicePointTable &dpt, hipStream_t stream, size_t slices = 0,
+               double **acc0 = nullptr, double **acc1 = nullptr) {
+  std::vector<int64_t> hsrc, hrec;
+  TIDE_CHECK(fetch_indices(src, (int64_t)p.n_shots * p.n_src, hsrc, stream));
+  TIDE_CHECK(fetch_indices(rec, (int64_t)p.n_shots * p.n_rec, hrec, stream));
+  PointTable table;
+  if (!build_point_table_lanes(hsrc.data(), p.n_src, hrec.data(), p.n_rec, p.n_shots, p.g.ny,
+                               p.g.nx, plan.own_cols, plan.halo, table))
+    return kInvalidArgument;
+  double **const acc[2] = {acc0, acc1};
+  size_t bytes = N * Scratch::space<T>(state.total) +
+                 Scratch::space<T>((size_t)6 * (p.g.ny + p.g.nx)) +
+                 Scratch::space<int32_t>(DevicePointTable::row_slot_count(table)) +
+                 Scratch::space<int32_t>(DevicePointTable::seg_count(table)) +
+                 Scratch::space<int2>(DevicePointTable::ent_count(table));
+  for (double **a : acc) bytes += a != nullptr ? Scratch::space<double>(slices) : 0;
+  TIDE_CHECK(scr.reserve(bytes, tile_scratch_limit));
+  TIDE_CHECK(state.open(scr, loop, stream));
+  for (double **a : acc) {
+    if (a == nullptr) continue;
+    TIDE_CHECK(scr.alloc(a, slices));
+    TIDE_HIP_TRY(hipMemsetAsync(*a, 0, slices * sizeof(double), stream));
+  }
+  TIDE_CHECK(pack_profiles(p, scr, stream));
+  return put_table(table, dpt, &scr, stream);
+}
+
 template <typename T>
 int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_hx_z,
                   T *m_hz_x, const T *f, T *r, const int64_t *src, const int64_t *rec, int64_t nt,
@@ -329,16 +360,10 @@ int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_e
                                        ey_store || curl_store);
   const LaunchSteps loop(nt, plan.steps);
   Scratch scr(stream, arena, arena_cap);
-  scr.limit = tile_scratch_limit;
   StatePair<T, 7> state({ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x}, (size_t)total);
   DevicePointTable dpt;
-  int rc = state.open(scr, loop, stream);
-  if (rc == kOk) rc = upload_points_lanes(p, plan, src, rec, dpt, stream, &scr);
-  if (rc == kOk) rc = pack_profiles(p, scr, stream);
-  if (rc != kOk) {
-    dpt.release(stream);
-    return no_room(rc, scr);
-  }
+  const int rc = open_tiles(p, plan, src, rec, loop, scr, state, dpt, stream);
+  if (rc != kOk) return no_room(rc, scr);
   TileFwdArgs<T> a;
   std::memset(&a, 0, sizeof(a));
   a.g = p.g;
@@ -373,7 +398,6 @@ int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_e
   timer.finish(loop.launches);
   TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
-  dpt.release(stream);
   return kOk;
 }
 
@@ -387,7 +411,6 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
   const TilePlan plan = plan_tiles<T>(half, p.g.ny, p.g.nx, p.n_shots, true, true);
   const LaunchSteps loop(nt, plan.steps);
   Scratch scr(stream);
-  scr.limit = tile_scratch_limit;
   StatePair<T, 7> state({l_ey, l_hx, l_hz, ml_hz_x, ml_hx_z, ml_ey_x, ml_ey_z}, (size_t)total);
   TileAdjArgs<T> a;
   std::memset(&a, 0, sizeof(a));
@@ -396,21 +419,13 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
   // into gca / gcb in group order at the end (no atomics, repeatable).
   const int64_t n_groups = (n_shots + plan.group - 1) / plan.group;
   double *acc[2] = {nullptr, nullptr}, *const grad[2] = {gca, gcb};
-  const size_t slices = (size_t)(n_groups * numel);
   const bool sliced = n_groups > 1 && !a.per_shot_grad;
-  DevicePointTable dpt;
-  int rc = state.open(scr, loop, stream);
-  for (int k = 0; k < 2; ++k)
-    if (rc == kOk && sliced && grad[k] != nullptr) rc = scr.alloc(&acc[k], slices);
-  if (rc == kOk) rc = upload_points_lanes(p, plan, src, rec, dpt, stream);
-  if (rc == kOk) rc = pack_profiles(p, scr, stream);
-  if (rc != kOk) {
-    dpt.release(stream);
-    return no_room(rc, scr);
-  }
   if (sliced) a.group_stride = numel;
-  for (int k = 0; k < 2; ++k)
-    if (acc[k]) TIDE_HIP_TRY(hipMemsetAsync(acc[k], 0, slices * sizeof(double), stream));
+  DevicePointTable dpt;
+  const int rc = open_tiles(p, plan, src, rec, loop, scr, state, dpt, stream,
+                            (size_t)(n_groups * numel), sliced && gca ? &acc[0] : nullptr,
+                            sliced && gcb ? &acc[1] : nullptr);
+  if (rc != kOk) return no_room(rc, scr);
   a.g = p.g;
   a.pts = Points{dpt.row_slot, dpt.seg, dpt.ent, dpt.n_xt};
   a.ca = p.ca;
@@ -451,7 +466,6 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
     if (acc[k]) fold_groups<<<fold_blocks, 256, 0, stream>>>(grad[k], acc[k], numel, (int)n_groups);
   TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
-  dpt.release(stream);
   return kOk;
 }
 
@@ -465,18 +479,12 @@ int born_tiles(int half, Problem<T> p, T *const bg[7], T *const sc[7], const T *
   const TilePlan plan = plan_born<T>(half, p.g.ny, p.g.nx, p.n_shots);
   const LaunchSteps loop(nt, plan.steps);
   Scratch scr(stream);
-  scr.limit = tile_scratch_limit;
   StatePair<T, 14> state({bg[0], bg[1], bg[2], bg[3], bg[4], bg[5], bg[6], sc[0], sc[1], sc[2],
                           sc[3], sc[4], sc[5], sc[6]},
                          (size_t)total);
   DevicePointTable dpt;
-  int rc = state.open(scr, loop, stream);
-  if (rc == kOk) rc = upload_points_lanes(p, plan, src, rec, dpt, stream);
-  if (rc == kOk) rc = pack_profiles(p, scr, stream);
-  if (rc != kOk) {
-    dpt.release(stream);
-    return no_room(rc, scr);
-  }
+  const int rc = open_tiles(p, plan, src, rec, loop, scr, state, dpt, stream);
+  if (rc != kOk) return no_room(rc, scr);
   TileBornArgs<T> a;
   std::memset(&a, 0, sizeof(a));
   a.g = p.g;
@@ -508,7 +516,6 @@ int born_tiles(int half, Problem<T> p, T *const bg[7], T *const sc[7], const T *
   }
   TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
-  dpt.release(stream);
   return kOk;
 }
 
