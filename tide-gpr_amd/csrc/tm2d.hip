@@ -30,6 +30,7 @@
 #include "tm2d_fused.h"
 #include "tm2d_launch.h"
 #include "tm2d_launch_k.h"
+#include "tm2d_route.h"
 #include "tm2d_tile_launch.h"
 #include "tide_hip.h"
 #include "tide_storage.h"
@@ -89,6 +90,11 @@ struct LoopTimer {
     start = stop = nullptr;
   }
 };
+
+// What the calling thread's time loops have enqueued: launches on workgroup
+// tiles, launches on wavefront tiles, steps taken in place.
+enum { kTileLaunches = 0, kWavefrontLaunches, kInPlaceSteps };
+thread_local int64_t loop_counts[3] = {0, 0, 0};
 
 constexpr int kMaxLoopTiles = 4;  // wavefronts per workgroup of the shot-looping kernels
 
@@ -396,6 +402,7 @@ int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_e
     t += a.steps;
   }
   timer.finish(loop.launches);
+  loop_counts[kTileLaunches] += loop.launches;
   TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
   return kOk;
@@ -460,6 +467,7 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
     t -= a.steps;
   }
   timer.finish(loop.launches);
+  loop_counts[kTileLaunches] += loop.launches;
   TIDE_CHECK(launched());
   const unsigned fold_blocks = (unsigned)((numel + 255) / 256);
   for (int k = 0; k < 2; ++k)
@@ -514,6 +522,7 @@ int born_tiles(int half, Problem<T> p, T *const bg[7], T *const sc[7], const T *
     launch_tile_born<T>(half, plan, hist != nullptr, stream, a);
     t += a.steps;
   }
+  loop_counts[kTileLaunches] += loop.launches;
   TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
   return kOk;
@@ -540,11 +549,6 @@ int forward_impl(Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_h
   const bool staged = (ey_stage && ey_stage->active()) || (curl_stage && curl_stage->active());
   // K-step launches (K = 3, 4) need K ring slots at once, more than a
   // host-staged ring holds: staged calls use two-step launches.
-  // Without a setting the loop runs on workgroup tiles, whatever the size.
-  // fp32, us per step, tiles / two-step wavefront tiles, forward and with
-  // snapshots: 300 x 517 cells and 8 shots 6.1 / 8.2 and 7.7 / 9.3; 1024 x 1024
-  // and 4 11.7 / 16.3 and 20.9 / 22.0; 1500 x 1500 and 4 22.7 / 43 and 47 / 60;
-  // 400 x 901 and 12 13.7 / 18.0 and 26.4 / 23.7 (with its adjoint 62 / 66).
   if (g_tuning.fwd_steps == 0 && !staged) {
     int rc = forward_tiles(1, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r, src, rec,
                                  nt, start_t, step_ratio, ey_store, curl_store, fmt,
@@ -735,6 +739,7 @@ int forward_impl(Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_h
     for (int k = 0; k < 5; ++k) std::swap(cur[k], nxt[k]);
   }
   timer.finish(launches);
+  loop_counts[kWavefrontLaunches] += launches;
   TIDE_HIP_TRY(hipGetLastError());
   if (cur[0] != ey) {
     TIDE_HIP_TRY(hipMemcpyAsync(ey, cur[0], bytes, hipMemcpyDeviceToDevice, stream));
@@ -786,9 +791,7 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
   const int64_t n_shots = p.n_shots, total = n_shots * p.g.numel;
   const bool staged = (ey_stage && ey_stage->active()) || (curl_stage && curl_stage->active());
   // K-step launches need K ring slots at once (see forward_impl)
-  // As the forward: 300 x 517 cells and 8 shots 12.8 / 14.8 us per step, tiles
-  // / three-step wavefront tiles; 1024 x 1024 and 4 30.7 / 32.5; 400 x 901 and
-  // 12 35.5 / 42; 1500 x 1500 and 4 62.7 / 62.
+  const bool per_shot = (gca && p.g.ca_b) || (gcb && p.g.cb_b);
   if (g_tuning.adj_steps == 0 && !staged) {
     int rc = backward_tiles(1, p, grad_r, l_ey, l_hx, l_hz, ml_ey_x, ml_ey_z, ml_hx_z,
                                   ml_hz_x, ey_store, curl_store, fmt, store_step_bytes, grad_f, gca,
@@ -819,7 +822,7 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
   a.ca = p.ca;
   a.cb = p.cb;
   a.cq = p.cq;
-  a.per_shot_grad = ((gca && p.g.ca_b) || (gcb && p.g.cb_b)) ? 1 : 0;
+  a.per_shot_grad = per_shot ? 1 : 0;
   a.step_scale = (double)step_ratio;
   a.n_shots = p.n_shots;
   const int rows = rows_for<T>(g_tuning.adj_rows);
@@ -994,6 +997,7 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
     for (int k = 0; k < 7; ++k) std::swap(cur[k], nxt[k]);
   }
   timer.finish(launches);
+  loop_counts[kWavefrontLaunches] += launches;
   TIDE_HIP_TRY(hipGetLastError());
   const unsigned fold_blocks = (unsigned)((numel + 255) / 256);
   if (gacc) fold_groups<<<fold_blocks, 256, 0, stream>>>(gca, gacc, numel, (int)n_groups);
@@ -1130,10 +1134,11 @@ tm2d_ho::Problem<T> ho_problem(const T *ca, const T *cb, const T *cq, const T *c
   return hp;
 }
 
-// Whether a call of stencil order 4, 6 or 8 runs on workgroup tiles: every
+// Whether a call of stencil order 4, 6 or 8 can run on workgroup tiles: every
 // valid one whose snapshots stay on the device.  (A host-staged call needs the
 // ring slots step by step; an invalid one gets its message from tm2d_ho.)
-// tm2d_ho, which advances in place, also takes the calls that fall back.
+// tm2d_ho, which advances in place, also takes the calls that fall back and
+// those of tm2d_route.h.
 template <typename T>
 bool tiled_order(int stencil, const Problem<T> &p, int64_t nt, int fmt, const SnapshotStage &ey,
                  const SnapshotStage &curl) {
@@ -1186,7 +1191,8 @@ int forward_entry(T const *ca, T const *cb, T const *cq, T const *f, T *ey, T *h
     if (step_ratio <= 0) {
       set_error("step_ratio must be positive");
       rc = kInvalidArgument;
-    } else if (!tiled_order(stencil, p, nt, fmt, ey_st, curl_st)) {
+    } else if (!tiled_order(stencil, p, nt, fmt, ey_st, curl_st) ||
+               in_place_forward(stencil / 2, sizeof(T), n_shots, ny * nx, nt)) {
       in_place = true;
     } else {
       rc = forward_tiles<T>(stencil / 2, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r,
@@ -1198,6 +1204,7 @@ int forward_entry(T const *ca, T const *cb, T const *cq, T const *f, T *ey, T *h
       rc = tm2d_ho::forward<T>(stencil, hp, fld, f, r, sources_i, receivers_i, nt, start_t,
                                step_ratio, ey_store, curl_store, fmt, store_step_bytes, stream,
                                &ey_st, &curl_st);
+      if (rc == kOk) loop_counts[kInPlaceSteps] += nt;
     }
   }
   return close_stages(rc, ey_st, curl_st);
@@ -1287,7 +1294,7 @@ int backward_entry(T const *ca, T const *cb, T const *cq, T const *grad_r, T *la
                        m_lambda_hx_z, m_lambda_hz_x};
     bool in_place = true;
     if (tiled_order(stencil, p, nt, fmt, ey_st, curl_st) && (!ca_rg || ey_store_1) &&
-        (!cb_rg || curl_store_1)) {
+        (!cb_rg || curl_store_1) && !in_place_adjoint(nt)) {
       rc = backward_tiles<T>(stencil / 2, p, grad_r, lambda_ey, lambda_hx, lambda_hz,
                              m_lambda_ey_x, m_lambda_ey_z, m_lambda_hx_z, m_lambda_hz_x,
                              ey_store_1, curl_store_1, fmt, step_bytes, grad_f,
@@ -1300,6 +1307,7 @@ int backward_entry(T const *ca, T const *cb, T const *cq, T const *grad_r, T *la
                                 step_bytes, grad_f, ca_rg ? ga : nullptr, cb_rg ? gb : nullptr,
                                 sources_i, receivers_i, nt, start_t, step_ratio, stream, &ey_st,
                                 &curl_st);
+      if (rc == kOk) loop_counts[kInPlaceSteps] += nt;
     }
   }
   TIDE_CHECK(close_stages(rc, ey_st, curl_st));
@@ -1310,8 +1318,8 @@ int backward_entry(T const *ca, T const *cb, T const *cq, T const *grad_r, T *la
   return kOk;
 }
 
-// The Born forward of a valid call (of every order) runs on workgroup tiles,
-// unless its state copy does not fit and it falls back: those, and the messages
+// The Born forward of a valid call (of every order) runs on workgroup tiles but
+// for those of tm2d_route.h and those that fall back: these, and the messages
 // of invalid calls, stay with the step-by-step kernels of tm2d_ho.  A whole
 // Jacobian product, 200 x 301 cells and 16-cell CPML, 4 shots, 600 steps, fp32:
 // 17.9 ms with 8 launches per step, 3.5 ms with one per 4 to 8 steps.
@@ -1324,13 +1332,16 @@ int born_entry(int stencil, const tm2d_ho::Problem<T> &hp, T *const bg[7], T *co
                                        hp.ny, hp.nx, hp.n_src, hp.n_rec, hp.ca_b, hp.cb_b, hp.cq_b,
                                        hp.pml_y0, hp.pml_x0, hp.pml_y1, hp.pml_x1);
   const SnapshotStage none;
-  if ((dca == nullptr) == (dcb == nullptr) && tiled_order(stencil, p, nt, 1, none, none)) {
+  if ((dca == nullptr) == (dcb == nullptr) && tiled_order(stencil, p, nt, 1, none, none) &&
+      !in_place_born(stencil / 2, sizeof(T), hp.n_shots, hp.ny * hp.nx)) {
     int rc = born_tiles<T>(stencil / 2, p, bg, sc, dca, dcb, f0, df, r, bg_r, src, rec, nt, start_t,
                            stream, hist);
     if (!falls_back(rc)) return rc;
   }
-  return tm2d_ho::born_forward<T>(stencil, hp, bg, sc, dca, dcb, f0, df, r, bg_r, src, rec, nt,
-                                  start_t, stream, hist);
+  const int rc = tm2d_ho::born_forward<T>(stencil, hp, bg, sc, dca, dcb, f0, df, r, bg_r, src, rec,
+                                          nt, start_t, stream, hist);
+  if (rc == kOk) loop_counts[kInPlaceSteps] += nt;
+  return rc;
 }
 
 }  // namespace
@@ -1826,6 +1837,17 @@ extern "C" int tide_tm2d_get_adjoint_waves(int *out) {
   return kOk;
 }
 
+extern "C" int tide_tm2d_take_launches(int64_t *out3) {
+  if (out3 == nullptr) {
+    set_error("take_launches: output required");
+    return kInvalidArgument;
+  }
+  for (int k = 0; k < 3; ++k) {
+    out3[k] = loop_counts[k];
+    loop_counts[k] = 0;
+  }
+  return kOk;
+}
 extern "C" int tide_tm2d_set_tile_fallback(int on) {
   tile_fallback = on != 0;
   return kOk;

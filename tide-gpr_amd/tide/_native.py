@@ -317,6 +317,8 @@ def load() -> ctypes.CDLL:
     lib.tide_tm2d_set_time_block.argtypes = [ctypes.c_int] * 2
     lib.tide_tm2d_get_time_block.restype = ctypes.c_int
     lib.tide_tm2d_get_time_block.argtypes = [ctypes.POINTER(ctypes.c_int)]
+    lib.tide_tm2d_take_launches.restype = ctypes.c_int
+    lib.tide_tm2d_take_launches.argtypes = [ctypes.POINTER(ctypes.c_int64)]
     lib.tide_tm2d_set_tile_fallback.restype = ctypes.c_int
     lib.tide_tm2d_set_tile_fallback.argtypes = [ctypes.c_int]
     lib.tide_tm2d_set_tile_scratch_limit.restype = ctypes.c_int
@@ -486,6 +488,14 @@ def set_tm2d_time_block(fwd_steps: int, adj_steps: int) -> None:
     check(load().tide_tm2d_set_time_block(int(fwd_steps), int(adj_steps)))
 
 
+def take_tm2d_launches() -> tuple[int, int, int]:
+    """Launches on workgroup tiles and on wavefront tiles, and steps taken in
+    place, of this thread's 2-D calls since it last asked."""
+    out = (ctypes.c_int64 * 3)()
+    check(load().tide_tm2d_take_launches(out))
+    return int(out[0]), int(out[1]), int(out[2])
+
+
 def get_tm2d_time_block() -> tuple[int, int]:
     out = (ctypes.c_int * 2)()
     check(load().tide_tm2d_get_time_block(out))
@@ -547,6 +557,7 @@ __all__ = [
     "get_tm2d_shot_loop",
     "get_tm2d_tile_split",
     "get_tm2d_time_block",
+    "take_tm2d_launches",
     "get_tm2d_tuning",
     "int64_array",
     "ptr_array",
