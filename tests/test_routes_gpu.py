@@ -1,12 +1,22 @@
 """Which kernels the 2-D calls run on (MI355X): workgroup tiles, or the
-in-place kernels where those measured faster."""
+wavefront tiles and in-place kernels where those measured faster, and the
+latter against the CPU oracle over the forms of call that reach them.
+
+Tolerances as in test_tiles_gpu.py: everything bit-identical but the FP64
+coefficient gradients, which are reordered sums.
+"""
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
 import tide
+from gpu_abi import gpu_backward, gpu_forward
+from helpers import FIELD_NAMES, relative_l2
+from oracle import oracle as O
+from test_tiles_gpu import _case
 from tide.workflow import ReceiverObjective
 
 pytestmark = pytest.mark.gpu
@@ -43,12 +53,12 @@ def _family(fn):
 @pytest.mark.parametrize("case,forward,gradient", [
     # forward alone; forward with snapshots and adjoint of one gradient
     (dict(ny=96, nx=96, shots=1, nt=64), {TILES}, {TILES}),
-    (dict(ny=1065, nx=1065, shots=4, nt=64), {TILES}, {TILES}),
-    (dict(ny=1065, nx=1065, shots=4, nt=64, compression=True), {TILES}, {TILES}),
+    (dict(ny=1065, nx=1065, shots=4, nt=64), {TILES}, {TILES, WAVEFRONT}),
+    (dict(ny=1065, nx=1065, shots=4, nt=64, compression=True), {TILES}, {TILES, WAVEFRONT}),
     (dict(ny=1065, nx=1065, shots=4, nt=24), {TILES}, {TILES}),
     (dict(ny=1065, nx=1065, shots=3, nt=64), {TILES}, {TILES}),
-    (dict(ny=768, nx=800, shots=12, nt=64), {TILES}, {TILES}),
-    (dict(ny=441, nx=942, shots=12, nt=64), {TILES}, {TILES}),
+    (dict(ny=768, nx=800, shots=12, nt=64), {TILES}, {WAVEFRONT}),
+    (dict(ny=441, nx=942, shots=12, nt=64), {TILES}, {TILES, WAVEFRONT}),
     (dict(ny=441, nx=942, shots=12, nt=64, compression=True), {TILES}, {TILES}),
     (dict(ny=700, nx=700, shots=4, nt=64, dtype=torch.float64), {TILES}, {TILES}),
     (dict(ny=96, nx=96, shots=2, nt=7, stencil=4), {IN_PLACE}, {IN_PLACE, TILES}),
@@ -81,3 +91,32 @@ def test_jacobian_products_run_on_the_kernels_that_measured_faster(case, family)
                                  sigma=torch.zeros_like(model.sigma))
     with op.linearize(model) as lin:
         assert _family(lambda: lin.jvp(direction)) == {family}
+
+
+@pytest.mark.parametrize("store,interval,batched,one", [
+    ("full", 1, False, False), ("full", 1, True, False), ("full", 3, False, False),
+    ("bf16", 1, False, False), ("bf16", 2, False, False), ("full", 1, False, True)])
+@pytest.mark.parametrize("ny,nx,shots", [(41, 67, 7), (60, 75, 4)])
+def test_wavefront_tiles_match_the_oracle(store, interval, batched, one, ny, nx, shots):
+    """The two- and three-step wavefront tiles at their default shapes."""
+    case = _case(ny, nx, 23, shots=shots, batched=batched)
+    before = tide._native.get_tm2d_time_block()
+    tide._native.set_tm2d_time_block(2, 3)
+    try:
+        tide._native.take_tm2d_launches()
+        f_o, r_o, es, cs = O.tm2d_forward(case, store=store, interval=interval)
+        f_g, r_g, es_g, cs_g = gpu_forward(case, store=store, interval=interval)
+        assert np.array_equal(r_g, r_o)
+        assert np.array_equal(es_g, es) and np.array_equal(cs_g, cs)
+        for name, a, b in zip(FIELD_NAMES, f_g, f_o):
+            assert np.array_equal(a, b), name
+        w = np.random.default_rng(3).standard_normal(r_o.shape).astype(case.dtype)
+        ga_o, gb_o, gf_o, lam_o = O.tm2d_backward(case, w, es, cs, store=store, interval=interval)
+        ga, gb, gf, lam = gpu_backward(case, w, es_g, None if one else cs_g, store=store,
+                                       interval=interval)
+        assert all(np.array_equal(a.reshape(b.shape), b) for a, b in zip(lam, lam_o))
+        assert np.array_equal(gf, gf_o) and relative_l2(ga, ga_o) < 1e-12
+        assert one or relative_l2(gb, gb_o) < 1e-12
+        assert tide._native.take_tm2d_launches()[WAVEFRONT] == 12 + 8
+    finally:
+        tide._native.set_tm2d_time_block(*before)

@@ -549,7 +549,9 @@ int forward_impl(Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_h
   const bool staged = (ey_stage && ey_stage->active()) || (curl_stage && curl_stage->active());
   // K-step launches (K = 3, 4) need K ring slots at once, more than a
   // host-staged ring holds: staged calls use two-step launches.
-  if (g_tuning.fwd_steps == 0 && !staged) {
+  if (g_tuning.fwd_steps == 0 && !staged &&
+      !wavefront_forward(sizeof(T), n_shots, p.g.numel, nt, ey_store && curl_store, fmt, step_ratio,
+                         (int)p.g.ca_b + (int)p.g.cb_b + (int)p.g.cq_b)) {
     int rc = forward_tiles(1, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r, src, rec,
                                  nt, start_t, step_ratio, ey_store, curl_store, fmt,
                                  store_step_bytes, stream, arena, arena_cap);
@@ -792,7 +794,9 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
   const bool staged = (ey_stage && ey_stage->active()) || (curl_stage && curl_stage->active());
   // K-step launches need K ring slots at once (see forward_impl)
   const bool per_shot = (gca && p.g.ca_b) || (gcb && p.g.cb_b);
-  if (g_tuning.adj_steps == 0 && !staged) {
+  if (g_tuning.adj_steps == 0 && !staged &&
+      !wavefront_adjoint(sizeof(T), n_shots, p.g.numel, nt, (gca != nullptr) + (gcb != nullptr),
+                         per_shot)) {
     int rc = backward_tiles(1, p, grad_r, l_ey, l_hx, l_hz, ml_ey_x, ml_ey_z, ml_hx_z,
                                   ml_hz_x, ey_store, curl_store, fmt, store_step_bytes, grad_f, gca,
                                   gcb, src, rec, nt, start_t, step_ratio, stream);

@@ -1,6 +1,6 @@
 // Which kernels a 2-D TM call runs on when no time block is set: workgroup
-// tiles (tm2d_tile.h), or, where those measured slower, the in-place kernels of
-// tm2d_highorder.hip (orders 4 to 8, Born).  Every family
+// tiles (tm2d_tile.h), or, where those measured slower, wavefront tiles (order 2)
+// or the in-place kernels of tm2d_highorder.hip (orders 4 to 8).  Every family
 // gives the same fields, receivers and snapshots bit for bit.  The figures are
 // us per step of whole calls, tiles / other, fp32 unless noted; cells are
 // padded cells of all shots.
@@ -8,10 +8,47 @@
 
 #include "tm2d_device.h"
 
+#include <cmath>
 #include <cstdint>
 
 namespace tide_hip {
 namespace tm2d {
+
+// Order-2 forward on two-step wavefront tiles: calls that store both snapshot
+// streams at full fp32 width in every step, between 4.5 million cells and what
+// leaves their two state buffers (24 bytes a cell, 4 more for each per-shot
+// coefficient) in the 256 MB last-level cache: 600 x 640 cells and 12 shots 24.8 /
+// 21.0; 768 x 800 and 12 39.0 / 32.9; 950 x 950 and 8 36.0 / 31.0; 441 x 942 and
+// 12 25.9 / 23.1.  Below and above tiles are as fast or faster (560 x 600 x 12
+// 18.6 / 19.3; 1065 x 1065 x 12 77 / 90), so are they with fewer than 6 shots
+// (1300 x 1300 x 4 26.8 / 27.6), with small grids, whose border tiles weigh more
+// (441 x 500 x 24 27.1 / 28.9), with BF16 or sampled snapshots, and where a run is
+// so short that the wavefront path's many allocations weigh.
+inline bool wavefront_forward(size_t elem, int64_t n_shots, int64_t numel, int64_t nt,
+                              bool both_streams, int fmt, int64_t step_ratio,
+                              int batched_coefficients) {
+  const int64_t cells = n_shots * numel;
+  return elem == 4 && both_streams && fmt == 1 && step_ratio == 1 && nt >= 64 && n_shots >= 6 &&
+         numel >= 250000 && cells >= 4500000 &&
+         cells * (24 + 4 * batched_coefficients) <= 200000000;
+}
+
+// Order-2 adjoint on three-step wavefront tiles: large fp32 calls whose shots
+// fill workgroups of four, which share one FP64 gradient slice (tiles hold one
+// per shot).  Per cell the tiles' time is the same at every size, the wavefront
+// tiles' falls with the share of border tiles: the line is cells x the grid's
+// side, for two gradients: 1065 x 1065 cells and 4 shots (4.8e9) 30.4 / 29.3; 1300
+// x 1300 x 4 43.1 / 38.5; 2081 x 2081 x 4, BF16 107 / 89; 768 x 800 x 12 52.8 /
+// 45.8; below it 441 x 942 x 12 (3.2e9) 34.3 / 37.8, 900 x 900 x 4 (2.9e9) 21.8 /
+// 21.9.  Groups of three shots and fewer gain 4 % at most (2081 x 2081 x 2 55.4 /
+// 53.4) and lose as much (1000 x 1000 x 6 38.4 / 41.5); per-shot gradients have no
+// shared slice (1000 x 1000 x 8 58 / 98).
+inline bool wavefront_adjoint(size_t elem, int64_t n_shots, int64_t numel, int64_t nt,
+                              int gradients, bool per_shot) {
+  const double weight = 0.5 * gradients * (double)n_shots * (double)numel * std::sqrt((double)numel);
+  return elem == 4 && !per_shot && nt >= 64 && balanced_group((int)n_shots, 4) == 4 &&
+         weight >= 4.4e9;
+}
 
 // Orders 4 to 8 in place.  Runs of few steps: a tile loop's set-up (a second
 // state, packed profiles) takes 0.1 ms, an in-place step 12 us and more (order 4,
