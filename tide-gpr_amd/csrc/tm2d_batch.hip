@@ -3,7 +3,7 @@
 // workgroup tiles (tm2d_tile.h): one launch advances every problem by up to 8
 // steps, each from its own argument record; all problems share one tile shape
 // and step count per pass, chosen for the whole batch.  As settings, and for
-// the adjoint of large batches: one launch per time step, or one per two
+// the adjoint of some large batches: one launch per time step, or one per two
 // time steps with the two-step kernels of tm2d_fused.h; a problem whose nt is
 // odd takes its last step in a one-step launch over its own tiles.
 //
@@ -837,7 +837,7 @@ int build_step_launches(Plan &p, const std::vector<BatchItem<float>> &proto, boo
   std::vector<int32_t> tiles2, tiles2a;
   if (two) PLAN_CHECK(build_items2(p, tiles2, tiles2a));
   // problems with several shot groups accumulate into per-group FP64 slices
-  for (size_t m = 0; m < p.probs.size(); ++m) {
+  for (size_t m = 0; m < p.probs.size() && !p.tiles_a; ++m) {
     BatchItem<float> &it = p.h_adj[m];
     it.group_stride = 0;
     if (it.n_groups > 1 && (it.gca || it.gcb)) {
@@ -870,6 +870,24 @@ int build_step_launches(Plan &p, const std::vector<BatchItem<float>> &proto, boo
   return kOk;
 }
 
+// Whether a batch's adjoint runs two steps per launch, not on tiles: where at
+// least half its cells are in grids of 150 000 cells and more whose shots fill
+// workgroups of four (which share a gradient slice; tiles hold one per shot), from
+// 5.5 million cells.  ms of a 96-step adjoint, tiles / two-step: 8 x 425 x 445
+// cells and 4 shots 5.4 / 4.9, 3 x 725 x 745 x 4 4.7 / 4.4; below and beside it 4 x
+// 545 x 565 x 4 3.5 / 3.7, 24 x 325 x 345 x 4 8.8 / 9.9, 12 x 425 x 445 x 3 6.4 /
+// 6.8, 60 x 245 x 265 x 3 11.6 / 15.2, 4 x 1325 x 1325 x 1 4.7 / 12.5.
+bool two_step_adjoint(const tide_tm2d_problem *problems, int64_t n) {
+  double cells = 0.0, shared = 0.0;
+  for (int64_t m = 0; m < n; ++m) {
+    const tide_tm2d_problem &q = problems[m];
+    const double numel = (double)q.ny * (double)q.nx, c = numel * (double)q.n_shots;
+    cells += c;
+    if (numel >= 150000 && q.n_shots > 0 && balanced_group((int)q.n_shots, 4) == 4) shared += c;
+  }
+  return cells >= 5.5e6 && 2.0 * shared >= cells;
+}
+
 int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t storage_format,
                int64_t use_graph, int64_t device, bool tiles) {
   p->device = (int)device;
@@ -878,23 +896,14 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
   p->rows_f = rows_for<float>(g_tuning.fwd_rows);
   p->rows_a = rows_for<float>(g_tuning.adj_rows);
   p->group = g_tuning.adj_group;  // one group size for both passes
-  // One- or two-step launches as set (a K-step setting runs at 2).  Where
-  // neither pass has a setting the forward runs on tiles, the adjoint up to
-  // kBatchTileCells padded cells.  fp32, us per step, tiles / two-step launches,
-  // forward with snapshots and adjoint: 24 grids of 81 x 101 cells (x 1 shot)
-  // 3.5 / 9.8 and 6.5 / 21; 12 of 241 x 261 x 3 11 / 19 and 21 / 34; 12 of 341 x
-  // 361 x 4 26 / 38 and 50 / 50; 8 of 541 x 561 x 4 49 / 64 and 81 / 78; 8 of
-  // 741 x 781 x 4 99 / 104 to 137 and 139 / 129.
-  constexpr int64_t kBatchTileCells = 7000000;
-  int64_t cells = 0;
-  for (int64_t m = 0; m < n; ++m)
-    cells += std::max<int64_t>(problems[m].n_shots, 0) * std::max<int64_t>(problems[m].ny, 0) *
-             std::max<int64_t>(problems[m].nx, 0);
-  p->tiles_f = tiles && g_tuning.fwd_steps == 0 && g_tuning.adj_steps == 0;
-  p->tiles_a = p->tiles_f && cells <= kBatchTileCells;
+  // Each pass runs on tiles unless a time block is set (one- or two-step
+  // launches; a K-step setting runs at 2), the adjoint of some large batches too.
+  p->tiles_f = tiles && g_tuning.fwd_steps == 0;
+  p->tiles_a = tiles && g_tuning.adj_steps == 0 && !two_step_adjoint(problems, n);
   p->steps_f = g_tuning.fwd_steps == 1 ? 1 : 2;
   p->steps_a = g_tuning.adj_steps == 1 ? 1 : 2;
-  const bool two = !p->tiles_a && (p->steps_f == 2 || p->steps_a == 2);
+  const bool steps = !p->tiles_f || !p->tiles_a;  // a pass runs on step launches
+  const bool two = (!p->tiles_f && p->steps_f == 2) || (!p->tiles_a && p->steps_a == 2);
   p->probs.assign(problems, problems + n);
   std::stable_sort(p->probs.begin(), p->probs.end(),
                    [](const tide_tm2d_problem &a, const tide_tm2d_problem &b) { return a.nt > b.nt; });
@@ -952,7 +961,7 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
     std::vector<int64_t> hs, hr;
     PLAN_CHECK(fetch_host(q.sources_i, q.n_shots * q.n_src, hs));
     PLAN_CHECK(fetch_host(q.receivers_i, q.n_shots * q.n_rec, hr));
-    if (!p->tiles_a) {
+    if (steps) {
       PointTable table;
       if (!build_point_table(hs.data(), q.n_src, hr.data(), q.n_rec, q.n_shots, q.ny, q.nx, kOwn,
                              1, table))
@@ -1023,11 +1032,9 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
   }
   p->fmt_fwd = any_store ? fmt : 0;
   p->fmt_adj = any_grad ? fmt : 0;
-  if (p->tiles_a) {
-    p->h_fwd = p->h_adj = proto;
-  } else {
-    PLAN_CHECK(build_step_launches(*p, proto, two));
-  }
+  p->h_fwd = p->h_adj = proto;
+  if (steps) PLAN_CHECK(build_step_launches(*p, proto, two));
+  if (p->tiles_a) p->h_adj = proto;
   if (p->tiles_f) PLAN_CHECK(build_tiles_forward(*p));
   if (p->tiles_a && p->probs[0].lambda[0] != nullptr) PLAN_CHECK(build_tiles_backward(*p));
   TIDE_HIP_TRY(hipDeviceSynchronize());
