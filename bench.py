@@ -677,12 +677,9 @@ def main() -> None:
     sizes = plan.sizes
     tuning = None
     if not args.no_autotune:
-        from tide.autotune import (ADJ_AUTOMATIC, ADJ_CANDIDATES, FWD_AUTOMATIC, FWD_CANDIDATES,
-                                   tune_tm2d)
+        from tide.autotune import tune_tm2d
 
-        t = tune_tm2d(ny_p, nx_p, sizes, device=dev, max_store_bytes=64 << 30,
-                      fwd_candidates=(FWD_AUTOMATIC, *FWD_CANDIDATES),
-                      adj_candidates=(ADJ_AUTOMATIC, *ADJ_CANDIDATES))
+        t = tune_tm2d(ny_p, nx_p, sizes, device=dev, max_store_bytes=64 << 30)
         log(f"autotuned on chunks {sizes}: forward {t['forward']} adjoint {t['adjoint']} "
             f"{t['chosen_us_per_step']} us per step (tuned in {t.get('seconds', 0)} s)")
         tuning = t

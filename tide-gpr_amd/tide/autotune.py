@@ -8,7 +8,8 @@ launch parameters:
   shots and summing the FP64 gradient in LDS; the shot-loop family gives
   each wavefront one tile and walks every shot of the call (G is then tiles
   per workgroup);
-* time steps per launch: 1, 2 (two-step kernels that recompute a halo of
+* time steps per launch: 0 (the library's own choice by size, workgroup
+  tiles mostly; the default), 1, 2 (two-step kernels that recompute a halo of
   two and touch the wavefield state once per two steps, the interior and
   border tiles as one kernel or two) or K = 3, 4 (a halo of K, border
   tiles first in one kernel; host-staged snapshots run at 2);
@@ -34,25 +35,24 @@ from .maxwell.tm2d import prepare_tm2d
 from .utils import C0
 
 # (rows, group, shot loop, steps per launch, interior/border split,
-#  border tile rows)
+#  border tile rows); 0 steps per launch (the library's default): it picks the
+# kernels and their steps from the problem
+FWD_AUTOMATIC = (4, 1, 0, 0, 0, 0)
+ADJ_AUTOMATIC = (4, 4, 0, 0, 0, 2)
 FWD_CANDIDATES: tuple[tuple[int, int, int, int, int, int], ...] = (
+    FWD_AUTOMATIC,
     (2, 4, 0, 1, 0, 0), (4, 2, 0, 1, 0, 0), (4, 4, 0, 1, 0, 0), (8, 4, 0, 1, 0, 0),
     (16, 4, 0, 1, 0, 0), (2, 4, 1, 1, 0, 0), (4, 2, 1, 1, 0, 0),
     (2, 2, 0, 2, 0, 0), (4, 1, 0, 2, 0, 0), (4, 2, 0, 2, 0, 0), (4, 4, 0, 2, 0, 0),
     (8, 2, 0, 2, 0, 0), (4, 1, 0, 2, 0, 2), (4, 2, 0, 2, 0, 2),
     (4, 1, 0, 2, 1, 0), (4, 2, 0, 2, 1, 0), (4, 2, 0, 3, 0, 0), (8, 2, 0, 3, 0, 0))
 ADJ_CANDIDATES: tuple[tuple[int, int, int, int, int, int], ...] = (
+    ADJ_AUTOMATIC,
     (2, 2, 0, 1, 0, 0), (2, 4, 0, 1, 0, 0), (2, 8, 0, 1, 0, 0), (4, 4, 0, 1, 0, 0),
     (8, 2, 0, 1, 0, 0), (2, 4, 1, 1, 0, 0), (4, 2, 1, 1, 0, 0),
     (4, 4, 0, 2, 1, 0), (4, 8, 0, 2, 1, 0), (4, 4, 0, 2, 1, 2), (4, 8, 0, 2, 1, 2),
     (2, 4, 0, 2, 0, 0), (4, 2, 0, 2, 0, 0), (4, 4, 0, 2, 0, 0), (4, 8, 0, 2, 0, 0),
     (4, 4, 0, 2, 0, 2), (4, 8, 0, 2, 0, 2), (4, 4, 0, 3, 0, 2), (4, 2, 0, 3, 0, 2))
-
-# 0 steps per launch (the library's default): it picks workgroup or wavefront
-# tiles and their steps from the problem.  Add these to the lists to time
-# them against the fixed shapes.
-FWD_AUTOMATIC = (4, 1, 0, 0, 0, 0)
-ADJ_AUTOMATIC = (4, 4, 0, 0, 0, 2)
 
 _cache: dict[tuple, tuple[tuple[int, ...], tuple[int, ...]]] = {}
 
@@ -250,6 +250,8 @@ def tune_tm2d(
     _cache[key] = (best_f, best_a)
 
     def label(k):
+        if k[3] == 0:
+            return "automatic"
         return (f"{k[0]}x{k[1]}{'L' if k[2] else ''}{f'/{k[3]}' if k[3] > 1 else ''}"
                 f"{'s' if k[4] else ''}{f'b{k[5]}' if k[5] else ''}")
 
