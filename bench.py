@@ -752,7 +752,7 @@ def main() -> None:
         kname = f"{stem}_step" if spl == 1 else (f"{stem}2_step" if spl == 2 else f"{stem}k_step")
         if stem == "adj" and spl >= 3 and adj_w4:
             kname = "adjk_step_w4"
-        if spl > 4:
+        if d["family"] == "tiles":
             kname = f"tile_{stem}"
         kernels[name] = {
             "kernel": kname,

@@ -1250,12 +1250,12 @@ int tide_tm2d_set_time_block(int fwd_steps, int adj_steps);
 int tide_tm2d_get_time_block(int *out2);
 
 /*
- * What the 2-D forward, adjoint and Born-forward calls of the calling thread
- * have enqueued since it last asked: launches on workgroup tiles, launches on
- * wavefront tiles, and time steps taken in place (several launches each).
- * No reference counterpart.
+ * What the 2-D calls of the calling thread have enqueued since it last asked,
+ * per pass (0 forward and Born forward, 1 adjoint): launches on workgroup
+ * tiles, launches on wavefront tiles, and time steps taken in place (several
+ * launches each).  No reference counterpart.
  */
-int tide_tm2d_take_launches(int64_t *out3);
+int tide_tm2d_take_launches(int pass, int64_t *out3);
 
 /*
  * Scratch of the workgroup-tile loops, as settings of the calling thread.

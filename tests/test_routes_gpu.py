@@ -43,38 +43,39 @@ def _operator(ny, nx, shots, nt, stencil, dtype, compression=False, pml=8):
     return op, model, torch.zeros(nt, shots, rec.shape[1], device=dev, dtype=dtype)
 
 
-def _family(fn):
-    tide._native.take_tm2d_launches()
+def _families(fn):
+    """Kernel families of the forward and of the adjoint that fn() runs."""
+    for p in (0, 1):
+        tide._native.take_tm2d_launches(p)
     fn()
-    counts = tide._native.take_tm2d_launches()
-    return {k for k, n in enumerate(counts) if n}
+    return [{k for k, n in enumerate(tide._native.take_tm2d_launches(p)) if n} for p in (0, 1)]
 
 
-@pytest.mark.parametrize("case,forward,gradient", [
-    # forward alone; forward with snapshots and adjoint of one gradient
-    (dict(ny=96, nx=96, shots=1, nt=64), {TILES}, {TILES}),
-    (dict(ny=1065, nx=1065, shots=4, nt=64), {TILES}, {TILES, WAVEFRONT}),
-    (dict(ny=1065, nx=1065, shots=4, nt=64, compression=True), {TILES}, {TILES, WAVEFRONT}),
-    (dict(ny=1065, nx=1065, shots=4, nt=24), {TILES}, {TILES}),
-    (dict(ny=1065, nx=1065, shots=3, nt=64), {TILES}, {TILES}),
-    (dict(ny=768, nx=800, shots=12, nt=64), {TILES}, {WAVEFRONT}),
-    (dict(ny=441, nx=942, shots=12, nt=64), {TILES}, {TILES, WAVEFRONT}),
-    (dict(ny=441, nx=942, shots=12, nt=64, compression=True), {TILES}, {TILES}),
-    (dict(ny=700, nx=700, shots=4, nt=64, dtype=torch.float64), {TILES}, {TILES}),
-    (dict(ny=96, nx=96, shots=2, nt=7, stencil=4), {IN_PLACE}, {IN_PLACE, TILES}),
-    (dict(ny=96, nx=96, shots=2, nt=3, stencil=6), {IN_PLACE}, {IN_PLACE}),
-    (dict(ny=96, nx=96, shots=2, nt=8, stencil=8), {TILES}, {TILES}),
-    (dict(ny=400, nx=400, shots=4, nt=16, stencil=8, dtype=torch.float64), {IN_PLACE},
-     {IN_PLACE, TILES}),
-    (dict(ny=400, nx=400, shots=4, nt=16, stencil=6, dtype=torch.float64), {TILES}, {TILES}),
+@pytest.mark.parametrize("case,forward,storing,adjoint", [
+    (dict(ny=96, nx=96, shots=1, nt=64), TILES, TILES, TILES),
+    (dict(ny=1065, nx=1065, shots=4, nt=64), TILES, TILES, WAVEFRONT),
+    (dict(ny=1065, nx=1065, shots=4, nt=64, compression=True), TILES, TILES, WAVEFRONT),
+    (dict(ny=1065, nx=1065, shots=4, nt=24), TILES, TILES, TILES),
+    (dict(ny=1065, nx=1065, shots=3, nt=64), TILES, TILES, TILES),
+    (dict(ny=768, nx=800, shots=12, nt=64), TILES, WAVEFRONT, WAVEFRONT),
+    (dict(ny=441, nx=942, shots=12, nt=64), TILES, WAVEFRONT, TILES),
+    (dict(ny=441, nx=942, shots=12, nt=64, compression=True), TILES, TILES, TILES),
+    (dict(ny=700, nx=700, shots=4, nt=64, dtype=torch.float64), TILES, TILES, TILES),
+    (dict(ny=96, nx=96, shots=2, nt=7, stencil=4), IN_PLACE, IN_PLACE, TILES),
+    (dict(ny=96, nx=96, shots=2, nt=3, stencil=6), IN_PLACE, IN_PLACE, IN_PLACE),
+    (dict(ny=96, nx=96, shots=2, nt=8, stencil=8), TILES, TILES, TILES),
+    (dict(ny=400, nx=400, shots=4, nt=16, stencil=8, dtype=torch.float64), IN_PLACE,
+     IN_PLACE, TILES),
+    (dict(ny=400, nx=400, shots=4, nt=16, stencil=6, dtype=torch.float64), TILES, TILES, TILES),
 ])
-def test_calls_run_on_the_kernels_that_measured_faster(case, forward, gradient):
+def test_calls_run_on_the_kernels_that_measured_faster(case, forward, storing, adjoint):
     print(case, flush=True)
     case = dict(dict(stencil=2, dtype=torch.float32), **case)
     op, model, observed = _operator(**case)
-    assert _family(lambda: op(model)) == forward
+    assert _families(lambda: op(model)) == [{forward}, set()]
     objective = ReceiverObjective(observed)
-    assert _family(lambda: objective.value_and_gradient(op.linearize(model))) == gradient
+    assert (_families(lambda: objective.value_and_gradient(op.linearize(model)))
+            == [{storing}, {adjoint}])
 
 
 @pytest.mark.parametrize("case,family", [
@@ -90,7 +91,7 @@ def test_jacobian_products_run_on_the_kernels_that_measured_faster(case, family)
     direction = tide.EMDirection(epsilon=torch.ones_like(model.epsilon),
                                  sigma=torch.zeros_like(model.sigma))
     with op.linearize(model) as lin:
-        assert _family(lambda: lin.jvp(direction)) == {family}
+        assert _families(lambda: lin.jvp(direction)) == [{family}, set()]
 
 
 @pytest.mark.parametrize("store,interval,batched,one", [
@@ -103,7 +104,8 @@ def test_wavefront_tiles_match_the_oracle(store, interval, batched, one, ny, nx,
     before = tide._native.get_tm2d_time_block()
     tide._native.set_tm2d_time_block(2, 3)
     try:
-        tide._native.take_tm2d_launches()
+        for p in (0, 1):
+            tide._native.take_tm2d_launches(p)
         f_o, r_o, es, cs = O.tm2d_forward(case, store=store, interval=interval)
         f_g, r_g, es_g, cs_g = gpu_forward(case, store=store, interval=interval)
         assert np.array_equal(r_g, r_o)
@@ -117,6 +119,29 @@ def test_wavefront_tiles_match_the_oracle(store, interval, batched, one, ny, nx,
         assert all(np.array_equal(a.reshape(b.shape), b) for a, b in zip(lam, lam_o))
         assert np.array_equal(gf, gf_o) and relative_l2(ga, ga_o) < 1e-12
         assert one or relative_l2(gb, gb_o) < 1e-12
-        assert tide._native.take_tm2d_launches()[WAVEFRONT] == 12 + 8
+        assert [tide._native.take_tm2d_launches(p)[WAVEFRONT] for p in (0, 1)] == [12, 8]
     finally:
+        tide._native.set_tm2d_time_block(*before)
+
+
+def test_the_kernel_timer_counts_the_launches_made():
+    from tide.maxwell.tm2d import KernelTimer, set_kernel_timer
+
+    op, model, observed = _operator(ny=96, nx=96, shots=2, nt=64, stencil=2, dtype=torch.float32)
+    before = tide._native.get_tm2d_time_block()
+    try:
+        for block, family, launches in ((0, "tiles", (8, 8)), (2, "wavefront", (32, 32)),
+                                        (3, "wavefront", (22, 22))):
+            tide._native.set_tm2d_time_block(block, block)
+            timer = KernelTimer()
+            set_kernel_timer(timer)
+            ReceiverObjective(observed).value_and_gradient(op.linearize(model))
+            torch.cuda.synchronize()
+            summary = timer.summary()
+            for name, n in zip(("forward_store", "adjoint"), launches):
+                assert summary[name]["launches"] == n and summary[name]["steps"] == 64
+                assert summary[name]["steps_per_launch"] == round(64 / n)
+                assert summary[name]["family"] == family
+    finally:
+        set_kernel_timer(None)
         tide._native.set_tm2d_time_block(*before)

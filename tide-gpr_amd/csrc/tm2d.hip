@@ -91,10 +91,11 @@ struct LoopTimer {
   }
 };
 
-// What the calling thread's time loops have enqueued: launches on workgroup
-// tiles, launches on wavefront tiles, steps taken in place.
+// What the calling thread's time loops have enqueued per pass (0 forward, Born
+// too, 1 adjoint): launches on workgroup tiles, launches on wavefront tiles,
+// steps taken in place.
 enum { kTileLaunches = 0, kWavefrontLaunches, kInPlaceSteps };
-thread_local int64_t loop_counts[3] = {0, 0, 0};
+thread_local int64_t loop_counts[2][3] = {{0, 0, 0}, {0, 0, 0}};
 
 constexpr int kMaxLoopTiles = 4;  // wavefronts per workgroup of the shot-looping kernels
 
@@ -402,7 +403,7 @@ int forward_tiles(int half, Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_e
     t += a.steps;
   }
   timer.finish(loop.launches);
-  loop_counts[kTileLaunches] += loop.launches;
+  loop_counts[0][kTileLaunches] += loop.launches;
   TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
   return kOk;
@@ -467,7 +468,7 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
     t -= a.steps;
   }
   timer.finish(loop.launches);
-  loop_counts[kTileLaunches] += loop.launches;
+  loop_counts[1][kTileLaunches] += loop.launches;
   TIDE_CHECK(launched());
   const unsigned fold_blocks = (unsigned)((numel + 255) / 256);
   for (int k = 0; k < 2; ++k)
@@ -522,7 +523,7 @@ int born_tiles(int half, Problem<T> p, T *const bg[7], T *const sc[7], const T *
     launch_tile_born<T>(half, plan, hist != nullptr, stream, a);
     t += a.steps;
   }
-  loop_counts[kTileLaunches] += loop.launches;
+  loop_counts[0][kTileLaunches] += loop.launches;
   TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
   return kOk;
@@ -741,7 +742,7 @@ int forward_impl(Problem<T> p, T *ey, T *hx, T *hz, T *m_ey_x, T *m_ey_z, T *m_h
     for (int k = 0; k < 5; ++k) std::swap(cur[k], nxt[k]);
   }
   timer.finish(launches);
-  loop_counts[kWavefrontLaunches] += launches;
+  loop_counts[0][kWavefrontLaunches] += launches;
   TIDE_HIP_TRY(hipGetLastError());
   if (cur[0] != ey) {
     TIDE_HIP_TRY(hipMemcpyAsync(ey, cur[0], bytes, hipMemcpyDeviceToDevice, stream));
@@ -1001,7 +1002,7 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
     for (int k = 0; k < 7; ++k) std::swap(cur[k], nxt[k]);
   }
   timer.finish(launches);
-  loop_counts[kWavefrontLaunches] += launches;
+  loop_counts[1][kWavefrontLaunches] += launches;
   TIDE_HIP_TRY(hipGetLastError());
   const unsigned fold_blocks = (unsigned)((numel + 255) / 256);
   if (gacc) fold_groups<<<fold_blocks, 256, 0, stream>>>(gca, gacc, numel, (int)n_groups);
@@ -1208,7 +1209,7 @@ int forward_entry(T const *ca, T const *cb, T const *cq, T const *f, T *ey, T *h
       rc = tm2d_ho::forward<T>(stencil, hp, fld, f, r, sources_i, receivers_i, nt, start_t,
                                step_ratio, ey_store, curl_store, fmt, store_step_bytes, stream,
                                &ey_st, &curl_st);
-      if (rc == kOk) loop_counts[kInPlaceSteps] += nt;
+      if (rc == kOk) loop_counts[0][kInPlaceSteps] += nt;
     }
   }
   return close_stages(rc, ey_st, curl_st);
@@ -1311,7 +1312,7 @@ int backward_entry(T const *ca, T const *cb, T const *cq, T const *grad_r, T *la
                                 step_bytes, grad_f, ca_rg ? ga : nullptr, cb_rg ? gb : nullptr,
                                 sources_i, receivers_i, nt, start_t, step_ratio, stream, &ey_st,
                                 &curl_st);
-      if (rc == kOk) loop_counts[kInPlaceSteps] += nt;
+      if (rc == kOk) loop_counts[1][kInPlaceSteps] += nt;
     }
   }
   TIDE_CHECK(close_stages(rc, ey_st, curl_st));
@@ -1344,7 +1345,7 @@ int born_entry(int stencil, const tm2d_ho::Problem<T> &hp, T *const bg[7], T *co
   }
   const int rc = tm2d_ho::born_forward<T>(stencil, hp, bg, sc, dca, dcb, f0, df, r, bg_r, src, rec,
                                           nt, start_t, stream, hist);
-  if (rc == kOk) loop_counts[kInPlaceSteps] += nt;
+  if (rc == kOk) loop_counts[0][kInPlaceSteps] += nt;
   return rc;
 }
 
@@ -1841,14 +1842,14 @@ extern "C" int tide_tm2d_get_adjoint_waves(int *out) {
   return kOk;
 }
 
-extern "C" int tide_tm2d_take_launches(int64_t *out3) {
-  if (out3 == nullptr) {
-    set_error("take_launches: output required");
+extern "C" int tide_tm2d_take_launches(int pass, int64_t *out3) {
+  if (out3 == nullptr || pass < 0 || pass > 1) {
+    set_error("take_launches: pass must be 0 or 1, with an output");
     return kInvalidArgument;
   }
   for (int k = 0; k < 3; ++k) {
-    out3[k] = loop_counts[k];
-    loop_counts[k] = 0;
+    out3[k] = loop_counts[pass][k];
+    loop_counts[pass][k] = 0;
   }
   return kOk;
 }

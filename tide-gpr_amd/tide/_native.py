@@ -318,7 +318,7 @@ def load() -> ctypes.CDLL:
     lib.tide_tm2d_get_time_block.restype = ctypes.c_int
     lib.tide_tm2d_get_time_block.argtypes = [ctypes.POINTER(ctypes.c_int)]
     lib.tide_tm2d_take_launches.restype = ctypes.c_int
-    lib.tide_tm2d_take_launches.argtypes = [ctypes.POINTER(ctypes.c_int64)]
+    lib.tide_tm2d_take_launches.argtypes = [ctypes.c_int, ctypes.POINTER(ctypes.c_int64)]
     lib.tide_tm2d_set_tile_fallback.restype = ctypes.c_int
     lib.tide_tm2d_set_tile_fallback.argtypes = [ctypes.c_int]
     lib.tide_tm2d_set_tile_scratch_limit.restype = ctypes.c_int
@@ -488,11 +488,12 @@ def set_tm2d_time_block(fwd_steps: int, adj_steps: int) -> None:
     check(load().tide_tm2d_set_time_block(int(fwd_steps), int(adj_steps)))
 
 
-def take_tm2d_launches() -> tuple[int, int, int]:
+def take_tm2d_launches(pass_index: int) -> tuple[int, int, int]:
     """Launches on workgroup tiles and on wavefront tiles, and steps taken in
-    place, of this thread's 2-D calls since it last asked."""
+    place, of this thread's 2-D calls since it last asked (pass 0: forward and
+    Born forward, 1: adjoint)."""
     out = (ctypes.c_int64 * 3)()
-    check(load().tide_tm2d_take_launches(out))
+    check(load().tide_tm2d_take_launches(pass_index, out))
     return int(out[0]), int(out[1]), int(out[2])
 
 

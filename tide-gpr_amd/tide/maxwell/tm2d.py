@@ -64,35 +64,53 @@ class KernelTimer:
 
     When installed with :func:`set_kernel_timer`, every forward and adjoint
     sweep is bracketed by events on the stream the kernels run on, and the
-    record ``(pass, n_steps, cells_per_step, start, end)`` is kept so a
+    record ``(pass, n_steps, cells_per_step, launches, start, end)`` is kept so a
     caller can derive per-launch kernel durations without a profiler.
+    ``launches`` counts per kernel family, see :data:`FAMILIES`.
     """
 
+    # workgroup tiles, wavefront tiles, in place (a step counts as a launch)
+    FAMILIES = ("tiles", "wavefront", "in_place")
+
     def __init__(self) -> None:
-        self.records: list[tuple[str, int, int, int, torch.cuda.Event, torch.cuda.Event]] = []
+        self.records: list[tuple[str, int, int, tuple[int, int, int], torch.cuda.Event,
+                                 torch.cuda.Event]] = []
 
     def start(self) -> torch.cuda.Event:
+        for p in (0, 1):
+            _native.take_tm2d_launches(p)
         ev = torch.cuda.Event(enable_timing=True)
         ev.record()
         return ev
 
     def stop(self, name: str, steps: int, cells: int, start: torch.cuda.Event,
              steps_per_launch: int = 1) -> None:
+        """Ends a sweep of ``steps`` steps.  ``steps_per_launch`` is used where
+        no launches were counted since :meth:`start`."""
         ev = torch.cuda.Event(enable_timing=True)
         ev.record()
-        self.records.append((name, steps, cells, max(1, steps_per_launch), start, ev))
+        launches = _native.take_tm2d_launches(1 if name == "adjoint" else 0)
+        if not any(launches):
+            launches = (0, -(-steps // max(1, steps_per_launch)), 0)
+        self.records.append((name, steps, cells, launches, start, ev))
 
-    def summary(self) -> dict[str, dict[str, float]]:
-        """Per pass: total ms, launches (time steps / steps per launch), time
-        steps, and cell-updates (after a sync)."""
-        out: dict[str, dict[str, float]] = {}
-        for name, steps, cells, spl, a, b in self.records:
-            d = out.setdefault(name, {"ms": 0.0, "launches": 0, "steps": 0, "cell_updates": 0.0,
-                                      "steps_per_launch": spl})
+    def summary(self) -> dict[str, dict[str, Any]]:
+        """Per pass: total ms, launches, time steps, steps per launch, kernel
+        family with the most launches, and cell-updates (after a sync)."""
+        out: dict[str, dict[str, Any]] = {}
+        families: dict[str, list[int]] = {}
+        for name, steps, cells, launches, a, b in self.records:
+            d = out.setdefault(name, {"ms": 0.0, "launches": 0, "steps": 0, "cell_updates": 0.0})
+            f = families.setdefault(name, [0, 0, 0])
+            for k, n in enumerate(launches):
+                f[k] += n
             d["ms"] += a.elapsed_time(b)
-            d["launches"] += (steps + spl - 1) // spl
+            d["launches"] += sum(launches)
             d["steps"] += steps
             d["cell_updates"] += float(steps) * cells
+        for name, d in out.items():
+            d["steps_per_launch"] = max(1, round(d["steps"] / max(1, d["launches"])))
+            d["family"] = self.FAMILIES[max(range(3), key=families[name].__getitem__)]
         return out
 
 
