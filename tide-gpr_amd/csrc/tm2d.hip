@@ -422,16 +422,13 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
   StatePair<T, 7> state({l_ey, l_hx, l_hz, ml_hz_x, ml_hx_z, ml_ey_x, ml_ey_z}, (size_t)total);
   TileAdjArgs<T> a;
   std::memset(&a, 0, sizeof(a));
-  a.per_shot_grad = ((gca && p.g.ca_b) || (gcb && p.g.cb_b)) ? 1 : 0;
-  // Several shot groups: each accumulates into its own FP64 slice, folded
-  // into gca / gcb in group order at the end (no atomics, repeatable).
-  const int64_t n_groups = (n_shots + plan.group - 1) / plan.group;
+  // Gradients summed over shots: each shot accumulates into its own FP64 slice,
+  // folded into gca / gcb in shot order at the end (no atomics, repeatable).
   double *acc[2] = {nullptr, nullptr}, *const grad[2] = {gca, gcb};
-  const bool sliced = n_groups > 1 && !a.per_shot_grad;
-  if (sliced) a.group_stride = numel;
+  const bool sliced = n_shots > 1 && !((gca && p.g.ca_b) || (gcb && p.g.cb_b));
   DevicePointTable dpt;
   const int rc = open_tiles(p, plan, src, rec, loop, scr, state, dpt, stream,
-                            (size_t)(n_groups * numel), sliced && gca ? &acc[0] : nullptr,
+                            (size_t)total, sliced && gca ? &acc[0] : nullptr,
                             sliced && gcb ? &acc[1] : nullptr);
   if (rc != kOk) return no_room(rc, scr);
   a.g = p.g;
@@ -444,7 +441,6 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
   a.halo = plan.halo;
   a.own_rows = plan.own_rows;
   a.order = tile_order(plan, p.g, half);
-  a.group = plan.group;
   a.r_stride = n_shots * p.n_rec;
   a.f_stride = n_shots * p.n_src;
   LoopTimer timer(1, stream);
@@ -472,7 +468,7 @@ int backward_tiles(int half, Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T 
   TIDE_CHECK(launched());
   const unsigned fold_blocks = (unsigned)((numel + 255) / 256);
   for (int k = 0; k < 2; ++k)
-    if (acc[k]) fold_groups<<<fold_blocks, 256, 0, stream>>>(grad[k], acc[k], numel, (int)n_groups);
+    if (acc[k]) fold_groups<<<fold_blocks, 256, 0, stream>>>(grad[k], acc[k], numel, (int)n_shots);
   TIDE_CHECK(launched());
   TIDE_CHECK(state.close(stream));
   return kOk;

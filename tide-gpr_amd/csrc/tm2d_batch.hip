@@ -590,7 +590,7 @@ int build_items2(Plan &p, std::vector<int32_t> &tile_item, std::vector<int32_t> 
 std::vector<int64_t> tile_grids(const Plan &p, const TilePlan &t) {
   std::vector<int64_t> grid;
   for (const tide_tm2d_problem &q : p.probs) {
-    const TilePlan one = make_tile_plan(1, (int)q.ny, (int)q.nx, t.waves, t.rows, t.steps, 1);
+    const TilePlan one = make_tile_plan(1, (int)q.ny, (int)q.nx, t.waves, t.rows, t.steps);
     const int64_t n = (int64_t)one.n_xt * one.n_yt * q.n_shots, l = LaunchSteps(q.nt, t.steps).launches;
     if ((int64_t)grid.size() < l) grid.resize((size_t)l, 0);
     for (int64_t k = 0; k < l; ++k) grid[(size_t)k] += n;
@@ -605,7 +605,7 @@ TilePlan plan_batch_tiles(const Plan &p, bool adjoint, bool storing) {
   double best_us = 1e300;
   for (int rows = 2; rows <= 4; rows += 2) {
     for (int steps = 1; steps <= kTileSteps; ++steps) {
-      const TilePlan t = make_tile_plan(1, 1, 1, kTileWaves, rows, steps, 1);
+      const TilePlan t = make_tile_plan(1, 1, 1, kTileWaves, rows, steps);
       double us = 0.0;
       for (int64_t n : tile_grids(p, t)) {
         const double r = (double)n / 256.0;
@@ -640,7 +640,7 @@ int upload_pass(Plan &p, TilePass<A> &t, const std::vector<A> &table,
 int tile_problem(Plan &p, size_t m, const TilePlan &t, TilePlan &one, Points &pts,
                  std::vector<int32_t> &tile_item) {
   const tide_tm2d_problem &q = p.probs[m];
-  one = make_tile_plan(1, (int)q.ny, (int)q.nx, t.waves, t.rows, t.steps, 1);
+  one = make_tile_plan(1, (int)q.ny, (int)q.nx, t.waves, t.rows, t.steps);
   std::vector<int64_t> hs, hr;
   PLAN_CHECK(fetch_host(q.sources_i, q.n_shots * q.n_src, hs));
   PLAN_CHECK(fetch_host(q.receivers_i, q.n_shots * q.n_rec, hr));
@@ -742,13 +742,12 @@ int build_tiles_backward(Plan &p) {
     a.halo = one.halo;
     a.own_rows = one.own_rows;
     a.order = tile_order(one, it.g, 1);
-    a.group = 1;
     a.r_stride = q.n_shots * q.n_rec;
     a.f_stride = q.n_shots * q.n_src;
     // one FP64 slice per shot, folded in shot order after the loop
     it.n_groups = a.n_shots;
     if (q.n_shots > 1 && (q.grad_ca || q.grad_cb)) {
-      it.group_stride = a.group_stride = numel;
+      it.group_stride = numel;
       if (q.grad_ca) PLAN_CHECK(tile_alloc(p, &it.gca, (size_t)total));
       if (q.grad_cb) PLAN_CHECK(tile_alloc(p, &it.gcb, (size_t)total));
     }

@@ -105,12 +105,10 @@ template <typename T> struct TileAdjArgs {
   T *grad_f;        // source-term gradients of that step (null: not wanted)
   int64_t r_stride, f_stride;
   const void *ey_store[kTileSteps], *curl_store[kTileSteps];  // null: no term
-  double *gca, *gcb;  // FP64 accumulators; null: not wanted
-  int32_t per_shot_grad;
+  double *gca, *gcb;  // FP64 accumulators, one plane per shot; null: not wanted
   double step_scale;
-  int32_t n_shots, steps, halo, own_rows, group, tile0;
+  int32_t n_shots, steps, halo, own_rows, tile0;
   TileOrder order;
-  int64_t group_stride;  // shot group k adds into gca / gcb + k * group_stride
 };
 
 // A kernel's arguments, read anew at each call: the compiler loads every
@@ -909,7 +907,7 @@ __global__ __launch_bounds__(64 * W) void tile_born(TileBornArgs<T>) {
 // memories; dHx/dz carries the negated term, so that its differences swap
 // their operands instead of negating (bit-identical).
 template <typename T, int P, int R, int FMT, bool EDGE>
-__device__ __forceinline__ void tile_adjoint(ArgRef<TileAdjArgs<T>> args, const TilePlace &c, int s0, int s1, int group,
+__device__ __forceinline__ void tile_adjoint(ArgRef<TileAdjArgs<T>> args, const TilePlace &c, int s,
                                              const TileRows<T, P> &lds) {
   using Args = TileAdjArgs<T>;
   constexpr int HS = 2 * P - 1;
@@ -917,7 +915,7 @@ __device__ __forceinline__ void tile_adjoint(ArgRef<TileAdjArgs<T>> args, const 
   const Geom<T> &g = a.g;
   const T rdy = g.rdy, rdx = g.rdx;
   const int steps = a.steps;
-  const int64_t numel = g.numel;
+  const int64_t base = (int64_t)s * g.numel;
   const int ny = g.ny, nx = g.nx, x = c.x;
   const int halo = a.halo;
   const bool own = c.lane >= halo && c.lane < 64 - halo && x < nx;
@@ -947,205 +945,193 @@ __device__ __forceinline__ void tile_adjoint(ArgRef<TileAdjArgs<T>> args, const 
 #pragma unroll
   for (int r = 0; r < R; ++r) ga[r] = gb[r] = 0.0;
 
-  for (int s = s0; s < s1; ++s) {
-    const int64_t base = (int64_t)s * numel;
-    const Args &a = args();
-    const Geom<T> &g = a.g;
-    T ley[R], lhx[R], lhz[R], ca[R], cb[R], cq[R];
-    load_rows<T, R>(ley, as_global(a.in[0]) + base, at);
-    load_rows<T, R>(cb, as_global(a.cb) + (g.cb_b ? base : 0), at);
-    load_rows<T, R>(lhx, as_global(a.in[1]) + base, at);
-    load_rows<T, R>(lhz, as_global(a.in[2]) + base, at);
-    load_rows<T, R>(cq, as_global(a.cq) + (g.cq_b ? base : 0), at);
-    load_rows<T, R>(ca, as_global(a.ca) + (g.ca_b ? base : 0), at);
-    T mx[R], my[R], nxm[R], nz[R];
-    if constexpr (EDGE) {
+  T ley[R], lhx[R], lhz[R], ca[R], cb[R], cq[R];
+  load_rows<T, R>(ley, as_global(a.in[0]) + base, at);
+  load_rows<T, R>(cb, as_global(a.cb) + (g.cb_b ? base : 0), at);
+  load_rows<T, R>(lhx, as_global(a.in[1]) + base, at);
+  load_rows<T, R>(lhz, as_global(a.in[2]) + base, at);
+  load_rows<T, R>(cq, as_global(a.cq) + (g.cq_b ? base : 0), at);
+  load_rows<T, R>(ca, as_global(a.ca) + (g.ca_b ? base : 0), at);
+  T mx[R], my[R], nxm[R], nz[R];
+  if constexpr (EDGE) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) mx[r] = my[r] = nxm[r] = nz[r] = (T)0;
-      if (any_x) {
-        load_rows<T, R>(mx, as_global(a.in[3]) + base, at);
-        load_rows<T, R>(nxm, as_global(a.in[5]) + base, at);
-      }
-      if ((rows.pe | rows.ph) != 0) {
-        load_rows<T, R>(my, as_global(a.in[4]) + base, at);
-        load_rows<T, R>(nz, as_global(a.in[6]) + base, at);
-      }
+    for (int r = 0; r < R; ++r) mx[r] = my[r] = nxm[r] = nz[r] = (T)0;
+    if (any_x) {
+      load_rows<T, R>(mx, as_global(a.in[3]) + base, at);
+      load_rows<T, R>(nxm, as_global(a.in[5]) + base, at);
     }
-    TilePoints<T, R> points;
-    points.load(a.pts, c, g.ny, a.n_shots, s, lds.entries);
-    points.amplitudes(lds.amp, c, steps, 1, a.grad_r, -a.r_stride);
-    wait_loads();
+    if ((rows.pe | rows.ph) != 0) {
+      load_rows<T, R>(my, as_global(a.in[4]) + base, at);
+      load_rows<T, R>(nz, as_global(a.in[6]) + base, at);
+    }
+  }
+  TilePoints<T, R> points;
+  points.load(a.pts, c, g.ny, a.n_shots, s, lds.entries);
+  points.amplitudes(lds.amp, c, steps, 1, a.grad_r, -a.r_stride);
+  wait_loads();
 
-    for (int j = 0; j < steps; ++j) {
-      const int lo = halo - (steps - 1 - j) * HS, hi = c.rows - lo;
-      const bool active = c.row0 < hi + P - 1 && c.row0 + R > lo - P;  // uniform
-      const RowBits b = rows.again();
-      // this step's snapshots, read well before the gradient needs them
-      const Args &a = args();
-      const bool have = want && (a.ey_store[j] != nullptr || a.curl_store[j] != nullptr);
-      T se[R], sc[R];
-      if constexpr (FMT != 0) {
-        if (have && b.own != 0) {  // uniform
-          // an absent stream reads the other one; its sum is never stored
-          const void *const e = a.ey_store[j], *const q = a.curl_store[j];
-          const int64_t off = base * (FMT == 2 ? 2 : (int64_t)sizeof(T));
-          const char *const pe = as_global((const char *)(e ? e : q)) + off;
-          const char *const pq = as_global((const char *)(q ? q : e)) + off;
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            se[r] = (T)get_store32<T, FMT>(pe, at[r]);
-            sc[r] = (T)get_store32<T, FMT>(pq, at[r]);
-          }
-        } else {
-#pragma unroll
-          for (int r = 0; r < R; ++r) se[r] = sc[r] = (T)0;
-        }
-      }
-      T nr[R];  // negated adjoint of dHx/dz
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const bool pye = EDGE && (b.pe >> r & 1);
-        Prof<T> py = {(T)0, (T)0, 1.0};  // read with every lane active
-        if constexpr (EDGE) py = RowProfs<T>::at(yp.e, r, pye);
-        nr[r] = (T)0;
-        if (e_col && (!EDGE || (b.e >> r & 1))) {
-          const T q = cb[r] * ley[r];
-          nr[r] = q;
-          if (pye) {
-            const T mn = py.b * my[r] - q;
-            my[r] = mn;
-            nr[r] = py.over(q) - py.a * mn;
-          }
-        }
-      }
-      put_a<T, P, R>(lds, c, nr);
-      if (active) {
+  for (int j = 0; j < steps; ++j) {
+    const int lo = halo - (steps - 1 - j) * HS, hi = c.rows - lo;
+    const bool active = c.row0 < hi + P - 1 && c.row0 + R > lo - P;  // uniform
+    const RowBits b = rows.again();
+    // this step's snapshots, read well before the gradient needs them
+    const Args &a = args();
+    const bool have = want && (a.ey_store[j] != nullptr || a.curl_store[j] != nullptr);
+    T se[R], sc[R];
+    if constexpr (FMT != 0) {
+      if (have && b.own != 0) {  // uniform
+        // an absent stream reads the other one; its sum is never stored
+        const void *const e = a.ey_store[j], *const q = a.curl_store[j];
+        const int64_t off = base * (FMT == 2 ? 2 : (int64_t)sizeof(T));
+        const char *const pe = as_global((const char *)(e ? e : q)) + off;
+        const char *const pq = as_global((const char *)(q ? q : e)) + off;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const bool in = e_col && (!EDGE || (b.e >> r & 1));
-          T rx = (T)0;  // adjoint of dHz/dx
-          if (in) {
-            const T q = cb[r] * ley[r];
-            rx = q;
-            if (pml_xe) {
-              const T mn = px.b * mx[r] + q;
-              mx[r] = mn;
-              rx = px.a * mn + px.over(q);
-            }
-          }
-          T h[2 * P + 1];
-          lane_window<T, P>(rx, h);
-          const T d = d_int_adj<T, P>([&](int o) { return h[P + o]; }, rdx);
-          if (in) lhz[r] = lhz[r] + d;
-        }
-      }
-      __syncthreads();
-      T rz[R];
-      if (active) {
-        T n[R + 2 * P - 1];
-        get_a<T, P, R>(lds, c, nr, n);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const bool pyh = EDGE && (b.ph >> r & 1);
-          Prof<T> py = {(T)0, (T)0, 1.0};  // read with every lane active
-          if constexpr (EDGE) py = RowProfs<T>::at(yp.h, r, pyh);
-          // n holds the negated terms: the transposed difference of the terms
-          // is the plain half-point difference of their negatives
-          const T d = d_half<T, P>([&](int o) { return n[P - 1 + r + o]; }, rdy);
-          if (e_col && (!EDGE || (b.e >> r & 1))) lhx[r] = lhx[r] + d;
-          rz[r] = (T)0;  // adjoint of dEy/dz
-          if (e_col && (!EDGE || (b.h >> r & 1))) {
-            const T q = -cq[r] * lhx[r];
-            rz[r] = q;
-            if (pyh) {
-              const T mn = py.b * nz[r] + q;
-              nz[r] = mn;
-              rz[r] = py.a * mn + py.over(q);
-            }
-          }
+          se[r] = (T)get_store32<T, FMT>(pe, at[r]);
+          sc[r] = (T)get_store32<T, FMT>(pq, at[r]);
         }
       } else {
 #pragma unroll
-        for (int r = 0; r < R; ++r) rz[r] = (T)0;
-      }
-      put_b<T, P, R>(lds, c, rz);
-      T dx[R];
-      if (active) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            T rxh = (T)0;  // adjoint of dEy/dx
-          if (hz_col && (!EDGE || (b.e >> r & 1))) {
-            const T q = cq[r] * lhz[r];
-            rxh = q;
-            if (pml_xh) {
-              const T mn = pxh.b * nxm[r] + q;
-              nxm[r] = mn;
-              rxh = pxh.a * mn + pxh.over(q);
-            }
-          }
-          T h[2 * P + 1];
-          lane_window<T, P>(rxh, h);
-          dx[r] = d_half_adj<T, P>([&](int o) { return h[P + o]; }, rdx);
-        }
-      }
-      __syncthreads();
-      if (active) {
-        T z[R + 2 * P - 1];
-        get_b<T, P, R>(lds, c, rz, z);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const bool in = e_col && (!EDGE || (b.e >> r & 1));
-          const T dz = d_half_adj<T, P>([&](int o) { return z[P + r + o]; }, rdy);
-          if (in) ley[r] = ca[r] * ley[r] + (dz + dx[r]);
-        }
-        if (points.fast >= 0) {  // uniform
-          const Args &q = args();
-          const T *const gr = q.grad_r != nullptr ? q.grad_r - j * q.r_stride : nullptr;
-          T *const gf = q.grad_f != nullptr ? q.grad_f - j * q.f_stride : nullptr;
-          points.adjoint(q.pts, c, q.n_shots, s, lds.amp_at(c, steps, j), gr, gf, own, b.own, ley);
-        }
-        if constexpr (FMT != 0) {
-          if (have) {  // uniform; rim cells hold snapshots of 0 or are never added
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-              const double lm = (double)ley[r];
-              ga[r] = fma(lm, (double)se[r], ga[r]);
-              gb[r] = fma(lm, (double)sc[r], gb[r]);
-            }
-          }
-        }
+        for (int r = 0; r < R; ++r) se[r] = sc[r] = (T)0;
       }
     }
-
-    const Args &z = args();
+    T nr[R];  // negated adjoint of dHx/dz
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      if (!(rows.own >> r & 1) || !own) continue;
-      const uint32_t o = at[r];
-      *elem32(as_global(z.out[0]) + base, o) = ley[r];
-      *elem32(as_global(z.out[1]) + base, o) = lhx[r];
-      *elem32(as_global(z.out[2]) + base, o) = lhz[r];
-      if constexpr (EDGE) {
-        if (e_col && (rows.e >> r & 1)) {
-          if (pml_xe) *elem32(as_global(z.out[3]) + base, o) = mx[r];
-          if (rows.pe >> r & 1) *elem32(as_global(z.out[4]) + base, o) = my[r];
-          if (x < nx - P && pml_xh) *elem32(as_global(z.out[5]) + base, o) = nxm[r];
-          if (rows.h & rows.ph & (1 << r)) *elem32(as_global(z.out[6]) + base, o) = nz[r];
-        }
-      }
-      if constexpr (FMT != 0) {
-        // the shots' sum once per group, or each shot's own gradient
-        if (want && (z.per_shot_grad || s + 1 == s1) && e_col &&
-            (!EDGE || (rows.e >> r & 1))) {
-          const int64_t gp = z.per_shot_grad ? base : group * z.group_stride;
-          if (z.gca) *elem32(as_global(z.gca) + gp, o) += ga[r] * z.step_scale;
-          if (z.gcb) *elem32(as_global(z.gcb) + gp, o) += gb[r] * z.step_scale;
+      const bool pye = EDGE && (b.pe >> r & 1);
+      Prof<T> py = {(T)0, (T)0, 1.0};  // read with every lane active
+      if constexpr (EDGE) py = RowProfs<T>::at(yp.e, r, pye);
+      nr[r] = (T)0;
+      if (e_col && (!EDGE || (b.e >> r & 1))) {
+        const T q = cb[r] * ley[r];
+        nr[r] = q;
+        if (pye) {
+          const T mn = py.b * my[r] - q;
+          my[r] = mn;
+          nr[r] = py.over(q) - py.a * mn;
         }
       }
     }
-    if (z.per_shot_grad) {
+    put_a<T, P, R>(lds, c, nr);
+    if (active) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) ga[r] = gb[r] = 0.0;
+      for (int r = 0; r < R; ++r) {
+        const bool in = e_col && (!EDGE || (b.e >> r & 1));
+        T rx = (T)0;  // adjoint of dHz/dx
+        if (in) {
+          const T q = cb[r] * ley[r];
+          rx = q;
+          if (pml_xe) {
+            const T mn = px.b * mx[r] + q;
+            mx[r] = mn;
+            rx = px.a * mn + px.over(q);
+          }
+        }
+        T h[2 * P + 1];
+        lane_window<T, P>(rx, h);
+        const T d = d_int_adj<T, P>([&](int o) { return h[P + o]; }, rdx);
+        if (in) lhz[r] = lhz[r] + d;
+      }
+    }
+    __syncthreads();
+    T rz[R];
+    if (active) {
+      T n[R + 2 * P - 1];
+      get_a<T, P, R>(lds, c, nr, n);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const bool pyh = EDGE && (b.ph >> r & 1);
+        Prof<T> py = {(T)0, (T)0, 1.0};  // read with every lane active
+        if constexpr (EDGE) py = RowProfs<T>::at(yp.h, r, pyh);
+        // n holds the negated terms: the transposed difference of the terms
+        // is the plain half-point difference of their negatives
+        const T d = d_half<T, P>([&](int o) { return n[P - 1 + r + o]; }, rdy);
+        if (e_col && (!EDGE || (b.e >> r & 1))) lhx[r] = lhx[r] + d;
+        rz[r] = (T)0;  // adjoint of dEy/dz
+        if (e_col && (!EDGE || (b.h >> r & 1))) {
+          const T q = -cq[r] * lhx[r];
+          rz[r] = q;
+          if (pyh) {
+            const T mn = py.b * nz[r] + q;
+            nz[r] = mn;
+            rz[r] = py.a * mn + py.over(q);
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) rz[r] = (T)0;
+    }
+    put_b<T, P, R>(lds, c, rz);
+    T dx[R];
+    if (active) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        T rxh = (T)0;  // adjoint of dEy/dx
+        if (hz_col && (!EDGE || (b.e >> r & 1))) {
+          const T q = cq[r] * lhz[r];
+          rxh = q;
+          if (pml_xh) {
+            const T mn = pxh.b * nxm[r] + q;
+            nxm[r] = mn;
+            rxh = pxh.a * mn + pxh.over(q);
+          }
+        }
+        T h[2 * P + 1];
+        lane_window<T, P>(rxh, h);
+        dx[r] = d_half_adj<T, P>([&](int o) { return h[P + o]; }, rdx);
+      }
+    }
+    __syncthreads();
+    if (active) {
+      T z[R + 2 * P - 1];
+      get_b<T, P, R>(lds, c, rz, z);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const bool in = e_col && (!EDGE || (b.e >> r & 1));
+        const T dz = d_half_adj<T, P>([&](int o) { return z[P + r + o]; }, rdy);
+        if (in) ley[r] = ca[r] * ley[r] + (dz + dx[r]);
+      }
+      if (points.fast >= 0) {  // uniform
+        const Args &q = args();
+        const T *const gr = q.grad_r != nullptr ? q.grad_r - j * q.r_stride : nullptr;
+        T *const gf = q.grad_f != nullptr ? q.grad_f - j * q.f_stride : nullptr;
+        points.adjoint(q.pts, c, q.n_shots, s, lds.amp_at(c, steps, j), gr, gf, own, b.own, ley);
+      }
+      if constexpr (FMT != 0) {
+        if (have) {  // uniform; rim cells hold snapshots of 0 or are never added
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            const double lm = (double)ley[r];
+            ga[r] = fma(lm, (double)se[r], ga[r]);
+            gb[r] = fma(lm, (double)sc[r], gb[r]);
+          }
+        }
+      }
+    }
+  }
+
+  const Args &z = args();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (!(rows.own >> r & 1) || !own) continue;
+    const uint32_t o = at[r];
+    *elem32(as_global(z.out[0]) + base, o) = ley[r];
+    *elem32(as_global(z.out[1]) + base, o) = lhx[r];
+    *elem32(as_global(z.out[2]) + base, o) = lhz[r];
+    if constexpr (EDGE) {
+      if (e_col && (rows.e >> r & 1)) {
+        if (pml_xe) *elem32(as_global(z.out[3]) + base, o) = mx[r];
+        if (rows.pe >> r & 1) *elem32(as_global(z.out[4]) + base, o) = my[r];
+        if (x < nx - P && pml_xh) *elem32(as_global(z.out[5]) + base, o) = nxm[r];
+        if (rows.h & rows.ph & (1 << r)) *elem32(as_global(z.out[6]) + base, o) = nz[r];
+      }
+    }
+    if constexpr (FMT != 0) {
+      if (want && e_col && (!EDGE || (rows.e >> r & 1))) {
+        if (z.gca) *elem32(as_global(z.gca) + base, o) += ga[r] * z.step_scale;
+        if (z.gcb) *elem32(as_global(z.gcb) + base, o) += gb[r] * z.step_scale;
+      }
     }
   }
 }
@@ -1155,14 +1141,12 @@ __device__ __forceinline__ void tile_adj_group(ArgRef<TileAdjArgs<T>> args, int 
   extern __shared__ double tile_lds[];
   const TileAdjArgs<T> &a = args();
   const TileRows<T, P> lds(tile_lds, (int)blockDim.y, a.steps, (int)threadIdx.x);
-  const int n_groups = (a.n_shots + a.group - 1) / a.group;
-  const int tile = flat / n_groups, k = flat - tile * n_groups;
-  const int s0 = k * a.group, s1 = min(s0 + a.group, a.n_shots);
+  const int tile = flat / a.n_shots, s = flat - tile * a.n_shots;
   const TilePlace c = tile_place<T, P, R>(a.g, a.order, a.pts.n_xt, tile, a.halo, a.own_rows);
   if (c.edge)  // uniform over the workgroup
-    tile_adjoint<T, P, R, FMT, true>(args, c, s0, s1, k, lds);
+    tile_adjoint<T, P, R, FMT, true>(args, c, s, lds);
   else
-    tile_adjoint<T, P, R, FMT, false>(args, c, s0, s1, k, lds);
+    tile_adjoint<T, P, R, FMT, false>(args, c, s, lds);
 }
 
 template <typename T, int P, int R, int W, int FMT>

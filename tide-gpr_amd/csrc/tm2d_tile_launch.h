@@ -13,10 +13,10 @@ namespace tm2d {
 
 struct TilePlan {
   int waves, rows, steps;  // wavefronts per workgroup, rows per wavefront, steps per launch
-  int halo, own_rows, own_cols, n_xt, n_yt, group;
+  int halo, own_rows, own_cols, n_xt, n_yt;
 };
 
-inline TilePlan make_tile_plan(int half, int ny, int nx, int waves, int rows, int steps, int group) {
+inline TilePlan make_tile_plan(int half, int ny, int nx, int waves, int rows, int steps) {
   TilePlan p;
   p.waves = waves;
   p.rows = rows;
@@ -26,7 +26,6 @@ inline TilePlan make_tile_plan(int half, int ny, int nx, int waves, int rows, in
   p.own_cols = 64 - 2 * p.halo;
   p.n_xt = (nx + p.own_cols - 1) / p.own_cols;
   p.n_yt = (ny + p.own_rows - 1) / p.own_rows;
-  p.group = group;
   return p;
 }
 
@@ -74,10 +73,8 @@ double tile_launch_us(int half, int rows, int steps, bool adjoint, bool storing)
 // (fp32, order 2, us per step, forward / adjoint): 171 000 cells 2.1 / 3.5
 // with 32-row tiles of 8 steps (64-row: 2.8 / 5.1), 577 000 cells 3.3 / 5.7
 // with 64-row tiles of 6 (32-row: 4.5 / 7.6).
-// `us_per_step` gets the modelled time per step.
 template <typename T>
-TilePlan plan_tiles(int half, int ny, int nx, int n_shots, bool adjoint, bool storing,
-                    double *us_per_step = nullptr) {
+TilePlan plan_tiles(int half, int ny, int nx, int n_shots, bool adjoint, bool storing) {
   constexpr int kCus = 256;
   TilePlan best{};
   double best_us = 1e30;
@@ -90,7 +87,7 @@ TilePlan plan_tiles(int half, int ny, int nx, int n_shots, bool adjoint, bool st
       const int halo = steps * (2 * half - 1);
       // at least a quarter of the tile's rows and half its columns owned
       if (halo > 16 || waves * rows - 2 * halo < waves * rows / 4) break;
-      const TilePlan p = make_tile_plan(half, ny, nx, waves, rows, steps, 1);
+      const TilePlan p = make_tile_plan(half, ny, nx, waves, rows, steps);
       const double n = (double)p.n_xt * p.n_yt * n_shots;
       const double rounds = n <= kCus ? 1.0 : std::min(std::ceil(n / kCus), n / kCus + 0.3);
       const double us = rounds * tile_launch_us<T>(half, rows, steps, adjoint, storing) / steps;
@@ -100,7 +97,6 @@ TilePlan plan_tiles(int half, int ny, int nx, int n_shots, bool adjoint, bool st
       }
     }
   }
-  if (us_per_step) *us_per_step = best_us;
   return best;
 }
 
@@ -120,7 +116,7 @@ template <typename T> TilePlan plan_born(int half, int ny, int nx, int n_shots) 
   for (int steps = 1; steps <= kTileSteps; ++steps) {
     const int halo = steps * (2 * half - 1);
     if (kBornRows - 2 * halo < kBornRows / 4) break;
-    const TilePlan p = make_tile_plan(half, ny, nx, waves, rows, steps, 1);
+    const TilePlan p = make_tile_plan(half, ny, nx, waves, rows, steps);
     const double rounds = std::max(1.0, (double)p.n_xt * p.n_yt * n_shots / 256.0);
     const double us = std::min(std::ceil(rounds), rounds + 0.3) *
                       (10.0 + (rows == 2 ? 1.8 : 3.0) * steps) / steps;
@@ -181,8 +177,7 @@ void tile_fwd_fmt(const TilePlan &p, int fmt, hipStream_t stream, const TileFwdA
 template <typename T, int P, int R, int W>
 void tile_adj_fmt(const TilePlan &p, int fmt, hipStream_t stream, const TileAdjArgs<T> &a) {
   const dim3 block(64, (unsigned)p.waves);
-  const int n_groups = (a.n_shots + a.group - 1) / a.group;
-  const unsigned grid = (unsigned)((int64_t)p.n_xt * p.n_yt * n_groups);
+  const unsigned grid = (unsigned)((int64_t)p.n_xt * p.n_yt * a.n_shots);
   const size_t lds = TileRows<T, P>::bytes(p.waves, a.steps);
   if (fmt == 0) return tile_adj<T, P, R, W, 0><<<grid, block, lds, stream>>>(a);
   if constexpr (sizeof(T) == 4)
