@@ -53,11 +53,12 @@ def _families(fn):
 
 @pytest.mark.parametrize("case,forward,storing,adjoint", [
     (dict(ny=96, nx=96, shots=1, nt=64), TILES, TILES, TILES),
-    (dict(ny=1065, nx=1065, shots=4, nt=64), TILES, TILES, WAVEFRONT),
-    (dict(ny=1065, nx=1065, shots=4, nt=64, compression=True), TILES, TILES, WAVEFRONT),
-    (dict(ny=1065, nx=1065, shots=4, nt=24), TILES, TILES, TILES),
-    (dict(ny=1065, nx=1065, shots=3, nt=64), TILES, TILES, TILES),
-    (dict(ny=768, nx=800, shots=12, nt=64), TILES, WAVEFRONT, WAVEFRONT),
+    (dict(ny=1065, nx=1065, shots=4, nt=64), TILES, TILES, TILES),
+    (dict(ny=1300, nx=1300, shots=4, nt=64), TILES, TILES, WAVEFRONT),
+    (dict(ny=1300, nx=1300, shots=4, nt=64, compression=True), TILES, TILES, TILES),
+    (dict(ny=1300, nx=1300, shots=4, nt=24), TILES, TILES, TILES),
+    (dict(ny=1300, nx=1300, shots=3, nt=64), TILES, TILES, TILES),
+    (dict(ny=768, nx=800, shots=12, nt=64), TILES, WAVEFRONT, TILES),
     (dict(ny=441, nx=942, shots=12, nt=64), TILES, WAVEFRONT, TILES),
     (dict(ny=441, nx=942, shots=12, nt=64, compression=True), TILES, TILES, TILES),
     (dict(ny=700, nx=700, shots=4, nt=64, dtype=torch.float64), TILES, TILES, TILES),

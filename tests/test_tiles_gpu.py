@@ -283,7 +283,7 @@ def test_batched_plans_without_room_for_tiles_fall_back(no_room, graph):
 @pytest.mark.parametrize("blocks", [(0, 2), (0, 1), (2, 0), (1, 0), (0, 3)])
 @pytest.mark.parametrize("compression,interval,graph", [(False, 1, True), (True, 2, False)])
 def test_batched_plans_with_one_pass_on_tiles(blocks, compression, interval, graph):
-    """Tiles in one pass and step launches in the other, as large batches run."""
+    """Tiles in one pass, step launches in the other."""
     before = tide._native.get_tm2d_time_block()
     tide._native.set_tm2d_time_block(*blocks)
     try:

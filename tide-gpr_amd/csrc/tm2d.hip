@@ -793,7 +793,7 @@ int backward_impl(Problem<T> p, const T *grad_r, T *l_ey, T *l_hx, T *l_hz, T *m
   const bool per_shot = (gca && p.g.ca_b) || (gcb && p.g.cb_b);
   if (g_tuning.adj_steps == 0 && !staged &&
       !wavefront_adjoint(sizeof(T), n_shots, p.g.numel, nt, (gca != nullptr) + (gcb != nullptr),
-                         per_shot)) {
+                         fmt, step_ratio, per_shot)) {
     int rc = backward_tiles(1, p, grad_r, l_ey, l_hx, l_hz, ml_ey_x, ml_ey_z, ml_hx_z,
                                   ml_hz_x, ey_store, curl_store, fmt, store_step_bytes, grad_f, gca,
                                   gcb, src, rec, nt, start_t, step_ratio, stream);

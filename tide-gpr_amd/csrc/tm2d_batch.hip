@@ -2,9 +2,9 @@
 // shot counts and nt) advanced together.  By default the time loops run on
 // workgroup tiles (tm2d_tile.h): one launch advances every problem by up to 8
 // steps, each from its own argument record; all problems share one tile shape
-// and step count per pass, chosen for the whole batch.  As settings, and for
-// the adjoint of some large batches: one launch per time step, or one per two
-// time steps with the two-step kernels of tm2d_fused.h; a problem whose nt is
+// and step count per pass, chosen for the whole batch.  As settings, and where
+// the tiles' memory does not fit: one launch per time step, or one per two time
+// steps with the two-step kernels of tm2d_fused.h; a problem whose nt is
 // odd takes its last step in a one-step launch over its own tiles.
 //
 // Every problem keeps its own arrays; a plan holds a device table with one
@@ -869,24 +869,6 @@ int build_step_launches(Plan &p, const std::vector<BatchItem<float>> &proto, boo
   return kOk;
 }
 
-// Whether a batch's adjoint runs two steps per launch, not on tiles: where at
-// least half its cells are in grids of 150 000 cells and more whose shots fill
-// workgroups of four (which share a gradient slice; tiles hold one per shot), from
-// 5.5 million cells.  ms of a 96-step adjoint, tiles / two-step: 8 x 425 x 445
-// cells and 4 shots 5.4 / 4.9, 3 x 725 x 745 x 4 4.7 / 4.4; below and beside it 4 x
-// 545 x 565 x 4 3.5 / 3.7, 24 x 325 x 345 x 4 8.8 / 9.9, 12 x 425 x 445 x 3 6.4 /
-// 6.8, 60 x 245 x 265 x 3 11.6 / 15.2, 4 x 1325 x 1325 x 1 4.7 / 12.5.
-bool two_step_adjoint(const tide_tm2d_problem *problems, int64_t n) {
-  double cells = 0.0, shared = 0.0;
-  for (int64_t m = 0; m < n; ++m) {
-    const tide_tm2d_problem &q = problems[m];
-    const double numel = (double)q.ny * (double)q.nx, c = numel * (double)q.n_shots;
-    cells += c;
-    if (numel >= 150000 && q.n_shots > 0 && balanced_group((int)q.n_shots, 4) == 4) shared += c;
-  }
-  return cells >= 5.5e6 && 2.0 * shared >= cells;
-}
-
 int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t storage_format,
                int64_t use_graph, int64_t device, bool tiles) {
   p->device = (int)device;
@@ -896,9 +878,13 @@ int build_plan(Plan *p, const tide_tm2d_problem *problems, int64_t n, int64_t st
   p->rows_a = rows_for<float>(g_tuning.adj_rows);
   p->group = g_tuning.adj_group;  // one group size for both passes
   // Each pass runs on tiles unless a time block is set (one- or two-step
-  // launches; a K-step setting runs at 2), the adjoint of some large batches too.
+  // launches; a K-step setting runs at 2).  ms of 96 steps, tiles / two-step
+  // launches, forward with snapshots and adjoint: 24 grids of 245 x 265 cells (x 3
+  // shots) 2.2 / 3.3 and 4.0 / 6.2; 4 of 1325 x 1325 x 1 3.0 / 5.1 and 4.4 / 12.2;
+  // 8 of 425 x 445 x 4 2.7 / 3.4 and 4.7 / 4.8; 4 of 725 x 745 x 4 3.7 / 5.2 and
+  // 5.8 / 5.9; 12 of 545 x 565 x 4 7.0 / 11.2 and 9.5 / 11.6.
   p->tiles_f = tiles && g_tuning.fwd_steps == 0;
-  p->tiles_a = tiles && g_tuning.adj_steps == 0 && !two_step_adjoint(problems, n);
+  p->tiles_a = tiles && g_tuning.adj_steps == 0;
   p->steps_f = g_tuning.fwd_steps == 1 ? 1 : 2;
   p->steps_a = g_tuning.adj_steps == 1 ? 1 : 2;
   const bool steps = !p->tiles_f || !p->tiles_a;  // a pass runs on step launches

@@ -8,7 +8,6 @@
 
 #include "tm2d_device.h"
 
-#include <cmath>
 #include <cstdint>
 
 namespace tide_hip {
@@ -17,37 +16,40 @@ namespace tm2d {
 // Order-2 forward on two-step wavefront tiles: calls that store both snapshot
 // streams at full fp32 width in every step, between 4.5 million cells and what
 // leaves their two state buffers (24 bytes a cell, 4 more for each per-shot
-// coefficient) in the 256 MB last-level cache: 600 x 640 cells and 12 shots 24.8 /
-// 21.0; 768 x 800 and 12 39.0 / 32.9; 950 x 950 and 8 36.0 / 31.0; 441 x 942 and
-// 12 25.9 / 23.1.  Below and above tiles are as fast or faster (560 x 600 x 12
-// 18.6 / 19.3; 1065 x 1065 x 12 77 / 90), so are they with fewer than 6 shots
-// (1300 x 1300 x 4 26.8 / 27.6), with small grids, whose border tiles weigh more
-// (441 x 500 x 24 27.1 / 28.9), with BF16 or sampled snapshots, and where a run is
-// so short that the wavefront path's many allocations weigh.
+// coefficient) well inside the 256 MB last-level cache: 600 x 640 cells and 12
+// shots 25.4 / 22.5; 768 x 800 and 12 39.4 / 35.3; 950 x 950 and 8 36.1 / 33.5; 441 x
+// 942 and 12 26.2 / 24.8; 500 x 640 and 24 43 / 38.  Below and above tiles are as
+// fast or faster (560 x 600 x 12 18.6 / 19.3; 640 x 800 x 16 34.5 / 38.9; 1065 x
+// 1065 x 12 77 / 90), so are they with fewer than 6 shots (1300 x 1300 x 4 26.8 /
+// 27.6), with small grids, whose border tiles weigh more (441 x 500 x 24 27.1 /
+// 28.9), with BF16 or sampled snapshots, and where a run is so short that the
+// wavefront path's many allocations weigh.
 inline bool wavefront_forward(size_t elem, int64_t n_shots, int64_t numel, int64_t nt,
                               bool both_streams, int fmt, int64_t step_ratio,
                               int batched_coefficients) {
   const int64_t cells = n_shots * numel;
   return elem == 4 && both_streams && fmt == 1 && step_ratio == 1 && nt >= 64 && n_shots >= 6 &&
          numel >= 250000 && cells >= 4500000 &&
-         cells * (24 + 4 * batched_coefficients) <= 200000000;
+         cells * (24 + 4 * batched_coefficients) <= 185000000;
 }
 
 // Order-2 adjoint on three-step wavefront tiles: large fp32 calls whose shots
 // fill workgroups of four, which share one FP64 gradient slice (tiles hold one
-// per shot).  Per cell the tiles' time is the same at every size, the wavefront
-// tiles' falls with the share of border tiles: the line is cells x the grid's
-// side, for two gradients: 1065 x 1065 cells and 4 shots (4.8e9) 30.4 / 29.3; 1300
-// x 1300 x 4 43.1 / 38.5; 2081 x 2081 x 4, BF16 107 / 89; 768 x 800 x 12 52.8 /
-// 45.8; below it 441 x 942 x 12 (3.2e9) 34.3 / 37.8, 900 x 900 x 4 (2.9e9) 21.8 /
-// 21.9.  Groups of three shots and fewer gain 4 % at most (2081 x 2081 x 2 55.4 /
-// 53.4) and lose as much (1000 x 1000 x 6 38.4 / 41.5); per-shot gradients have no
-// shared slice (1000 x 1000 x 8 58 / 98).
+// per shot).  Per cell the tiles' time grows with the state, the wavefront tiles'
+// falls with the share of border tiles; the line is cells x cells of a grid, with
+// two gradients from full snapshots of every step: 1300 x 1300 cells and 4 shots
+// (1.14e13) 41.3 / 38.9; 2081 x 2081 x 4 102 / 90; 1541 x 1541 x 8 115 / 109; 1065 x
+// 1065 x 12 (1.5e13) 91 / 86; below it 1065 x 1065 x 8 (1.03e13) 57.7 / 59.1, 1065 x
+// 1065 x 4 28.4 / 29.5, 800 x 800 x 16 66 / 70.  With fewer gradient bytes it lies
+// higher: BF16 1541 x 1541 x 4 (2.3e13) 54.6 / 55.9, 2081 x 2081 x 4 (7.5e13) 94 /
+// 91.  Groups of three shots and fewer gain at most 2 % (2100 x 2100 x 3 78.1 /
+// 76.8); per-shot gradients have no shared slice (1000 x 1000 x 8 58 / 98).
 inline bool wavefront_adjoint(size_t elem, int64_t n_shots, int64_t numel, int64_t nt,
-                              int gradients, bool per_shot) {
-  const double weight = 0.5 * gradients * (double)n_shots * (double)numel * std::sqrt((double)numel);
-  return elem == 4 && !per_shot && nt >= 64 && balanced_group((int)n_shots, 4) == 4 &&
-         weight >= 4.4e9;
+                              int gradients, int fmt, int64_t step_ratio, bool per_shot) {
+  const bool full = gradients == 2 && fmt == 1 && step_ratio == 1;
+  const double weight = (double)n_shots * (double)numel * (double)numel;
+  return elem == 4 && gradients > 0 && !per_shot && nt >= 64 &&
+         balanced_group((int)n_shots, 4) == 4 && weight >= (full ? 1.1e13 : 5e13);
 }
 
 // Orders 4 to 8 in place.  Runs of few steps: a tile loop's set-up (a second
