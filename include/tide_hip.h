@@ -1234,11 +1234,13 @@ int tide_tm2d_set_shot_loop(int fwd_loop, int adj_loop);
 int tide_tm2d_get_shot_loop(int *out2);
 
 /*
- * Time steps per launch of the single-problem TM2D path, per pass (0 to
- * 4).  0 (the default) picks the kernels and their steps from the problem:
- * workgroup tiles of up to 8 steps per launch (64 columns x 32 or 64 rows held
- * in registers, halo recomputed), or, where many shots of a large grid fill
- * the device, two (forward) or three (adjoint) steps as below.  With K >= 2, K steps run in one launch of the K-step kernels
+ * Time steps per launch of the single-problem TM2D path of stencil order 2,
+ * per pass (0 to 4).  0 (the default) picks the kernels and their steps from
+ * the problem: workgroup tiles of up to 8 steps per launch (64 columns x 32 or
+ * 64 rows held in registers, halo recomputed), or, for some large fp32 gradients,
+ * two (forward) or three (adjoint) steps as below (tm2d_route.h).  Batched plans
+ * take 0 as workgroup tiles, 1 as one step and more as two steps per launch.
+ * With K >= 2, K steps run in one launch of the K-step kernels
  * (64 - 2K owned columns per wavefront, a recomputed halo of K), which read
  * and write the wavefield state once per K steps; results are bitwise
  * those of single steps.  A remainder runs as two-step and single-step

@@ -87,8 +87,9 @@ def test_em3d_storage_and_adjoint_match_oracle(store):
 
 def test_em3d_adjoint_many_shots_and_tunings():
     """More shots than a workgroup holds (each group writes its own FP64
-    gradient slice, the slices are summed in a fixed order afterwards) and
-    every launch shape give the oracle's adjoint."""
+    gradient slice, the slices are summed in a fixed order afterwards), at
+    several shots per workgroup and both workgroup orders, give the oracle's
+    adjoint (the z-plane settings are accepted and have no effect)."""
     case = _case(torch.float64, nz=9, ny=10, nx=12, nt=16, shots=10)
     _, r_o, s_o = O.em3d_forward(case, store="full")
     rng = np.random.default_rng(5)

@@ -5,9 +5,11 @@
 // maxwell_tm_core.cuh:448-599; exact adjoint and reverse loop
 // maxwell_tm_cuda_inst.cu:922-1254, 2540-2731).
 //
-// Calls whose snapshots stay on the device run on the workgroup tiles of
-// tm2d_tile.h (one launch for up to four steps).  These kernels serve what
-// those do not: host-staged snapshots, Debye dispersion and the Born products.
+// Most calls whose snapshots stay on the device run on the workgroup tiles of
+// tm2d_tile.h (one launch for up to five steps).  These kernels serve the
+// others: host-staged snapshots, Debye dispersion, the Born adjoint, the calls
+// that are faster in place (tm2d_route.h) and those without room for a second
+// state.
 // They run one cell per lane: a workgroup is a 64 x 4 tile of one shot (64
 // consecutive cells of a row per wavefront, coalesced), and every time step is
 // a short sequence of launches:
