@@ -65,9 +65,13 @@ def _families(fn):
     (dict(ny=96, nx=96, shots=2, nt=7, stencil=4), IN_PLACE, IN_PLACE, TILES),
     (dict(ny=96, nx=96, shots=2, nt=3, stencil=6), IN_PLACE, IN_PLACE, IN_PLACE),
     (dict(ny=96, nx=96, shots=2, nt=8, stencil=8), TILES, TILES, TILES),
-    (dict(ny=400, nx=400, shots=4, nt=16, stencil=8, dtype=torch.float64), IN_PLACE,
+    (dict(ny=420, nx=440, shots=4, nt=16, stencil=8, dtype=torch.float64), IN_PLACE,
      IN_PLACE, TILES),
     (dict(ny=400, nx=400, shots=4, nt=16, stencil=6, dtype=torch.float64), TILES, TILES, TILES),
+    (dict(ny=110, nx=120, shots=40, nt=8, stencil=6, dtype=torch.float64), IN_PLACE,
+     IN_PLACE, TILES),
+    (dict(ny=64, nx=200, shots=40, nt=8, stencil=6, dtype=torch.float64), TILES, TILES, TILES),
+    (dict(ny=64, nx=200, shots=40, nt=8, stencil=8, dtype=torch.float64), TILES, TILES, TILES),
 ])
 def test_calls_run_on_the_kernels_that_measured_faster(case, forward, storing, adjoint):
     print(case, flush=True)

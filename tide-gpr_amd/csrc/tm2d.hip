@@ -1150,6 +1150,14 @@ bool tiled_order(int stencil, const Problem<T> &p, int64_t nt, int fmt, const Sn
 }
 
 template <typename T>
+bool faster_in_place(int half, const Problem<T> &p, int64_t nt, bool storing) {
+  const TilePlan plan = plan_tiles<T>(half, p.g.ny, p.g.nx, p.n_shots, false, storing);
+  const TileOrder order = tile_order(plan, p.g, half);
+  return in_place_forward(half, sizeof(T), p.n_shots, p.g.numel, nt, plan,
+                          order.edges(plan.n_xt) == plan.n_xt * plan.n_yt);
+}
+
+template <typename T>
 int forward_entry(T const *ca, T const *cb, T const *cq, T const *f, T *ey, T *hx, T *hz,
                   T *m_ey_x, T *m_ey_z, T *m_hx_z, T *m_hz_x, T *r, T const *ay,
                   T const *by, T const *ayh, T const *byh, T const *ax, T const *bx,
@@ -1193,7 +1201,7 @@ int forward_entry(T const *ca, T const *cb, T const *cq, T const *f, T *ey, T *h
       set_error("step_ratio must be positive");
       rc = kInvalidArgument;
     } else if (!tiled_order(stencil, p, nt, fmt, ey_st, curl_st) ||
-               in_place_forward(stencil / 2, sizeof(T), n_shots, ny * nx, nt)) {
+               faster_in_place(stencil / 2, p, nt, ey_store || curl_store)) {
       in_place = true;
     } else {
       rc = forward_tiles<T>(stencil / 2, p, ey, hx, hz, m_ey_x, m_ey_z, m_hx_z, m_hz_x, f, r,

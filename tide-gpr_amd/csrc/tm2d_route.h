@@ -6,7 +6,7 @@
 // padded cells of all shots.
 #pragma once
 
-#include "tm2d_device.h"
+#include "tm2d_tile_launch.h"
 
 #include <cstdint>
 
@@ -55,15 +55,25 @@ inline bool wavefront_adjoint(size_t elem, int64_t n_shots, int64_t numel, int64
 // Orders 4 to 8 in place.  Runs of few steps: a tile loop's set-up (a second
 // state, packed profiles) takes 0.1 ms, an in-place step 12 us and more (order 4,
 // 441 x 942 cells and 4 shots, 1 step with snapshots 168 / 99 us, 8 steps 30 / 44
-// us per step; adjoint 2 steps 224 / 122, 5 steps 64 / 97).  fp64 forward of orders
-// 6 and 8, whose halo of 5 and 7 cells a step leaves 22 x 54 and 18 x 50 cells of a
-// tile: order 6 441 x 942 x 12 131 / 101, 1065 x 1065 x 4 102 / 96, but 700 x 700
-// x 4 44 / 46; order 8 441 x 942 x 12 151 / 106, 700 x 700 x 4 54 / 48, but 360 x
-// 380 x 4 21.9 / 22.7.
-inline bool in_place_forward(int half, size_t elem, int64_t n_shots, int64_t numel, int64_t nt) {
+// us per step; adjoint 2 steps 224 / 122, 5 steps 64 / 97).
+// fp64 forward of orders 6 and 8, whose halo of 5 and 7 cells a step leaves 22 x 54
+// and 18 x 50 cells of a tile.  Order 8 (one step per launch) takes about 6 us per
+// round of workgroups, in place 19 us per million cells and 8 more than tiles at
+// the start: 441 x 942 x 12 151 / 106, 700 x 700 x 4 54 / 48, 110 x 120 x 40 34 / 26,
+// but 360 x 380 x 4 21.9 / 22.7, 64 x 200 x 40 27 / 28, 200 x 220 x 12 25.1 / 25.5.
+// Order 6: large calls (441 x 942 x 12 131 / 101, 1065 x 1065 x 4 102 / 96, but 700 x
+// 700 x 4 44 / 46), and many shots of grids with edge tiles only, 9 us a round (128
+// x 128 x 64 45 / 33, 110 x 120 x 40 29 / 24, but 150 x 150 x 32 28 / 29, 64 x 200 x
+// 40 21 / 26).
+inline bool in_place_forward(int half, size_t elem, int64_t n_shots, int64_t numel, int64_t nt,
+                             const TilePlan &plan, bool edge_tiles_only) {
   if (nt < 8) return true;
-  const int64_t cells = n_shots * numel;
-  return elem == 8 && ((half == 3 && cells >= 2500000) || (half == 4 && cells >= 600000));
+  if (elem == 4 || half < 3) return false;
+  const double cells = 1e-6 * (double)n_shots * (double)numel;
+  const int64_t rounds = ((int64_t)plan.n_xt * plan.n_yt * n_shots + 255) / 256;
+  if (half == 4) return 6.0 * (double)rounds >= 8.5 + 19.0 * cells;
+  return cells >= 2.5 || (plan.steps == 1 && edge_tiles_only &&
+                          9.0 * (double)rounds >= 12.5 + 17.5 * cells + 0.1 * (double)n_shots);
 }
 inline bool in_place_adjoint(int64_t nt) { return nt < 4; }
 
